@@ -108,6 +108,14 @@ struct tpm_box_dev {
     // inside the softening length: 1 / (2 rs)^2 in 2^-64 units (x^2 = r2 *
     // inv4rs2_s) and 4 / (3 sqrt(pi)) / (2 rs)^3 in 2^-96 units
     float inv4rs2_s, k3_s;
+    // far pairs (pp_far): lengths times far_s are x sqrt(log2 e), x = r / (2 rs)
+    float far_s;                // per 2^-32 unit
+    float far_near2, far_cull2; // squared distances from a tile's box, far_s units: below the first a source's
+                                // pairs take the general law, at or beyond the second it is dropped
+    float far_ulo, far_uhi;     // the cutoff as u, less and more than any rounding of u
+    float far_wrap;             // largest |offset| + box half width whose differences cannot wrap
+    float far_g, far_ph;        // sums of pp_far -> box units
+    uint64_t rcut2i;            // a pair is inside the cutoff when its squared raw offset is below this
     // kick epilogue
     float GM, phi0, eta, t0, scale, hsoft;
     double drift;  // t0 of the drift step (batched path)

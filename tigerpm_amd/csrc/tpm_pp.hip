@@ -8,15 +8,15 @@
 //
 // Source staging: the wave walks the 27 neighbour cells (the candidate set
 // of kick_pme.cu:265-318) 64 particles at a time; each lane tests one source
-// against the integer bounding box of the tile's active sinks and survivors
-// are compacted (ballot + mbcnt) into an LDS buffer as exact int32 offsets
-// from the tile's first particle plus the source index.  A source whose box
+// against the box of the tile's active sinks and survivors are compacted
+// (ballot + mbcnt) into LDS, as exact int32 offsets (near sources) or float
+// offsets (far ones) from the box's centre.  A source whose box
 // distance exceeds rcut has r >= rcut to every sink, so dropping it changes
-// no result; smaller tiles have tighter boxes and drop more.  The inner loop
-// reads one staged source per stream with a ds_read_b128 (prefetched one
-// step ahead) and evaluates compute_pp_interaction (kick_treepm.cu:242-283).
+// no result; smaller tiles have tighter boxes and drop more.  Near pairs
+// evaluate compute_pp_interaction (kick_treepm.cu:242-283), far ones the same
+// law without its softening (pp_far).
 //
-// Pair distances are int32(sink - source) converted to float, which is the
+// Near pairs: distances are int32(sink - source) converted to float, which is the
 // reference's distance() (gravity_short.hpp:20-22) in units of 2^-32; every
 // constant is pre-scaled by the matching power of two so the FP32 arithmetic
 // is the reference's up to exact power-of-two factors, except that inside
@@ -26,6 +26,7 @@
 // evaluated like any other source, as in the reference: inside the
 // softening branch it contributes -35/16 h^-1 to phi and nothing to g.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <vector>
 
@@ -33,7 +34,13 @@
 
 #include <climits>
 
-#define SBUF 256  // staged sources per flush (4 KiB LDS)
+// Staged sources of a wave: far ones (float offsets) and near ones (int32
+// offsets), 5 KiB of LDS together, so 32 waves fill a CU's 160 KiB.  A list
+// is flushed when a further round of 64 might not fit.
+#define FAR_AT 112
+#define FAR_CAP 208   // FAR_AT + 64 + 32: four rounds of padding for 8 streams
+#define NEAR_AT 48
+#define NEAR_CAP 112  // NEAR_AT + 64
 // Per-sink source lists (LISTS, 16-sink tiles): a flush of <= LCAP staged
 // sources (staging flushes above LFLUSH), the far dummy at LFAR.
 #define LCAP 144
@@ -126,6 +133,353 @@ __device__ __forceinline__ void static_for(F& f) {
     static_for_t<0, N>::run(f);
 }
 
+// Minimum / maximum over the TS sinks of a tile (every stream holds a copy of
+// them): the 16-lane steps are DPP moves, the wider ones shuffles.
+template <int TS, class Op>
+__device__ __forceinline__ int tile_reduce(int v, Op op) {
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));   // lane ^ 1
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));   // lane ^ 2
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));  // half-row mirror: the other four
+    if constexpr (TS > 8) v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));  // row mirror
+#pragma unroll
+    for (int o = 16; o < TS; o <<= 1) v = op(v, __shfl_xor(v, o));
+    return v;
+}
+template <int TS>
+__device__ __forceinline__ int tile_min(int v) {
+    return tile_reduce<TS>(v, [](int a, int b) { return min(a, b); });
+}
+template <int TS>
+__device__ __forceinline__ int tile_max(int v) {
+    return tile_reduce<TS>(v, [](int a, int b) { return max(a, b); });
+}
+
+// The short-range sums of one tile, by one wave: lane l has sink l % TS (raw
+// position px, py, pz) and walks stream l / TS.  The sources are those of the
+// 27 cells around cell (cx, cy, cz), whose x neighbours are contiguous in
+// memory: 9 rows of up to 3 cells, each a run of particles (two where the
+// row wraps), taken 64 at a time.  Each source is tested against the box of
+// the tile's active sinks (centre and half widths, in far_s units):
+//   beyond the cutoff (far_cull2, a margin of 2048 raw units over rcut, float
+//     rounding stays below 600): dropped;
+//   within far_near2 of the box: near list, as int32 offsets from the centre,
+//     evaluated with the general law (pp_pair);
+//   else: far list, as float offsets, evaluated with pp_far.  Every pair of a
+//     far source is at least FAR_X0 2 rs and h apart.
+// At 512^3 nine pairs of ten are far ones.
+// The cutoff of a far pair: float offsets are rounded by up to a few raw
+// units, and a pair on the wrong side of the cutoff is an error of
+// 5e-4 of a typical force, larger than all rounding together.  So u is
+// compared with both ends of a window that covers its rounding; a flush that
+// met a pair inside the window (about one in 200 at 512^3) is followed by a
+// pass that adds those of them whose exact squared integer offset is inside;
+// a near pair that close to the cutoff is decided the same way
+// (pp_pair_exact).  The decision is then the same for every tile size and
+// order.
+template <int TS, bool PME, class Sync>
+__device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, int cx, int cy, int cz, uint32_t px,
+                                       uint32_t py, uint32_t pz, uint32_t rx, uint32_t ry, uint32_t rz, bool inbox,
+                                       int nact, float4* __restrict__ fbuf, int4* __restrict__ nbuf, Sync lds_sync,
+                                       float& gx, float& gy, float& gz, float& ph, unsigned long long& executed) {
+    constexpr int SPLIT = 64 / TS;  // source streams per wave
+    constexpr int BLK = 4 * SPLIT;  // sources of a block of the far loop
+    static_assert(TS >= 8 && FAR_AT + 64 + BLK <= FAR_CAP, "room for the padding");
+    const int lane = (int)lane_id();
+    const int stream = lane / TS;
+    const int C = B.C;
+    const bool cull = B.cull != 0;
+    const float fs = B.far_s;
+    // the box of the sinks with inbox: centre (raw) and half widths
+    int ox = (int)(px - rx), oy = (int)(py - ry), oz = (int)(pz - rz);
+    const int lox = tile_min<TS>(inbox ? ox : INT_MAX), hix = tile_max<TS>(inbox ? ox : INT_MIN);
+    const int loy = tile_min<TS>(inbox ? oy : INT_MAX), hiy = tile_max<TS>(inbox ? oy : INT_MIN);
+    const int loz = tile_min<TS>(inbox ? oz : INT_MAX), hiz = tile_max<TS>(inbox ? oz : INT_MIN);
+    // halves first: hi - lo may exceed 2^31 - 1 only for a cell wider than
+    // half the box, which C >= 3 rules out, but lo + hi may not fit
+    const int mx = lox + (hix - lox) / 2, my = loy + (hiy - loy) / 2, mz = loz + (hiz - loz) / 2;
+    const uint32_t qx = rx + (uint32_t)mx, qy = ry + (uint32_t)my, qz = rz + (uint32_t)mz;
+    const float hx = (float)max(hix - mx, mx - lox) * fs, hy = (float)max(hiy - my, my - loy) * fs,
+                hz = (float)max(hiz - mz, mz - loz) * fs;
+    ox -= mx;
+    oy -= my;
+    oz -= mz;
+    const float fox = (float)ox * fs, foy = (float)oy * fs, foz = (float)oz * fs;
+    // kept in vector registers: an SGPR operand costs a VALU instruction half its rate
+    float ulo = B.far_ulo, uhi = B.far_uhi;
+    asm volatile("" : "+v"(ulo), "+v"(uhi));
+    // lane l < 18: run l & 1 of row l >> 1 (0: the cells cx - 1 .. cx + 1 that
+    // do not wrap, 1: the one that does)
+    int rb = 0, re = 0;
+    if (lane < 18) {
+        const int r = lane >> 1;
+        int jy = cy + r % 3 - 1, jz = cz + r / 3 - 1;
+        jy += jy < 0 ? C : (jy >= C ? -C : 0);
+        jz += jz < 0 ? C : (jz >= C ? -C : 0);
+        int x0 = max(cx - 1, 0), x1 = min(cx + 1, C - 1);
+        if (lane & 1) {
+            x0 = cx == 0 ? C - 1 : 0;
+            x1 = cx == 0 || cx == C - 1 ? x0 : -1;  // no wrap: an empty run
+        }
+        const int row = B.cell0 + (jz * C + jy) * C;
+        rb = a.cell_begin[row + x0];
+        re = a.cell_begin[row + x1 + 1];
+    }
+    gx = gy = gz = ph = 0.f;
+    float ngx = 0.f, ngy = 0.f, ngz = 0.f, nph = 0.f;
+    int nfar = 0, nnear = 0;
+    int run = -1, j0 = 0, je = 0;
+    bool more = true;
+    while (more) {
+        // stage until a list is nearly full or the sources end
+        for (;;) {
+            if (j0 >= je) {
+                do {
+                    run++;
+                    if (run == 18) break;
+                    j0 = __builtin_amdgcn_readlane(rb, run);
+                    je = __builtin_amdgcn_readlane(re, run);
+                } while (j0 >= je);
+                if (run == 18) {
+                    more = false;
+                    break;
+                }
+            }
+            const int j = j0 + lane;
+            j0 += 64;
+            bool far = false, near = false;
+            int dx = 0, dy = 0, dz = 0;
+            float fx = 0.f, fy = 0.f, fz = 0.f;
+            if (j < je) {
+                dx = (int)(a.x[j] - qx);
+                dy = (int)(a.y[j] - qy);
+                dz = (int)(a.z[j] - qz);
+                fx = (float)dx * fs;
+                fy = (float)dy * fs;
+                fz = (float)dz * fs;
+                const float ex = fmaxf(fabsf(fx) - hx, 0.f), ey = fmaxf(fabsf(fy) - hy, 0.f),
+                            ez = fmaxf(fabsf(fz) - hz, 0.f);
+                const float d2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+                near = d2 < B.far_near2;
+                if (cull) {
+                    far = !near && d2 < B.far_cull2;
+                } else {
+                    // a difference of float offsets does not wrap round the
+                    // box as the int32 one does: sources for which it would
+                    // (C < 5) take the general law
+                    near = near || fmaxf(fabsf(fx) + hx, fmaxf(fabsf(fy) + hy, fabsf(fz) + hz)) > B.far_wrap;
+                    far = !near;
+                }
+            }
+            const unsigned long long mf = __ballot(far), mn = __ballot(near);
+            if (far) fbuf[nfar + (int)count_below(mf)] = make_float4(fx, fy, fz, __int_as_float(j));
+            nfar += __popcll(mf);
+            if (mn) {
+                if (near) nbuf[nnear + (int)count_below(mn)] = make_int4(dx, dy, dz, j);
+                nnear += __popcll(mn);
+            }
+            if (nfar > FAR_AT || nnear > NEAR_AT) break;
+        }
+        if (nfar > FAR_AT || (!more && nfar > 0)) {
+            // Whole blocks of 4 rounds (four pairs in flight per lane: 83
+            // cycles per 64 pairs, 95 with two); the rest stays in the list,
+            // and after the last source is filled up with padding sources
+            // beyond any cutoff (e = 0).
+            int nblk = nfar / BLK * BLK;
+            if (!more && nblk < nfar) {
+                if (lane < BLK) fbuf[nfar + lane] = make_float4(1e15f, 1e15f, 1e15f, 0.f);
+                nblk += BLK;
+            }
+            lds_sync();
+            unsigned long long window = 0ull;
+#pragma unroll 1
+            for (int q = 0; q < nblk; q += BLK) {
+                float4 s[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) s[k] = fbuf[q + k * SPLIT + stream];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
+                    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    float e = __builtin_amdgcn_exp2f(-u);
+                    if (!PME) {
+                        const bool in = u < ulo;
+                        window |= __ballot(u < uhi) & ~__ballot(in);
+                        e = in ? e : 0.f;
+                    }
+                    pp_far(dx, dy, dz, u, e, gx, gy, gz, ph);
+                }
+            }
+            if (!PME && window) {
+                for (int q = 0; q < nblk; q += SPLIT) {
+                    const float4 s = fbuf[q + stream];
+                    const float dx = s.x - fox, dy = s.y - foy, dz = s.z - foz;
+                    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    if (u >= ulo && u < uhi) {
+                        const int j = __float_as_int(s.w);
+                        if (pp_inside(B, (int)((qx + (uint32_t)ox) - a.x[j]), (int)((qy + (uint32_t)oy) - a.y[j]),
+                                      (int)((qz + (uint32_t)oz) - a.z[j])))
+                            pp_far(dx, dy, dz, u, __builtin_amdgcn_exp2f(-u), gx, gy, gz, ph);
+                    }
+                }
+            }
+            const int done = min(nblk, nfar), rest = nfar - done;
+            executed += (unsigned long long)done * (unsigned long long)nact;
+            if (rest > 0) {
+                const float4 t = fbuf[done + min(lane, rest - 1)];
+                lds_sync();
+                if (lane < rest) fbuf[lane] = t;
+            }
+            nfar = rest;
+            lds_sync();
+        }
+        if (nnear > NEAR_AT || (!more && nnear > 0)) {
+            lds_sync();
+            for (int q = stream; q < nnear; q += SPLIT) {
+                if constexpr (PME)
+                    pp_pair<true>(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
+                else
+                    pp_pair_exact(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
+            }
+            executed += (unsigned long long)nnear * (unsigned long long)nact;
+            nnear = 0;
+            lds_sync();
+        }
+    }
+    // box units: pp_pair's sums are in 2^-32 units, pp_far's in far_s units
+    gx = fmaf(ngx, 0x1p64f, gx * B.far_g);
+    gy = fmaf(ngy, 0x1p64f, gy * B.far_g);
+    gz = fmaf(ngz, 0x1p64f, gz * B.far_g);
+    ph = fmaf(nph, 0x1p32f, -ph * B.far_ph);
+}
+
+// The same sums with per-sink source lists (16-sink tiles, culling on).
+template <class Sync>
+__device__ __forceinline__ void pp_sum_lists(const PPArgs& a, const tpm_box_dev& B, int cx, int cy, int cz, int ox,
+                                             int oy, int oz, uint32_t rx, uint32_t ry, uint32_t rz, bool active,
+                                             int4* __restrict__ sbuf, uint8_t* __restrict__ lst,
+                                             float4* __restrict__ sinkf, Sync lds_sync, float& gx, float& gy,
+                                             float& gz, float& ph, unsigned long long& executed) {
+    const int lane = (int)lane_id(), slot = lane % 16, stream = lane / 16;
+    // Tile bounding box as floats.  float(int32) rounds by <= 64 raw units, so
+    // box distances below carry <= 192 units of error, inside the 512-unit
+    // margin of cull2s: the test never drops a source with r < rcut to any
+    // sink.
+    const float lox = (float)tile_min<16>(active ? ox : INT_MAX), hix = (float)tile_max<16>(active ? ox : INT_MIN);
+    const float loy = (float)tile_min<16>(active ? oy : INT_MAX), hiy = (float)tile_max<16>(active ? oy : INT_MIN);
+    const float loz = (float)tile_min<16>(active ? oz : INT_MAX), hiz = (float)tile_max<16>(active ? oz : INT_MIN);
+    const int C = B.C;
+    const float cull2s = B.cull2s;
+    int nbuf = 0;
+    gx = gy = gz = ph = 0.f;
+    // Far dummy of the per-sink lists: offset -2^31 on every
+    // axis, i.e. at least 1/2 - 1/C of the box from every sink of
+    // the tile (a sink lies within one cell of the tile's first
+    // particle), so r > rcut whenever culling is on (C >= 5).
+    const int4 far = make_int4(INT_MIN, INT_MIN, INT_MIN, -1);
+    // Per-sink lists: the tile's sinks as floats in LDS, read by
+    // every lane alike (an inactive sink sits far from every
+    // source: empty list).
+    {
+        if (lane < 16)
+            sinkf[lane] = make_float4(active ? (float)ox : 3.0e9f, active ? (float)oy : 3.0e9f,
+                                      active ? (float)oz : 3.0e9f, 0.f);
+        if (lane == 0) sbuf[LFAR] = far;
+    }
+    // Sources in range of no sink cost nothing but the test: a
+    // source joins sink k's list when its float distance to the
+    // sink is inside the cull distance (float(int32) offsets are
+    // off by <= 8 raw units here, far inside the 512-unit margin),
+    // so no pair with r < rcut is dropped and the pair law's own
+    // cutoff decides as before.
+    auto flush_lists = [&]() {
+        lds_sync();
+        int cntv = 0;  // lane k < 16: entries of sink k's list
+        for (int r0 = 0; r0 < nbuf; r0 += 64) {
+            const int e = r0 + lane;
+            // lanes past the staged sources test the far dummy,
+            // which is in range of no sink
+            const int4 sv = sbuf[e < nbuf ? e : LFAR];
+            const float fx = (float)sv.x, fy = (float)sv.y, fz = (float)sv.z;
+            // sink k's position is read from LDS in its own step
+            // (48 positions kept live would cost occupancy); its
+            // count lives in lane k of cntv
+            auto sink_test = [&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const float4 sk = sinkf[k];
+                const float dx = fx - sk.x, dy = fy - sk.y, dz = fz - sk.z;
+                const bool in = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < cull2s;
+                const unsigned long long m = __ballot(in);
+                const int base = __builtin_amdgcn_readlane(cntv, k);
+                if (in) lst[k * LCAP + base + (int)count_below(m)] = (uint8_t)e;
+                const int nb = base + __popcll(m);
+                asm volatile("v_writelane_b32 %0, %1, %2" : "+v"(cntv) : "s"(nb), "i"(k));
+            };
+            static_for<16>(sink_test);
+        }
+        lds_sync();
+        const int mycnt = __shfl(cntv, slot);
+        const int mx = wave_max(cntv);
+        int tot = cntv;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) tot += __shfl_xor(tot, o);
+        tot = __builtin_amdgcn_readfirstlane(tot);
+        // stream s of sink k takes entries s, s + 4, ... of list k;
+        // the index read one step ahead stays inside the lists'
+        // slack (4 * ceil(LCAP / 4) + 3 < LCAP + 16)
+        const uint8_t* my = lst + slot * LCAP + stream;
+        const int steps = (mx + 3) >> 2;
+        int pidx = stream;
+        int4 sc = sbuf[pidx < mycnt ? (int)my[0] : LFAR];
+#pragma unroll 2
+        for (int i = 0; i < steps; i++) {
+            const int pn = pidx + 4;
+            const int4 sn = sbuf[pn < mycnt ? (int)my[4 * i + 4] : LFAR];
+            pp_pair<false>(B, ox, oy, oz, sc, gx, gy, gz, ph);
+            sc = sn;
+            pidx = pn;
+        }
+        executed += (unsigned long long)tot;
+        nbuf = 0;
+        lds_sync();
+    };
+    for (int nb = 0; nb < 27; nb++) {
+        int jx = cx + (nb % 3) - 1, jy = cy + (nb / 3) % 3 - 1, jz = cz + nb / 9 - 1;
+        jx += (jx < 0) ? C : 0;
+        jx -= (jx >= C) ? C : 0;
+        jy += (jy < 0) ? C : 0;
+        jy -= (jy >= C) ? C : 0;
+        jz += (jz < 0) ? C : 0;
+        jz -= (jz >= C) ? C : 0;
+        const int c2 = B.cell0 + (jz * C + jy) * C + jx;
+        const int sb = a.cell_begin[c2], se = a.cell_begin[c2 + 1];
+        for (int j0 = sb; j0 < se; j0 += 64) {
+            const int j = j0 + lane;
+            bool keep = false;
+            int4 sv = make_int4(0, 0, 0, j);
+            if (j < se) {
+                sv.x = (int)(a.x[j] - rx);
+                sv.y = (int)(a.y[j] - ry);
+                sv.z = (int)(a.z[j] - rz);
+                const float fx = (float)sv.x, fy = (float)sv.y, fz = (float)sv.z;
+                const float ex = fmaxf(fmaxf(lox - fx, fx - hix), 0.f);
+                const float ey = fmaxf(fmaxf(loy - fy, fy - hiy), 0.f);
+                const float ez = fmaxf(fmaxf(loz - fz, fz - hiz), 0.f);
+                keep = fmaf(ex, ex, fmaf(ey, ey, ez * ez)) < cull2s;
+            }
+            const unsigned long long m = __ballot(keep);
+            if (keep) sbuf[nbuf + (int)count_below(m)] = sv;
+            nbuf += __popcll(m);
+            if (nbuf > LFLUSH) flush_lists();
+        }
+    }
+    if (nbuf > 0) flush_lists();
+    // back to box units: g in 2^-64, phi in 2^-32
+    gx *= 0x1p64f;
+    gy *= 0x1p64f;
+    gz *= 0x1p64f;
+    ph *= 0x1p32f;
+}
+
 // WPG = tiles per workgroup, one wave each (1 or 4).  The waves of a
 // workgroup run on one CU and take consecutive tiles of their XCD's run,
 // mostly of one chain cell, so their source loads meet in that CU's L1;
@@ -142,15 +496,12 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
     static_assert(WPG == 1 || (WPG == 4 && !PERSIST), "several tiles per workgroup: one-shot launch only");
     static_assert(!LISTS || (TS == 16 && !PME), "per-sink lists: 16-sink tiles, kick_treepm's law");
     constexpr int SPLIT = 64 / TS;  // source streams per wave
-    constexpr int NSB = LISTS ? LSBUF : SBUF;
-    constexpr int FLUSH_AT = LISTS ? LFLUSH : SBUF - 2 * 64;
-    __shared__ int4 sbufs[WPG][NSB];
-    __shared__ uint8_t lsts[WPG][LISTS ? 16 * LCAP + 16 : 4];
-    __shared__ float4 sinkfs[WPG][LISTS ? 16 : 1];
+    // staged sources: the far and near lists, or with LISTS the staged
+    // sources, the sinks' lists and the sinks
+    constexpr int NSB = FAR_CAP + NEAR_CAP > LSBUF + 16 + LCAP + 1 ? FAR_CAP + NEAR_CAP : LSBUF + 16 + LCAP + 1;
+    __shared__ int4 sbufs[WPG][LISTS ? NSB : FAR_CAP + NEAR_CAP];
     const int wslot = WPG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int4* const sbuf = sbufs[wslot];
-    uint8_t* const lst = lsts[wslot];
-    float4* const sinkf = sinkfs[wslot];
     // the staged list is written and read by the lanes of one wave
     auto lds_sync = [&]() {
         if constexpr (WPG == 1) {
@@ -213,154 +564,26 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
                 return;
         }
         {
-            const int ox = (int)(px - rx), oy = (int)(py - ry), oz = (int)(pz - rz);
             float gx = 0.f, gy = 0.f, gz = 0.f, ph = 0.f;
             if (!(a.flags & TPM_SKIP_PP)) {
-                // Tile bounding box as floats.  float(int32) rounds by <= 64
-                // raw units, so box distances below carry <= 192 units of
-                // error, inside the 512-unit margin of cull2s: the test never
-                // drops a source with r < rcut to any sink.
-                const float lox = (float)wave_min(active ? ox : INT_MAX), hix = (float)wave_max(active ? ox : INT_MIN);
-                const float loy = (float)wave_min(active ? oy : INT_MAX), hiy = (float)wave_max(active ? oy : INT_MIN);
-                const float loz = (float)wave_min(active ? oz : INT_MAX), hiz = (float)wave_max(active ? oz : INT_MIN);
                 const int C = B.C;
                 const int cid = tile.x - B.cell0;
                 const int cx = cid % C, cy = (cid / C) % C, cz = cid / (C * C);
-                const bool cull = B.cull != 0;
-                const float cull2s = B.cull2s;
-                int nbuf = 0;
                 unsigned long long executed = 0ull;
                 const int nact = __popcll(amask & ((TS == 64) ? ~0ull : ((1ull << TS) - 1)));
-                // Far dummy of the per-sink lists: offset -2^31 on every
-                // axis, i.e. at least 1/2 - 1/C of the box from every sink of
-                // the tile (a sink lies within one cell of the tile's first
-                // particle), so r > rcut whenever culling is on (C >= 5).
-                const int4 far = make_int4(INT_MIN, INT_MIN, INT_MIN, -1);
-                // Per-sink lists: the tile's sinks as floats in LDS, read by
-                // every lane alike (an inactive sink sits far from every
-                // source: empty list).
+                bool lists = false;
                 if constexpr (LISTS) {
-                    if (lane < 16)
-                        sinkf[lane] = make_float4(active ? (float)ox : 3.0e9f, active ? (float)oy : 3.0e9f,
-                                                  active ? (float)oz : 3.0e9f, 0.f);
-                    if (lane == 0) sbuf[LFAR] = far;
+                    lists = B.cull != 0;
+                    if (lists)
+                        pp_sum_lists(a, B, cx, cy, cz, (int)(px - rx), (int)(py - ry), (int)(pz - rz), rx, ry, rz,
+                                     active, sbuf, (uint8_t*)(sbuf + LSBUF + 16), (float4*)(sbuf + LSBUF), lds_sync,
+                                     gx, gy, gz, ph, executed);
                 }
-                // Sources in range of no sink cost nothing but the test: a
-                // source joins sink k's list when its float distance to the
-                // sink is inside the cull distance (float(int32) offsets are
-                // off by <= 8 raw units here, far inside the 512-unit margin),
-                // so no pair with r < rcut is dropped and the pair law's own
-                // cutoff decides as before.
-                auto flush_lists = [&]() {
-                    lds_sync();
-                    int cntv = 0;  // lane k < 16: entries of sink k's list
-                    for (int r0 = 0; r0 < nbuf; r0 += 64) {
-                        const int e = r0 + lane;
-                        // lanes past the staged sources test the far dummy,
-                        // which is in range of no sink
-                        const int4 sv = sbuf[e < nbuf ? e : LFAR];
-                        const float fx = (float)sv.x, fy = (float)sv.y, fz = (float)sv.z;
-                        // sink k's position is read from LDS in its own step
-                        // (48 positions kept live would cost occupancy); its
-                        // count lives in lane k of cntv
-                        auto sink_test = [&](auto kc) {
-                            constexpr int k = decltype(kc)::value;
-                            const float4 sk = sinkf[k];
-                            const float dx = fx - sk.x, dy = fy - sk.y, dz = fz - sk.z;
-                            const bool in = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < cull2s;
-                            const unsigned long long m = __ballot(in);
-                            const int base = __builtin_amdgcn_readlane(cntv, k);
-                            if (in) lst[k * LCAP + base + (int)count_below(m)] = (uint8_t)e;
-                            const int nb = base + __popcll(m);
-                            asm volatile("v_writelane_b32 %0, %1, %2" : "+v"(cntv) : "s"(nb), "i"(k));
-                        };
-                        static_for<16>(sink_test);
-                    }
-                    lds_sync();
-                    const int mycnt = __shfl(cntv, slot);
-                    const int mx = wave_max(cntv);
-                    int tot = cntv;
-#pragma unroll
-                    for (int o = 1; o < 16; o <<= 1) tot += __shfl_xor(tot, o);
-                    tot = __builtin_amdgcn_readfirstlane(tot);
-                    // stream s of sink k takes entries s, s + 4, ... of list k;
-                    // the index read one step ahead stays inside the lists'
-                    // slack (4 * ceil(LCAP / 4) + 3 < LCAP + 16)
-                    const uint8_t* my = lst + slot * LCAP + stream;
-                    const int steps = (mx + 3) >> 2;
-                    int pidx = stream;
-                    int4 sc = sbuf[pidx < mycnt ? (int)my[0] : LFAR];
-#pragma unroll 2
-                    for (int i = 0; i < steps; i++) {
-                        const int pn = pidx + 4;
-                        const int4 sn = sbuf[pn < mycnt ? (int)my[4 * i + 4] : LFAR];
-                        pp_pair<PME>(B, ox, oy, oz, sc, gx, gy, gz, ph);
-                        sc = sn;
-                        pidx = pn;
-                    }
-                    executed += (unsigned long long)tot;
-                    nbuf = 0;
-                    lds_sync();
-                };
-                auto flush = [&]() {
-                    if constexpr (LISTS) {
-                        if (cull) {
-                            flush_lists();
-                            return;
-                        }
-                    }
-                    // whole rounds of SPLIT sources, then the streams that
-                    // still have one (no padding source: with C < 8 a
-                    // stand-in placed anywhere can come within rcut of some
-                    // sink, and kick_pme's law has no cutoff at all)
-                    const int full = nbuf / SPLIT * SPLIT;
-                    lds_sync();
-                    int4 s = sbuf[stream];
-                    // the read one round ahead stays below full + 2 SPLIT <=
-                    // FLUSH_AT + 64 + SPLIT < NSB (and below LFAR with lists);
-                    // what it reads past nbuf is not used
-#pragma unroll 2
-                    for (int qq = 0; qq < full; qq += SPLIT) {
-                        const int4 sn = sbuf[qq + SPLIT + stream];
-                        pp_pair<PME>(B, ox, oy, oz, s, gx, gy, gz, ph);
-                        s = sn;
-                    }
-                    if (full + stream < nbuf) pp_pair<PME>(B, ox, oy, oz, s, gx, gy, gz, ph);
-                    executed += (unsigned long long)nbuf * (unsigned long long)nact;
-                    nbuf = 0;
-                    lds_sync();
-                };
-                for (int nb = 0; nb < 27; nb++) {
-                    int jx = cx + (nb % 3) - 1, jy = cy + (nb / 3) % 3 - 1, jz = cz + nb / 9 - 1;
-                    jx += (jx < 0) ? C : 0;
-                    jx -= (jx >= C) ? C : 0;
-                    jy += (jy < 0) ? C : 0;
-                    jy -= (jy >= C) ? C : 0;
-                    jz += (jz < 0) ? C : 0;
-                    jz -= (jz >= C) ? C : 0;
-                    const int c2 = B.cell0 + (jz * C + jy) * C + jx;
-                    const int sb = a.cell_begin[c2], se = a.cell_begin[c2 + 1];
-                    for (int j0 = sb; j0 < se; j0 += 64) {
-                        const int j = j0 + lane;
-                        bool keep = false;
-                        int4 sv = make_int4(0, 0, 0, j);
-                        if (j < se) {
-                            sv.x = (int)(a.x[j] - rx);
-                            sv.y = (int)(a.y[j] - ry);
-                            sv.z = (int)(a.z[j] - rz);
-                            const float fx = (float)sv.x, fy = (float)sv.y, fz = (float)sv.z;
-                            const float ex = fmaxf(fmaxf(lox - fx, fx - hix), 0.f);
-                            const float ey = fmaxf(fmaxf(loy - fy, fy - hiy), 0.f);
-                            const float ez = fmaxf(fmaxf(loz - fz, fz - hiz), 0.f);
-                            keep = !cull || fmaf(ex, ex, fmaf(ey, ey, ez * ez)) < cull2s;
-                        }
-                        const unsigned long long m = __ballot(keep);
-                        if (keep) sbuf[nbuf + (int)count_below(m)] = sv;
-                        nbuf += __popcll(m);
-                        if (nbuf > FLUSH_AT) flush();
-                    }
-                }
-                if (nbuf > 0) flush();
+                if (!lists)
+                    // (kick_pme's sums do not depend on which other particles
+                    // are active, and stay so: its box holds all of the tile)
+                    pp_sum<TS, PME>(a, B, cx, cy, cz, px, py, pz, rx, ry, rz, PME ? valid : active, nact, (float4*)sbuf,
+                                    sbuf + FAR_CAP, lds_sync, gx, gy, gz, ph, executed);
                 // sum the source streams
 #pragma unroll
                 for (int o = TS; o < 64; o <<= 1) {
@@ -370,11 +593,6 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
                     ph += __shfl_xor(ph, o);
                 }
                 if (lane == 0 && cnt) atomicAdd(&cnt[0], executed);
-                // back to box units: g in 2^-64, phi in 2^-32
-                gx *= 0x1p64f;
-                gy *= 0x1p64f;
-                gz *= 0x1p64f;
-                ph *= 0x1p32f;
             }
             {
                 // Then the kick, by each active sink's stream-0 lane, with the
@@ -724,6 +942,30 @@ void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_c
     b->hinv_s = hinv / S;
     b->h2inv_s = (hinv * hinv) / (S * S);
     b->h3inv_s = ((hinv * hinv * hinv) / (S * S)) / S;
+    // pp_far: lengths in far_s units are x sqrt(log2 e).  Offsets span at
+    // most two cells (half a box); a source's float offset is rounded when it
+    // is converted and when it is scaled, a sink's likewise and their
+    // difference once more: 2^-22.5 of the span bounds the sum per axis, and
+    // u's own arithmetic adds less than 2^-22.
+    {
+        const double two32 = 4294967296.0, l2e = 1.4426950408889634;
+        const float fs = (float)(std::sqrt(l2e) / (2.0 * p.rs) / two32);
+        const double fsd = fs;
+        b->far_s = fs;
+        const double nr = (std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * two32 + 2048.0) * fsd;
+        b->far_near2 = (float)(nr * nr * (1.0 + 1e-6));
+        const double cr = (p.rcut * two32 + 2048.0) * fsd;
+        b->far_cull2 = (float)(cr * cr * (1.0 + 1e-6));
+        const double rc = p.rcut * two32, uc = rc * rc * fsd * fsd;
+        const double span = std::min(2.0 / p.chain_dim, 0.5) * two32;
+        const double rel = 2.0 * std::sqrt(3.0) * std::exp2(-22.5) * span / rc + std::exp2(-22.0);
+        b->far_ulo = (float)(uc * (1.0 - rel) * (1.0 - 1e-7));
+        b->far_uhi = (float)(uc * (1.0 + rel) * (1.0 + 1e-7));
+        b->far_wrap = (float)(0x1p31 * fsd * (1.0 - 1e-5));
+        b->far_g = (float)(std::sqrt(l2e) / (4.0 * p.rs * p.rs));
+        b->far_ph = (float)(1.0 / (2.0 * p.rs));
+        b->rcut2i = (uint64_t)std::ceil(rc * rc);
+    }
     b->GM = (float)p.GM;
     b->phi0 = (float)(p.n_total * 4.0 * M_PI * p.rs * p.rs + (35.0 / 16.0) / p.hsoft);
     b->eta = (float)p.eta;

@@ -38,10 +38,11 @@ __device__ __forceinline__ int wave_max(int v) {
 // PME = true: kick_pme_kernel's law instead (kick_pme.cu:280-310): no cutoff,
 // and inside h the plain softened polynomials without the (erfc - 1) terms.
 // pp_law gives the pair's float offset (sink - source) and its force and
-// potential factors; pp_pair adds them to the sink's sums.
+// potential factors; pp_pair adds them to the sink's sums.  cut2s: the cutoff
+// that r2 is compared with.
 template <bool PME>
-__device__ __forceinline__ void pp_law(const tpm_box_dev& a, int ox, int oy, int oz, int4 s, float& dx, float& dy,
-                                       float& dz, float& rinv3, float& rinv1) {
+__device__ __forceinline__ void pp_law(const tpm_box_dev& a, int ox, int oy, int oz, int4 s, float cut2s, float& dx,
+                                       float& dy, float& dz, float& rinv3, float& rinv1) {
     dx = (float)(int)((unsigned)ox - (unsigned)s.x);
     dy = (float)(int)((unsigned)oy - (unsigned)s.y);
     dz = (float)(int)((unsigned)oz - (unsigned)s.z);
@@ -55,7 +56,7 @@ __device__ __forceinline__ void pp_law(const tpm_box_dev& a, int ox, int oy, int
     const float t1 = __builtin_amdgcn_rcpf(fmaf(a.p_inv2rs_s, r, 1.f));
     // exp(-x^2); the cutoff test (kick_treepm.cu:254) zeroes it, which
     // zeroes both erfc and the force factor below.
-    const float e = (PME || r2 < a.rcut2s) ? __builtin_amdgcn_exp2f(r2 * a.e2s) : 0.f;
+    const float e = (PME || r2 < cut2s) ? __builtin_amdgcn_exp2f(r2 * a.e2s) : 0.f;
     const float poly =
         t1 * fmaf(t1, fmaf(t1, fmaf(t1, fmaf(t1, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f),
                   0.254829592f);
@@ -107,11 +108,69 @@ template <bool PME>
 __device__ __forceinline__ void pp_pair(const tpm_box_dev& a, int ox, int oy, int oz, int4 s, float& gx, float& gy,
                                         float& gz, float& ph) {
     float dx, dy, dz, rinv3, rinv1;
-    pp_law<PME>(a, ox, oy, oz, s, dx, dy, dz, rinv3, rinv1);
+    pp_law<PME>(a, ox, oy, oz, s, a.rcut2s, dx, dy, dz, rinv3, rinv1);
     gx = fmaf(-dx, rinv3, gx);
     gy = fmaf(-dy, rinv3, gy);
     gz = fmaf(-dz, rinv3, gz);
     ph -= rinv1;
+}
+
+// Whether the pair at integer offset (ix, iy, iz) is inside the cutoff:
+// squares below 2^62, their sum below 2^64.
+__device__ __forceinline__ bool pp_inside(const tpm_box_dev& a, int ix, int iy, int iz) {
+    const int64_t x = ix, y = iy, z = iz;
+    return (uint64_t)(x * x) + (uint64_t)(y * y) + (uint64_t)(z * z) < a.rcut2i;
+}
+
+// pp_pair with the cutoff decided on the integer offset where the rounding
+// of r2 (four of 2^-24, and rcut2s's own) leaves it open.
+__device__ __forceinline__ void pp_pair_exact(const tpm_box_dev& a, int ox, int oy, int oz, int4 s, float& gx,
+                                              float& gy, float& gz, float& ph) {
+    const int ix = (int)((unsigned)ox - (unsigned)s.x), iy = (int)((unsigned)oy - (unsigned)s.y),
+              iz = (int)((unsigned)oz - (unsigned)s.z);
+    const float fx = (float)ix, fy = (float)iy, fz = (float)iz;
+    const float r2 = fmaf(fx, fx, fmaf(fy, fy, fz * fz));
+    float cut2s = a.rcut2s;
+    if (fabsf(r2 - cut2s) < cut2s * 1e-6f) cut2s = pp_inside(a, ix, iy, iz) ? 2.f * cut2s : 0.f;
+    float dx, dy, dz, rinv3, rinv1;
+    pp_law<false>(a, ox, oy, oz, s, cut2s, dx, dy, dz, rinv3, rinv1);
+    gx = fmaf(-dx, rinv3, gx);
+    gy = fmaf(-dy, rinv3, gy);
+    gz = fmaf(-dz, rinv3, gz);
+    ph -= rinv1;
+}
+
+// The same law for a pair at least FAR_X0 * 2 rs and h apart: no softening,
+// and erfc by one polynomial instead of A&S 7.1.26.  Lengths come scaled so
+// that u = x^2 log2(e), x = r / (2 rs): e = exp2(-u) = exp(-x^2) and
+// y = rsq(u).  erfc(x) / x = e y^2 P(y), P a polynomial of degree 6 in 1 / x
+// (the factors log2(e)^(k/2) are in its coefficients) fitted to erfcx(x) x
+// over x >= 0.71 to 5e-8 of erfc, a third of 7.1.26's error, and valid to
+// any distance (y -> 0 is the asymptotic series' end).  No reciprocal, no
+// int-to-float conversions and constants that are literals: measured issue
+// cycles per wave64 on gfx950 are 2 to 2.7 for multiplies, adds and FMAs, 4.3
+// for the conversion, 8.2 for exp / rsq / rcp and 4.5 for an FMA with an SGPR
+// operand, so 83 cycles per 64 pairs here against 116 for pp_pair (PP stage of a
+// 256^3 kick 25.1 -> 22.2 ms, kick_pme 60^3 16.5 -> 12.8 ms).
+// (dx, dy, dz): source - sink; the caller gates e by the cutoff.
+// Sums: g += (source - sink) F, ph += erfc(x) / x, in far_s units.
+#define FAR_X0 0.72
+__device__ __forceinline__ void pp_far(float dx, float dy, float dz, float u, float e, float& gx, float& gy,
+                                       float& gz, float& ph) {
+    const float y = __builtin_amdgcn_rsqf(u);
+    const float w = y * y;
+    float p = fmaf(y, -4.272549972e-02f, 2.757773399e-01f);
+    p = fmaf(y, p, -7.594215870e-01f);
+    p = fmaf(y, p, 1.130750060f);
+    p = fmaf(y, p, -8.754580617e-01f);
+    p = fmaf(y, p, 3.195298091e-02f);
+    p = fmaf(y, p, 8.133378625e-01f);
+    const float ew = e * w;
+    const float f = ew * fmaf(w, p, 1.128379167f);
+    gx = fmaf(dx, f, gx);
+    gy = fmaf(dy, f, gy);
+    gz = fmaf(dz, f, gz);
+    ph = fmaf(ew, p, ph);
 }
 
 // 6-point quintic weights (kick_treepm.cu:527-549) in Horner form.

@@ -314,7 +314,7 @@ __global__ __launch_bounds__(64, WAVES) void pp_sym_kernel(SymArgs a) {
 #pragma unroll
                         for (int k = 0; k < 4; k++) {
                             float dx, dy, dz, r3, r1;
-                            pp_law<false>(B, (int)p.x, (int)p.y, (int)p.z, sv[k], dx, dy, dz, r3, r1);
+                            pp_law<false>(B, (int)p.x, (int)p.y, (int)p.z, sv[k], B.rcut2s, dx, dy, dz, r3, r1);
                             const int sk = 4 * q + k;
                             const float a3 = sk >= si ? r3 : 0.f, a1 = sk >= si ? r1 : 0.f;
                             const float b3 = sk > si ? r3 : 0.f, b1 = sk > si ? r1 : 0.f;
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(64, WAVES) void pp_sym_kernel(SymArgs a) {
 #pragma unroll
                         for (int k = 0; k < 4; k++) {
                             float dx, dy, dz, r3, r1;
-                            pp_law<false>(B, (int)p.x, (int)p.y, (int)p.z, sv[k], dx, dy, dz, r3, r1);
+                            pp_law<false>(B, (int)p.x, (int)p.y, (int)p.z, sv[k], B.rcut2s, dx, dy, dz, r3, r1);
                             sx = fmaf(-dx, r3, sx);
                             sy = fmaf(-dy, r3, sy);
                             sz = fmaf(-dz, r3, sz);

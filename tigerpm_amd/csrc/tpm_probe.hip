@@ -1,14 +1,13 @@
 // tpm_probe.hip -- the issue-rate ceiling of the direct kernel's pair body.
 //
-// pair_rate_kernel runs pp_pair (the device function pp_kick_kernel uses)
-// with pp_kick_kernel's 16-sink tile layout (lane l: sink l % 16, source
-// stream l / 16), its flush loop (two pairs per trip, the next source read
-// one step ahead from LDS) and its 8-wave launch bound, over 256 sources
-// held in LDS, with nothing else in the loop: no staging, culling or
-// epilogue.  Sources fill a cube of side 2 rcut around the sinks, so about
-// half of the pairs are inside rcut and the softening branch is rare, as in
-// the kernel.  Pairs per second of this loop bound what the kernel's pair
-// loop can reach at the same occupancy.
+// pair_rate_kernel runs pp_far with its cutoff window (nine of ten pairs of
+// pp_kick_kernel) in that kernel's 16-sink tile layout (lane l: sink l % 16,
+// source stream l / 16), its far loop (four pairs per trip) and its 8-wave
+// launch bound, over 256 sources held in LDS, with nothing else in the loop:
+// no staging, culling, near pairs or epilogue.  Sources fill a cube of side
+// 2 rcut around the sinks, so about half of the pairs are inside rcut.  Pairs
+// per second of this loop bound what the kernel's far loop can reach at the
+// same occupancy.
 #include "tpm_pp_device.hpp"
 
 namespace {
@@ -18,34 +17,48 @@ constexpr int PROBE_TS = 16;
 constexpr int PROBE_SPLIT = 64 / PROBE_TS;
 
 __global__ __launch_bounds__(64, 8) void pair_rate_kernel(tpm_box_dev B, int iters, float* __restrict__ out) {
-    __shared__ int4 sbuf[PROBE_SRC + PROBE_SPLIT];
+    __shared__ float4 fbuf[PROBE_SRC];
     const int lane = (int)lane_id();
     const int slot = lane % PROBE_TS, stream = lane / PROBE_TS;
-    const float rc = sqrtf(B.rcut2s);
-    for (int k = lane; k < PROBE_SRC + PROBE_SPLIT; k += 64) {
+    const float rc = sqrtf(B.far_cull2);
+    for (int k = lane; k < PROBE_SRC; k += 64) {
         // a hash of (block, k): offsets uniform in [-rcut, rcut)^3
-        uint32_t h = (uint32_t)(blockIdx.x * (PROBE_SRC + PROBE_SPLIT) + k) * 2654435761u;
-        int c[3];
+        uint32_t h = (uint32_t)(blockIdx.x * PROBE_SRC + k) * 2654435761u;
+        float c[3];
         for (int d = 0; d < 3; d++) {
             h ^= h >> 15;
             h *= 2246822519u;
             h ^= h >> 13;
-            c[d] = (int)((float)(h >> 8) * 0x1p-24f * 2.f * rc - rc);
+            c[d] = (float)(h >> 8) * 0x1p-24f * 2.f * rc - rc;
         }
-        sbuf[k] = make_int4(c[0], c[1], c[2], k);
+        fbuf[k] = make_float4(c[0], c[1], c[2], 0.f);
     }
     __syncthreads();
-    const int ox = slot * 4099 - 32768, oy = 20011 - slot * 3001, oz = slot * 1777;
+    const float fox = (slot * 4099 - 32768) * B.far_s, foy = (20011 - slot * 3001) * B.far_s,
+                foz = slot * 1777 * B.far_s;
+    float ulo = B.far_ulo, uhi = B.far_uhi;
+    asm volatile("" : "+v"(ulo), "+v"(uhi));
     float gx = 0.f, gy = 0.f, gz = 0.f, ph = 0.f;
+    unsigned long long window = 0ull;
     for (int it = 0; it < iters; it++) {
-        int4 s = sbuf[stream];
-#pragma unroll 2
-        for (int qq = 0; qq < PROBE_SRC; qq += PROBE_SPLIT) {
-            const int4 sn = sbuf[qq + PROBE_SPLIT + stream];
-            pp_pair<false>(B, ox, oy, oz, s, gx, gy, gz, ph);
-            s = sn;
+#pragma unroll 1
+        for (int q = 0; q < PROBE_SRC; q += 4 * PROBE_SPLIT) {
+            float4 s[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) s[k] = fbuf[q + k * PROBE_SPLIT + stream];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
+                const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                float e = __builtin_amdgcn_exp2f(-u);
+                const bool in = u < ulo;
+                window |= __ballot(u < uhi) & ~__ballot(in);
+                e = in ? e : 0.f;
+                pp_far(dx, dy, dz, u, e, gx, gy, gz, ph);
+            }
         }
     }
+    if (window) ph += 1e-30f;
     out[blockIdx.x * 64 + lane] = gx + gy + gz + ph;
 }
 
