@@ -50,13 +50,13 @@ extern "C" tpm_status tpm_ctx_destroy(tpm_ctx* ctx) {
     void* bufs[] = {ctx->x,     ctx->y,       ctx->z,        ctx->vx,        ctx->vy,       ctx->vz,    ctx->rung,
                     ctx->gx,    ctx->gy,      ctx->gz,       ctx->pot,       ctx->x2,       ctx->y2,    ctx->z2,
                     ctx->vx2,   ctx->vy2,     ctx->vz2,      ctx->rung2,     ctx->keys,     ctx->keys2, ctx->idx,
-                    ctx->perm,  ctx->sort_tmp, ctx->bounds,  ctx->cell_begin, ctx->tile_cnt, ctx->tile_end,
-                    ctx->tiles, ctx->ntiles,  ctx->scan_tmp, ctx->rho_q,     ctx->rho,      ctx->rho_hat, ctx->rho_hat1,
+                    ctx->perm,  ctx->sort_tmp, ctx->bounds,  ctx->cell_begin, ctx->tile_cnt, ctx->tile_off,
+                    ctx->tiles, ctx->tile_part, ctx->rho_q,     ctx->rho,      ctx->rho_hat, ctx->rho_hat1,
                     ctx->phi,   ctx->green,   ctx->counters, ctx->dscratch, ctx->tree_pos, ctx->tree_tmp,
                     ctx->tree_cnt, ctx->node_begin, ctx->bucket_begin, ctx->tree_part, ctx->tree_flags, ctx->nodes,
                     ctx->buckets, ctx->h2d, ctx->h2d2, ctx->ref_perm, ctx->ref_cid, ctx->ref_cid2, ctx->ref_idx2,
                     ctx->ref_posa, ctx->ref_posb, ctx->ref_inv, ctx->ref_flag, ctx->ref_scan, ctx->ref_scan_tmp,
-                    ctx->ref_tab, ctx->moment_buf, ctx->box_tiles, ctx->box_count, ctx->box_buckets, ctx->tree_moved,
+                    ctx->ref_tab, ctx->moment_buf, ctx->box_buckets, ctx->tree_moved,
                     ctx->gsink, ctx->gsrc, ctx->gmesh, ctx->mesh_force, ctx->green_t};
     for (void* b : bufs)
         if (b) (void)hipFree(b);

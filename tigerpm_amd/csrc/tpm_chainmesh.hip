@@ -9,8 +9,8 @@
 // array, and a dense cell table cell_begin[C^3 + 1] found from the sorted
 // keys.  Cell ranges equal the reference partition's; the in-cell order is
 // deterministic (sub-cell, then previous order) so CPU and GPU agree bit for
-// bit.  Tiles of <= ctx->tile consecutive same-cell particles are the PP
-// work items.
+// bit.  The PP kernel's sink tiles are
+// made from the cells by every kick (tpm_pp.hip).
 #include <cstring>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -104,49 +104,6 @@ __global__ void cell_bounds_kernel(int64_t n, const uint32_t* __restrict__ key, 
 __global__ void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = v;
-}
-
-// Tile order: cells are visited in z-major blocks of TILE_BLOCK^3 cells
-// (blocks z-major, cells z-major inside a block), so the tiles the PP kernel
-// runs close together in time share their 27-cell neighbourhoods: a block's
-// sources (10^3 cells at 512^3, ~2 MB) and its stretch of the potential mesh
-// fit one XCD's L2.  rank(c) is this order's position of cell c, a bijection
-// onto [0, C^3) (edge blocks are smaller).  Each tile is computed
-// independently, so the order changes no result.
-#define TILE_BLOCK 8
-__device__ __forceinline__ int32_t tile_rank(int64_t c, int C) {
-    const int x = (int)(c % C), y = (int)((c / C) % C), z = (int)(c / ((int64_t)C * C));
-    const int bx = x / TILE_BLOCK, by = y / TILE_BLOCK, bz = z / TILE_BLOCK;
-    const int sy = min(TILE_BLOCK, C - by * TILE_BLOCK), sz = min(TILE_BLOCK, C - bz * TILE_BLOCK);
-    const int sx = min(TILE_BLOCK, C - bx * TILE_BLOCK);
-    const int64_t before = (int64_t)bz * TILE_BLOCK * C * C + (int64_t)sz * by * TILE_BLOCK * C +
-                           (int64_t)sz * sy * bx * TILE_BLOCK;
-    const int local = ((z - bz * TILE_BLOCK) * sy + (y - by * TILE_BLOCK)) * sx + (x - bx * TILE_BLOCK);
-    return (int32_t)(before + local);
-}
-
-__global__ void tiles_per_cell_kernel(int64_t ncell, int C, int ts, const int32_t* __restrict__ cell_begin,
-                                      int32_t* __restrict__ nt) {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t cnt = cell_begin[c + 1] - cell_begin[c];
-        nt[tile_rank(c, C)] = (cnt + ts - 1) / ts;
-    }
-}
-__global__ void tiles_write_kernel(int64_t ncell, int C, int ts, const int32_t* __restrict__ cell_begin,
-                                   const int32_t* __restrict__ tile_end, int4* __restrict__ tiles,
-                                   int32_t* __restrict__ ntiles) {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t b = cell_begin[c], e = cell_begin[c + 1];
-        const int32_t nt = (e - b + ts - 1) / ts;
-        const int32_t r = tile_rank(c, C);
-        const int32_t t0 = tile_end[r] - nt;
-        for (int32_t t = 0; t < nt; t++) {
-            const int32_t tb = b + t * ts;
-            const int32_t te = min(tb + ts, e);
-            tiles[t0 + t] = make_int4((int)c, tb, te, 0);
-        }
-        if (r == ncell - 1) *ntiles = tile_end[r];
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -404,25 +361,21 @@ tpm_status tpm_chainmesh_build(tpm_ctx* ctx) {
     }
     if (ncell + 1 > ctx->cells_cap) {
         if (ctx->cell_begin) TPM_HIP(ctx, hipFree(ctx->cell_begin));
-        if (ctx->tile_end) TPM_HIP(ctx, hipFree(ctx->tile_end));
+        if (ctx->tile_off) TPM_HIP(ctx, hipFree(ctx->tile_off));
         if (ctx->tile_cnt) TPM_HIP(ctx, hipFree(ctx->tile_cnt));
+        if (ctx->tile_part) TPM_HIP(ctx, hipFree(ctx->tile_part));
+        ctx->cell_begin = ctx->tile_off = ctx->tile_cnt = ctx->tile_part = nullptr;
+        ctx->cells_cap = 0;
         TPM_HIP(ctx, hipMalloc(&ctx->cell_begin, sizeof(int32_t) * (ncell + 1)));
-        TPM_HIP(ctx, hipMalloc(&ctx->tile_end, sizeof(int32_t) * (ncell + 1)));
+        TPM_HIP(ctx, hipMalloc(&ctx->tile_off, sizeof(int32_t) * (ncell + 1)));
         TPM_HIP(ctx, hipMalloc(&ctx->tile_cnt, sizeof(int32_t) * (ncell + 1)));
+        TPM_HIP(ctx, hipMalloc(&ctx->tile_part, sizeof(int32_t) * (ncell / 2048 + 2)));
         ctx->cells_cap = ncell + 1;
     }
     const int ts = ctx->tile;
-    const int64_t tiles_max = n / ts + ncell + 1;
-    if (tiles_max > ctx->tiles_cap) {
-        if (ctx->tiles) TPM_HIP(ctx, hipFree(ctx->tiles));
-        TPM_HIP(ctx, hipMalloc(&ctx->tiles, sizeof(int4) * tiles_max));
-        ctx->tiles_cap = tiles_max;
-    }
-    if (!ctx->ntiles) TPM_HIP(ctx, hipMalloc(&ctx->ntiles, sizeof(int32_t) * 4));
 
     if (n == 0) {
         fill_i32_kernel<<<grid_for(ncell + 1, 256), 256, 0, s>>>(ctx->cell_begin, ncell + 1, 0);
-        fill_i32_kernel<<<1, 64, 0, s>>>(ctx->ntiles, 1, 0);
         TPM_HIP(ctx, hipGetLastError());
         ctx->chain_valid = true;
         ctx->chain_C = C;
@@ -463,21 +416,6 @@ tpm_status tpm_chainmesh_build(tpm_ctx* ctx) {
     std::swap(ctx->rung, ctx->rung2);
 
     cell_bounds_kernel<<<g, 256, 0, s>>>(n, ctx->keys2, ncell, ctx->cell_begin);
-    // tiles per cell, then their inclusive scan.
-    tiles_per_cell_kernel<<<grid_for(ncell, 256), 256, 0, s>>>(ncell, C, ts, ctx->cell_begin, ctx->tile_cnt);
-    TPM_HIP(ctx, hipGetLastError());
-    size_t need2 = 0;
-    TPM_HIP(ctx, rocprim::inclusive_scan(nullptr, need2, ctx->tile_cnt, ctx->tile_end, (size_t)ncell,
-                                         rocprim::plus<int32_t>(), s));
-    if (need2 > ctx->scan_tmp_bytes) {
-        if (ctx->scan_tmp) TPM_HIP(ctx, hipFree(ctx->scan_tmp));
-        TPM_HIP(ctx, hipMalloc(&ctx->scan_tmp, need2));
-        ctx->scan_tmp_bytes = need2;
-    }
-    TPM_HIP(ctx, rocprim::inclusive_scan(ctx->scan_tmp, need2, ctx->tile_cnt, ctx->tile_end, (size_t)ncell,
-                                         rocprim::plus<int32_t>(), s));
-    tiles_write_kernel<<<grid_for(ncell, 256), 256, 0, s>>>(ncell, C, ts, ctx->cell_begin, ctx->tile_end, ctx->tiles,
-                                                            ctx->ntiles);
     TPM_HIP(ctx, hipGetLastError());
     ctx->chain_valid = true;
     ctx->chain_C = C;
@@ -724,27 +662,6 @@ __global__ __launch_bounds__(256) void bcell_order_kernel(int32_t ncell, const i
 }
 
 
-__global__ void btiles_count_kernel(int32_t ncell, int ts, const int32_t* __restrict__ cell_begin,
-                                    int32_t* __restrict__ nt) {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * blockDim.x)
-        nt[c] = (cell_begin[c + 1] - cell_begin[c] + ts - 1) / ts;
-}
-
-// Tiles (global cell, begin, end, box) in cell order.
-__global__ void btiles_write_kernel(int32_t ncell, int ts, int nbox, const tpm_box_dev* __restrict__ boxes,
-                                    const int32_t* __restrict__ cell_begin, const int32_t* __restrict__ tile_off,
-                                    int4* __restrict__ tiles) {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * blockDim.x) {
-        const int box = tpm_upper_index(nbox, c, [&](int k) { return (int64_t)boxes[k].cell0; });
-        const int32_t b = cell_begin[c], e = cell_begin[c + 1];
-        const int32_t t0 = tile_off[c];
-        for (int32_t t = 0; b + t * ts < e; t++) {
-            const int32_t tb = b + t * ts;
-            tiles[t0 + t] = make_int4((int)c, tb, min(tb + ts, e), box);
-        }
-    }
-}
-
 }  // namespace
 
 // Exclusive scan of in[0, n) into out[0, n] (out[n] = total) with the
@@ -768,7 +685,6 @@ tpm_status tpm_batch_chainmesh(tpm_batch* bt, const tpm_batch_layout& L) {
     hipStream_t s = bt->stream;
     const int32_t ncell = L.ncell;
     const int64_t n = L.n_arena;
-    const int ts = bt->tune.tile_sinks;
     // counts of the live cells and of the trash cell ncell
     bfill_i32_kernel<<<grid_for(ncell + 1, 256), 256, 0, s>>>(bt->cnt, ncell + 1, 0);
     if (n > 0)
@@ -796,16 +712,6 @@ tpm_status tpm_batch_chainmesh(tpm_batch* bt, const tpm_batch_layout& L) {
     std::swap(bt->vy, bt->vy2);
     std::swap(bt->vz, bt->vz2);
     std::swap(bt->rung, bt->rung2);
-    // tiles of <= ts sinks per cell
-    if (ncell > 0) {
-        btiles_count_kernel<<<grid_for(ncell, 256), 256, 0, s>>>(ncell, ts, bt->cell_begin, bt->tile_cnt);
-        TPM_HIP(bt, hipGetLastError());
-        TPM_TRY(tpm_scan_i32(bt->err, s, bt->tile_cnt, ncell, bt->scan_part, bt->tile_off));
-        btiles_write_kernel<<<grid_for(ncell, 256), 256, 0, s>>>(ncell, ts, L.nbox, bt->d_boxes, bt->cell_begin,
-                                                                 bt->tile_off, bt->tiles);
-    } else {
-        bfill_i32_kernel<<<1, 64, 0, s>>>(bt->tile_off, 1, 0);
-    }
     TPM_HIP(bt, hipGetLastError());
     return TPM_OK;
 }

@@ -10,6 +10,7 @@
 constexpr int TPM_COUNTER_SLOTS = 64;
 constexpr int TPM_COUNTER_STRIDE = 16;
 constexpr int TPM_COUNTER_WORDS = TPM_COUNTER_SLOTS * TPM_COUNTER_STRIDE;
+constexpr int TPM_COUNTER_TILES = 4;  // word of slot 0: tiles of the kicked cells' particles (candidate_pairs_kernel)
 
 // The counters of all slots (h: TPM_COUNTER_WORDS words copied from the
 // device) -> out[0] executed pairs, [1] max rung, [2] candidate pairs,
@@ -115,6 +116,7 @@ struct tpm_box_dev {
     float far_ulo, far_uhi;     // the cutoff as u, less and more than any rounding of u
     float far_wrap;             // largest |offset| + box half width whose differences cannot wrap
     float far_g, far_ph;        // sums of pp_far -> box units
+    uint32_t cell_w;            // 2^32 / C: cell k's float positions are offsets from k cell_w + cell_w / 2
     uint64_t rcut2i;            // a pair is inside the cutoff when its squared raw offset is below this
     // kick epilogue
     float GM, phi0, eta, t0, scale, hsoft;
@@ -162,13 +164,16 @@ struct tpm_ctx {
     uint32_t* bounds = nullptr;  // C split planes (raw values)
     int32_t* cell_begin = nullptr;
     int64_t cells_cap = 0;
-    int32_t* tile_cnt = nullptr;  // tiles per cell
-    int32_t* tile_end = nullptr;  // inclusive scan of tile_cnt
-    int4* tiles = nullptr;        // (cell id, begin, end, 0)
+    // The direct kernel's sink tiles, made by every kick (tpm_pp_tiles):
+    // tile t holds the particles order[begin .. end) (order: the sort's idx
+    // buffer) of one cell.  The float positions lie in the second buffer set
+    // (x2, y2, z2), free between chain-mesh builds.
+    int32_t* tile_cnt = nullptr;   // tiles per cell
+    int32_t* tile_off = nullptr;   // exclusive scan of tile_cnt, then their number
+    int32_t* tile_part = nullptr;  // scan scratch
+    int4* tiles = nullptr;         // (cell id, begin, end, 0)
     int64_t tiles_cap = 0;
-    int32_t* ntiles = nullptr;    // device scalar
-    void* scan_tmp = nullptr;
-    size_t scan_tmp_bytes = 0;
+    int64_t fpos_epoch = -1;       // the chain-mesh build whose float positions are there
     bool chain_valid = false;
     int chain_C = 0;
     int tile = 16;        // sinks per PP tile: 16, 32 or 64 (tuning)
@@ -255,9 +260,6 @@ struct tpm_ctx {
     // Kicks restricted to a box of chain cells (tpm_kick_box) and the
     // device budget that splits them (tpm_set_budget).
     int64_t budget = 0;              // bytes of one kick's working set; 0 = no limit
-    int4* box_tiles = nullptr;       // the tiles of the box being kicked
-    int64_t box_tiles_cap = 0;
-    int32_t* box_count = nullptr;    // device scalar: tiles in box_tiles
     int32_t* box_buckets = nullptr;  // tree walk: the buckets of the box
     int64_t box_buckets_cap = 0;
     std::vector<int32_t> h_cells;    // host copy of cell_begin ...
@@ -565,8 +567,8 @@ struct tpm_cell_box {
 tpm_status tpm_tree_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int first_call, unsigned flags,
                          tpm_stats* stats, const tpm_cell_box* box = nullptr);
 tpm_status tpm_pm_solve(tpm_ctx* ctx);
-// The direct kernel over every tile, or (box != nullptr) over the box_tiles
-// tiles of the box's cells (ntiles_box of them).
+// The direct kernel over every cell's sinks, or (box != nullptr) over those of
+// the box's cells (at most ntiles_box tiles).
 bool tpm_pp_sym_eligible(const tpm_ctx* ctx, int min_rung, unsigned flags, const tpm_cell_box* box);
 tpm_status tpm_pp_kick_sym(tpm_ctx* ctx, double scale, double t0, int first_call, unsigned flags, tpm_stats* stats);
 tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int first_call, unsigned flags,
@@ -592,6 +594,8 @@ tpm_status tpm_ewald_noalloc_run(tpm_ctx* ctx, int64_t ns, const uint32_t* spx, 
                                  const uint32_t* spz, double alpha, double* phi, double* gx, double* gy, double* gz);
 tpm_status tpm_ic_zeldovich_run(tpm_ctx* ctx, int n_side, uint64_t seed, double rms_disp, double spectral_index);
 tpm_status tpm_ic_uniform_run(tpm_ctx* ctx, int64_t n, uint64_t seed);
+// Exclusive scan (tpm_chainmesh.hip).
+tpm_status tpm_scan_i32(std::string& err, hipStream_t s, const int32_t* in, int64_t n, int32_t* part, int32_t* out);
 tpm_status tpm_fill_u64(tpm_ctx* ctx, unsigned long long* p, int64_t n);
 
 // FP64 momentum / energy reductions (tpm_moments.hip).  part holds

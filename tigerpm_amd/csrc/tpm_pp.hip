@@ -1,8 +1,8 @@
 // tpm_pp.hip -- fused short-range PP + mesh interpolation + kick.
 //
 // Reference: kick_treepm_kernel (kick_treepm.cu:460-759) and kick_pme_kernel
-// (kick_pme.cu:128-357).  Work item here = one tile of <= TS consecutive
-// sinks of one chain cell, processed by one wave64: lane l holds sink
+// (kick_pme.cu:128-357).  Work item here = one tile of <= TS active
+// sinks of one chain cell (tpm_tiles.hip), processed by one wave64: lane l holds sink
 // l % TS and walks source stream l / TS (64 / TS streams over one shared
 // source list), the streams are summed at the end.
 //
@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "tpm_pp_device.hpp"
+#include "tpm_tiles.hpp"
 
 #include <climits>
 
@@ -68,8 +69,12 @@ struct PPArgs {
     float* __restrict__ gz;
     float* __restrict__ pot;
     const int32_t* __restrict__ cell_begin;
+    const float* __restrict__ fx;   // float offsets from the cells' centres (tpm_float_positions)
+    const float* __restrict__ fy;
+    const float* __restrict__ fz;
     const int4* __restrict__ tiles;
     const int32_t* __restrict__ ntiles;
+    const uint32_t* __restrict__ order;  // the particles of a tile: order[tile.y .. tile.z)
     const float4* __restrict__ mesh;  // mesh force and potential per sink, made before the launch
                                       // by mesh_force_kernel (nullptr: no mesh term)
     unsigned long long* __restrict__ counters;
@@ -111,6 +116,24 @@ __device__ __forceinline__ tpm_box_dev tile_box(const PPArgs& a, int w) {
     } else {
         return a.box0;
     }
+}
+
+// The same record, read through the argument block la (the launch's PPArgs).
+template <bool BATCH>
+__device__ __forceinline__ tpm_box_dev late_box(const __attribute__((address_space(4))) PPArgs* la, int w) {
+    constexpr int NW = (int)(sizeof(tpm_box_dev) / 4);
+    using cword = const __attribute__((address_space(4))) int;
+    cword* src;
+    if constexpr (BATCH)
+        src = (cword*)(la->boxes + __builtin_amdgcn_readfirstlane(w));
+    else
+        src = (cword*)&la->box0;
+    int words[NW];
+#pragma unroll
+    for (int k = 0; k < NW; k++) words[k] = src[k];
+    tpm_box_dev b;
+    __builtin_memcpy(&b, words, sizeof b);
+    return b;
 }
 
 // f(integral_constant<int, k>) for k = 0 .. N-1, k a constant expression
@@ -156,14 +179,13 @@ __device__ __forceinline__ int tile_max(int v) {
 
 // The short-range sums of one tile, by one wave: lane l has sink l % TS (raw
 // position px, py, pz) and walks stream l / TS.  The sources are those of the
-// 27 cells around cell (cx, cy, cz), whose x neighbours are contiguous in
-// memory: 9 rows of up to 3 cells, each a run of particles (two where the
-// row wraps), taken 64 at a time.  Each source is tested against the box of
-// the tile's active sinks (centre and half widths, in far_s units):
+// 27 cells around cell (cx, cy, cz), 64 at a time, as float offsets from
+// their cell's centre: one FMA per axis makes them offsets from the centre of
+// the tile's box in far_s units.  Each source is tested against that box:
 //   beyond the cutoff (far_cull2, a margin of 2048 raw units over rcut, float
 //     rounding stays below 600): dropped;
-//   within far_near2 of the box: near list, as int32 offsets from the centre,
-//     evaluated with the general law (pp_pair);
+//   within far_near2 of the box: near list, as int32 offsets from the centre
+//     (made from the raw positions), evaluated with the general law (pp_pair);
 //   else: far list, as float offsets, evaluated with pp_far.  Every pair of a
 //     far source is at least FAR_X0 2 rs and h apart.
 // At 512^3 nine pairs of ten are far ones.
@@ -207,77 +229,80 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
     // kept in vector registers: an SGPR operand costs a VALU instruction half its rate
     float ulo = B.far_ulo, uhi = B.far_uhi;
     asm volatile("" : "+v"(ulo), "+v"(uhi));
-    // lane l < 18: run l & 1 of row l >> 1 (0: the cells cx - 1 .. cx + 1 that
-    // do not wrap, 1: the one that does)
+    // lane l < 27: neighbour cell l, its particles and its centre's offset
+    // from the box's
     int rb = 0, re = 0;
-    if (lane < 18) {
-        const int r = lane >> 1;
-        int jy = cy + r % 3 - 1, jz = cz + r / 3 - 1;
+    float lx = 0.f, ly = 0.f, lz = 0.f;
+    if (lane < 27) {
+        int jx = cx + lane % 3 - 1, jy = cy + (lane / 3) % 3 - 1, jz = cz + lane / 9 - 1;
+        jx += jx < 0 ? C : (jx >= C ? -C : 0);
         jy += jy < 0 ? C : (jy >= C ? -C : 0);
         jz += jz < 0 ? C : (jz >= C ? -C : 0);
-        int x0 = max(cx - 1, 0), x1 = min(cx + 1, C - 1);
-        if (lane & 1) {
-            x0 = cx == 0 ? C - 1 : 0;
-            x1 = cx == 0 || cx == C - 1 ? x0 : -1;  // no wrap: an empty run
-        }
-        const int row = B.cell0 + (jz * C + jy) * C;
-        rb = a.cell_begin[row + x0];
-        re = a.cell_begin[row + x1 + 1];
+        const int c2 = B.cell0 + (jz * C + jy) * C + jx;
+        rb = a.cell_begin[c2];
+        re = a.cell_begin[c2 + 1];
+        const uint32_t w = B.cell_w;
+        lx = (float)(int)((uint32_t)jx * w + w / 2 - qx) * fs;
+        ly = (float)(int)((uint32_t)jy * w + w / 2 - qy) * fs;
+        lz = (float)(int)((uint32_t)jz * w + w / 2 - qz) * fs;
     }
+    const uint32_t lane4 = 4u * (uint32_t)lane;
+    float fsv = fs;
+    asm volatile("" : "+v"(fsv));
     gx = gy = gz = ph = 0.f;
     float ngx = 0.f, ngy = 0.f, ngz = 0.f, nph = 0.f;
     int nfar = 0, nnear = 0;
-    int run = -1, j0 = 0, je = 0;
-    bool more = true;
-    while (more) {
-        // stage until a list is nearly full or the sources end
-        for (;;) {
-            if (j0 >= je) {
-                do {
-                    run++;
-                    if (run == 18) break;
-                    j0 = __builtin_amdgcn_readlane(rb, run);
-                    je = __builtin_amdgcn_readlane(re, run);
-                } while (j0 >= je);
-                if (run == 18) {
-                    more = false;
-                    break;
-                }
+    int cell = -1, j0 = 0, je = 0;
+    float cxo = 0.f, cyo = 0.f, czo = 0.f;
+    for (;;) {
+        // 64 sources, or after the last cell none
+        bool more = true;
+        while (j0 >= je) {
+            if (++cell == 27) {
+                more = false;
+                break;
             }
+            j0 = __builtin_amdgcn_readlane(rb, cell);
+            je = __builtin_amdgcn_readlane(re, cell);
+            cxo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lx), cell));
+            cyo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ly), cell));
+            czo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lz), cell));
+        }
+        if (more) {
+            // lanes past the cell's end read its last particle and are masked
+            const int left = je - j0;
+            const unsigned long long valid = left >= 64 ? ~0ull : (1ull << left) - 1ull;
+            const uint32_t off = min(lane4, 4u * (uint32_t)(left - 1));
+            const float fx = fmaf(*(const float*)((const char*)(a.fx + j0) + off), fsv, cxo);
+            const float fy = fmaf(*(const float*)((const char*)(a.fy + j0) + off), fsv, cyo);
+            const float fz = fmaf(*(const float*)((const char*)(a.fz + j0) + off), fsv, czo);
+            const float ex = fmaxf(fabsf(fx) - hx, 0.f), ey = fmaxf(fabsf(fy) - hy, 0.f),
+                        ez = fmaxf(fabsf(fz) - hz, 0.f);
+            const float d2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+            unsigned long long mn = __ballot(d2 < B.far_near2), mf;
+            if (cull) {
+                mf = __ballot(d2 < B.far_cull2) & ~mn & valid;
+            } else {
+                // a difference of float offsets does not wrap round the
+                // box as the int32 one does: sources for which it would
+                // (C < 5) take the general law
+                mn |= __ballot(fmaxf(fabsf(fx) + hx, fmaxf(fabsf(fy) + hy, fabsf(fz) + hz)) > B.far_wrap);
+                mf = ~mn & valid;
+            }
+            mn &= valid;
             const int j = j0 + lane;
-            j0 += 64;
-            bool far = false, near = false;
-            int dx = 0, dy = 0, dz = 0;
-            float fx = 0.f, fy = 0.f, fz = 0.f;
-            if (j < je) {
-                dx = (int)(a.x[j] - qx);
-                dy = (int)(a.y[j] - qy);
-                dz = (int)(a.z[j] - qz);
-                fx = (float)dx * fs;
-                fy = (float)dy * fs;
-                fz = (float)dz * fs;
-                const float ex = fmaxf(fabsf(fx) - hx, 0.f), ey = fmaxf(fabsf(fy) - hy, 0.f),
-                            ez = fmaxf(fabsf(fz) - hz, 0.f);
-                const float d2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
-                near = d2 < B.far_near2;
-                if (cull) {
-                    far = !near && d2 < B.far_cull2;
-                } else {
-                    // a difference of float offsets does not wrap round the
-                    // box as the int32 one does: sources for which it would
-                    // (C < 5) take the general law
-                    near = near || fmaxf(fabsf(fx) + hx, fmaxf(fabsf(fy) + hy, fabsf(fz) + hz)) > B.far_wrap;
-                    far = !near;
-                }
-            }
-            const unsigned long long mf = __ballot(far), mn = __ballot(near);
-            if (far) fbuf[nfar + (int)count_below(mf)] = make_float4(fx, fy, fz, __int_as_float(j));
+            if (__builtin_amdgcn_inverse_ballot_w64(mf))
+                fbuf[__builtin_amdgcn_mbcnt_hi((unsigned)(mf >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mf, nfar))] =
+                    make_float4(fx, fy, fz, __int_as_float(j));
             nfar += __popcll(mf);
             if (mn) {
-                if (near) nbuf[nnear + (int)count_below(mn)] = make_int4(dx, dy, dz, j);
+                if (__builtin_amdgcn_inverse_ballot_w64(mn))
+                    nbuf[__builtin_amdgcn_mbcnt_hi((unsigned)(mn >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)mn, nnear))] =
+                        make_int4((int)(a.x[j] - qx), (int)(a.y[j] - qy), (int)(a.z[j] - qz), j);
                 nnear += __popcll(mn);
             }
-            if (nfar > FAR_AT || nnear > NEAR_AT) break;
+            j0 += 64;
         }
         if (nfar > FAR_AT || (!more && nfar > 0)) {
             // Whole blocks of 4 rounds (four pairs in flight per lane: 83
@@ -344,6 +369,7 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
             nnear = 0;
             lds_sync();
         }
+        if (!more) break;
     }
     // box units: pp_pair's sums are in 2^-32 units, pp_far's in far_s units
     gx = fmaf(ngx, 0x1p64f, gx * B.far_g);
@@ -539,22 +565,17 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
         }
         const int4 tile = a.tiles[t];
         const tpm_box_dev B = tile_box<BATCH>(a, tile.w);
-        unsigned long long* const cnt =
-            a.counters ? a.counters + TPM_COUNTER_STRIDE * (blockIdx.x % TPM_COUNTER_SLOTS) : nullptr;
         const int lane = (int)lane_id();
         const int slot = lane % TS;
         const int stream = lane / TS;
-        const int i = tile.y + slot;
-        const bool valid = i < tile.z;
-        const uint32_t rx = a.x[tile.y], ry = a.y[tile.y], rz = a.z[tile.y];
-        uint32_t px = rx, py = ry, pz = rz;
-        int r = 0;
-        if (valid) {
-            px = a.x[i];
-            py = a.y[i];
-            pz = a.z[i];
-            r = a.rung[i];
-        }
+        const bool valid = tile.y + slot < tile.z;
+        const int i = (int)a.order[valid ? tile.y + slot : tile.y];
+        const uint32_t px = a.x[i], py = a.y[i], pz = a.z[i];
+        const int r = a.rung[i];
+        // the tile's first sink: the origin of its sinks' offsets
+        const uint32_t rx = (uint32_t)__builtin_amdgcn_readfirstlane((int)px),
+                       ry = (uint32_t)__builtin_amdgcn_readfirstlane((int)py),
+                       rz = (uint32_t)__builtin_amdgcn_readfirstlane((int)pz);
         const bool active = valid && r >= B.min_rung;
         const unsigned long long amask = __ballot(active);
         if (amask == 0ull) {
@@ -565,11 +586,11 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
         }
         {
             float gx = 0.f, gy = 0.f, gz = 0.f, ph = 0.f;
-            if (!(a.flags & TPM_SKIP_PP)) {
+            unsigned long long executed = 0ull;
+            {
                 const int C = B.C;
                 const int cid = tile.x - B.cell0;
                 const int cx = cid % C, cy = (cid / C) % C, cz = cid / (C * C);
-                unsigned long long executed = 0ull;
                 const int nact = __popcll(amask & ((TS == 64) ? ~0ull : ((1ull << TS) - 1)));
                 bool lists = false;
                 if constexpr (LISTS) {
@@ -592,29 +613,84 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
                     gz += __shfl_xor(gz, o);
                     ph += __shfl_xor(ph, o);
                 }
-                if (lane == 0 && cnt) atomicAdd(&cnt[0], executed);
             }
             {
                 // Then the kick, by each active sink's stream-0 lane, with the
-                // mesh force and potential made before the launch.
-                const tpm_kick_out o{a.gx, a.gy, a.gz, a.pot, a.vx, a.vy, a.vz, a.rung, cnt};
+                // mesh force and potential made before the launch.  What only
+                // the kick needs -- the output arrays and the epilogue's
+                // constants -- is read from the argument block here, through
+                // a pointer that the compiler cannot look through, and the
+                // sink's index and rung are read again: kept over the pair
+                // loop they take the SGPRs and VGPRs that it needs.
+                using cbyte = const __attribute__((address_space(4))) char;
+                using cargs = const __attribute__((address_space(4))) PPArgs;
+                cbyte* args = (cbyte*)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(args));
+                cargs* const la = (cargs*)args;
+                const tpm_box_dev E = late_box<BATCH>(la, tile.w);
+                unsigned long long* const lc = la->counters;
+                const tpm_kick_out o{la->gx,
+                                     la->gy,
+                                     la->gz,
+                                     la->pot,
+                                     la->vx,
+                                     la->vy,
+                                     la->vz,
+                                     la->rung,
+                                     lc ? lc + TPM_COUNTER_STRIDE * (blockIdx.x % TPM_COUNTER_SLOTS) : nullptr};
+                if (lane == 0 && o.counters) atomicAdd(&o.counters[0], executed);
                 int nr = -1;
                 if (active && stream == 0) {
+                    const int i = (int)la->order[tile.y + slot];
+                    const int r = la->rung[i];
                     float pgx = 0.f, pgy = 0.f, pgz = 0.f, pph = 0.f;
-                    if (a.mesh) {
-                        const float4 m = a.mesh[i];
+                    if (la->mesh) {
+                        const float4 m = la->mesh[i];
                         pgx = m.x;
                         pgy = m.y;
                         pgz = m.z;
                         pph = m.w;
                     }
-                    nr = kick_epilogue(B, a.flags, o, i, r, pgx, pgy, pgz, pph, gx, gy, gz, ph);
+                    nr = kick_epilogue(E, la->flags, o, i, r, pgx, pgy, pgz, pph, gx, gy, gz, ph);
                 }
                 max_rung_update(o, nr);
             }
         }
         if constexpr (!PERSIST) return;
     }
+}
+
+// The kick alone (TPM_SKIP_PP): the epilogue of every active particle of the
+// cells in [lo, hi) from its mesh term, one wave per cell and one lane per
+// particle (through 16-sink tiles, with a quarter of the lanes, it took
+// 0.44 ms at 256^3).
+template <bool BATCH>
+__global__ __launch_bounds__(256) void kick_only_kernel(PPArgs a, int ncell, int nbox, int3 lo, int3 hi) {
+    const int lane = (int)lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
+    const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
+    unsigned long long* const cnt =
+        a.counters ? a.counters + TPM_COUNTER_STRIDE * (blockIdx.x % TPM_COUNTER_SLOTS) : nullptr;
+    const tpm_kick_out o{a.gx, a.gy, a.gz, a.pot, a.vx, a.vy, a.vz, a.rung, cnt};
+    int nr = -1;
+    for (int c = wave; c < ncell; c += nwave) {
+        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
+        if (b == e) continue;
+        int box = 0;
+        if constexpr (BATCH) box = tpm_upper_index(nbox, c, [&](int k) { return (int64_t)a.boxes[k].cell0; });
+        const tpm_box_dev B = tile_box<BATCH>(a, box);
+        if (!BATCH) {
+            const int C = B.C, x = c % C, y = (c / C) % C, z = c / (C * C);
+            if (x < lo.x || x >= hi.x || y < lo.y || y >= hi.y || z < lo.z || z >= hi.z) continue;
+        }
+        for (int i = b + lane; i < e; i += 64) {
+            const int r = a.rung[i];
+            if (r < B.min_rung) continue;
+            const float4 m = a.mesh ? a.mesh[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            nr = max(nr, kick_epilogue(B, a.flags, o, i, r, m.x, m.y, m.z, m.w, 0.f, 0.f, 0.f, 0.f));
+        }
+    }
+    max_rung_update(o, nr);
 }
 
 // The mesh force and potential of every active sink of one box, as the PP
@@ -796,10 +872,11 @@ __global__ __launch_bounds__(256) void bmesh_force_kernel(const uint32_t* __rest
 // the global cells [0, ncell); with a box table, cell c belongs to the last
 // box whose cell0 <= c.
 // A single box's sinks may be restricted to the cells [lo, hi).
+// tiles (may be null): the cells' particles in tiles of ts, summed.
 __global__ void candidate_pairs_kernel(int64_t ncell, int nbox, const tpm_box_dev* __restrict__ boxes, int C0,
                                        const int32_t* __restrict__ cell_begin, unsigned long long* __restrict__ out,
-                                       int3 lo = make_int3(0, 0, 0), int3 hi = make_int3(INT_MAX, INT_MAX, INT_MAX)) {
-    unsigned long long acc = 0;
+                                       int ts = 1, unsigned long long* __restrict__ tiles = nullptr, int3 lo = make_int3(0, 0, 0), int3 hi = make_int3(INT_MAX, INT_MAX, INT_MAX)) {
+    unsigned long long acc = 0, nt = 0;
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * blockDim.x) {
         int C = C0;
         int64_t base = 0;
@@ -812,6 +889,7 @@ __global__ void candidate_pairs_kernel(int64_t ncell, int nbox, const tpm_box_de
         const int cx = (int)(l % C), cy = (int)((l / C) % C), cz = (int)(l / ((int64_t)C * C));
         if (cx < lo.x || cx >= hi.x || cy < lo.y || cy >= hi.y || cz < lo.z || cz >= hi.z) continue;
         const int64_t nc = cell_begin[c + 1] - cell_begin[c];
+        nt += (unsigned long long)((nc + ts - 1) / ts);
         int64_t s = 0;
         for (int nb = 0; nb < 27; nb++) {
             const int jx = (cx + nb % 3 - 1 + C) % C, jy = (cy + (nb / 3) % 3 - 1 + C) % C,
@@ -822,33 +900,8 @@ __global__ void candidate_pairs_kernel(int64_t ncell, int nbox, const tpm_box_de
         acc += (unsigned long long)(nc * s);
     }
     atomicAdd(out, acc);
+    if (tiles) atomicAdd(tiles, nt);
 }
-
-// The tiles whose cell lies in [lo, hi), appended to out (one atomic per
-// wave).  The order of out does not matter: every tile is computed on its
-// own.
-__global__ void box_tiles_kernel(const int4* __restrict__ tiles, const int32_t* __restrict__ ntiles, int C, int3 lo,
-                                 int3 hi, int4* __restrict__ out, int32_t* __restrict__ count) {
-    const int nt = *ntiles;
-    const int lane = (int)lane_id();
-    for (int64_t t0 = (int64_t)blockIdx.x * blockDim.x; t0 < nt; t0 += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t t = t0 + threadIdx.x;
-        int4 tile = make_int4(0, 0, 0, 0);
-        bool in = false;
-        if (t < nt) {
-            tile = tiles[t];
-            const int cx = tile.x % C, cy = (tile.x / C) % C, cz = tile.x / (C * C);
-            in = cx >= lo.x && cx < hi.x && cy >= lo.y && cy < hi.y && cz >= lo.z && cz < hi.z;
-        }
-        const unsigned long long m = __ballot(in);
-        int base = 0;
-        if (lane == 0 && m) base = atomicAdd(count, __popcll(m));
-        base = __shfl(base, 0);
-        if (in) out[base + (int)count_below(m)] = tile;
-    }
-}
-
-__global__ void set_i32_kernel(int32_t* p, int32_t v) { *p = v; }
 
 // Drift of every live particle by v * t0 of its box (fixed32, periodic):
 // raw += round(v t0 2^32) mod 2^32.
@@ -911,10 +964,15 @@ static void pp_launch(int ts, bool persistent, unsigned grid, hipStream_t s, con
 
 }  // namespace
 
+// One wave per cell, 4 per workgroup, up to a grid that fills the chip many
+// times over.
+static unsigned cell_grid(int64_t ncell) { return (unsigned)std::min<int64_t>((ncell + 3) / 4, 65536); }
+
 void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_call, double t0, double scale) {
     b->C = p.chain_dim;
     b->M = p.mesh_dim;
     b->ninv = 1.0 / p.chain_dim;
+    b->cell_w = (uint32_t)((uint64_t(1) << 32) / (uint64_t)p.chain_dim);
     b->min_rung = min_rung;
     b->first_call = first_call ? 1 : 0;
     b->do_phi = p.do_phi;
@@ -1016,15 +1074,14 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
     a.gz = ctx->gz;
     a.pot = ctx->pot;
     a.cell_begin = ctx->cell_begin;
-    a.tiles = ctx->tiles;
-    a.ntiles = ctx->ntiles;
     float4* gmesh = nullptr;
     a.counters = ctx->counters;
     a.queue = nullptr;
     a.boxes = nullptr;
     a.flags = flags;
     const int64_t ncell = (int64_t)ctx->C * ctx->C * ctx->C;
-    int64_t tiles_max = ctx->n / ctx->tile + ncell + 1;
+    const int64_t tiles_all = ctx->n / ctx->tile + ncell + 1;
+    int64_t tiles_max = tiles_all;
     // the mesh force and potential of the active sinks, made before the
     // pair kernel (LDS cube per chain cell when it fits 32 KiB)
     ctx->mesh_force_w = tpm_mesh_force_width(ctx->C, ctx->M);
@@ -1041,24 +1098,9 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
     }
     int3 blo = make_int3(0, 0, 0), bhi = make_int3(INT_MAX, INT_MAX, INT_MAX);
     if (box) {
-        // the box's tiles into box_tiles (ntiles_box of them, counted by the caller)
         blo = make_int3(box->lo[0], box->lo[1], box->lo[2]);
         bhi = make_int3(box->hi[0], box->hi[1], box->hi[2]);
-        // room for every tile of the context, so the append cannot overrun
-        if (tiles_max > ctx->box_tiles_cap) {
-            if (ctx->box_tiles) TPM_HIP(ctx, hipFree(ctx->box_tiles));
-            ctx->box_tiles = nullptr;
-            TPM_HIP(ctx, hipMalloc(&ctx->box_tiles, sizeof(int4) * tiles_max));
-            ctx->box_tiles_cap = tiles_max;
-        }
         if (ntiles_box > tiles_max) return tpm_fail(ctx, TPM_ERR_INVALID, "tpm_kick_box: tile count");
-        if (!ctx->box_count) TPM_HIP(ctx, hipMalloc(&ctx->box_count, sizeof(int32_t)));
-        set_i32_kernel<<<1, 1, 0, s>>>(ctx->box_count, 0);
-        box_tiles_kernel<<<grid_for(tiles_max, 256), 256, 0, s>>>(ctx->tiles, ctx->ntiles, ctx->C, blo, bhi,
-                                                                  ctx->box_tiles, ctx->box_count);
-        TPM_HIP(ctx, hipGetLastError());
-        a.tiles = ctx->box_tiles;
-        a.ntiles = ctx->box_count;
         tiles_max = ntiles_box;
     }
     tpm_box_fill(&a.box0, ctx->p, min_rung, first_call, t0, scale);
@@ -1111,20 +1153,64 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
 #undef TPM_MF
         TPM_HIP(ctx, hipGetLastError());
     }
-    if (ctx->n > 0 && blocks > 0) {
+    if (ctx->n > 0 && (flags & TPM_SKIP_PP)) {
+        kick_only_kernel<false><<<cell_grid(ncell), 256, 0, s>>>(a, (int)ncell, 1, blo, bhi);
+        TPM_HIP(ctx, hipGetLastError());
+    } else if (ctx->n > 0 && blocks > 0) {
+        // the tiles of the active sinks (kick_pme: of every sink, so that its
+        // sums do not depend on which are active) and, once per chain mesh,
+        // the float positions
+        if (tiles_all > ctx->tiles_cap) {
+            if (ctx->tiles) TPM_HIP(ctx, hipFree(ctx->tiles));
+            ctx->tiles = nullptr;
+            ctx->tiles_cap = 0;
+            TPM_HIP(ctx, hipMalloc(&ctx->tiles, sizeof(int4) * tiles_all));
+            ctx->tiles_cap = tiles_all;
+        }
+        tpm_tile_args t{};
+        t.x = ctx->x;
+        t.y = ctx->y;
+        t.z = ctx->z;
+        t.rung = ctx->rung;
+        t.cell_begin = ctx->cell_begin;
+        t.ncell = (int32_t)ncell;
+        t.C = ctx->C;
+        t.min_rung = min_rung;
+        t.cell_w = a.box0.cell_w;
+        t.lo = blo;
+        t.hi = bhi;
+        t.ts = ctx->tile;
+        t.all = pme ? 1 : 0;
+        t.cnt = ctx->tile_cnt;
+        t.off = ctx->tile_off;
+        t.part = ctx->tile_part;
+        t.tiles = ctx->tiles;
+        t.order = ctx->idx;
+        float *fx = reinterpret_cast<float*>(ctx->x2), *fy = reinterpret_cast<float*>(ctx->y2),
+              *fz = reinterpret_cast<float*>(ctx->z2);
+        if (ctx->fpos_epoch != ctx->chain_epoch) {
+            TPM_TRY(tpm_float_positions(ctx->err, s, t, fx, fy, fz));
+            ctx->fpos_epoch = ctx->chain_epoch;
+        }
+        TPM_TRY(tpm_tiles_make(ctx->err, s, t));
+        a.fx = fx;
+        a.fy = fy;
+        a.fz = fz;
+        a.tiles = ctx->tiles;
+        a.ntiles = ctx->tile_off + ncell;
+        a.order = ctx->idx;
         pp_launch<false>(ctx->tile, false, (unsigned)blocks, s, a, pme, wpg, ctx->pp_lists != 0);
         TPM_HIP(ctx, hipGetLastError());
     }
     TPM_HIP(ctx, hipEventRecord(e1, s));
     if (stats) {
         candidate_pairs_kernel<<<grid_for(ncell, 256), 256, 0, s>>>(ncell, 0, nullptr, ctx->C, ctx->cell_begin,
-                                                                    ctx->counters + 2, blo, bhi);
+                                                                    ctx->counters + 2, ctx->tile,
+                                                                    ctx->counters + TPM_COUNTER_TILES, blo, bhi);
         TPM_HIP(ctx, hipGetLastError());
         std::vector<unsigned long long> hw(TPM_COUNTER_WORDS);
-        int32_t nt = 0;
         TPM_HIP(ctx, hipMemcpyAsync(hw.data(), ctx->counters, sizeof(unsigned long long) * TPM_COUNTER_WORDS,
                                     hipMemcpyDeviceToHost, s));
-        TPM_HIP(ctx, hipMemcpyAsync(&nt, a.ntiles, sizeof(nt), hipMemcpyDeviceToHost, s));
         TPM_HIP(ctx, hipStreamSynchronize(s));
         float ms = 0.f;
         TPM_HIP(ctx, hipEventElapsedTime(&ms, e0, e1));
@@ -1134,7 +1220,7 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
         stats->max_rung = (int)hc[1];
         stats->candidate_pairs = (double)hc[2];
         stats->ms_pp = ms;
-        stats->n_tiles = nt;
+        stats->n_tiles = (int64_t)hw[TPM_COUNTER_TILES];
     }
     return TPM_OK;
 }
@@ -1147,7 +1233,8 @@ tpm_status tpm_candidate_pairs(tpm_ctx* ctx, unsigned long long* dst, const tpm_
         hi = make_int3(box->hi[0], box->hi[1], box->hi[2]);
     }
     candidate_pairs_kernel<<<grid_for(ncell, 256), 256, 0, ctx->stream>>>(ncell, 0, nullptr, ctx->C, ctx->cell_begin,
-                                                                          dst, lo, hi);
+                                                                          dst, ctx->tile,
+                                                                          ctx->counters + TPM_COUNTER_TILES, lo, hi);
     TPM_HIP(ctx, hipGetLastError());
     return TPM_OK;
 }
@@ -1168,8 +1255,6 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
     a.gz = bt->gz;
     a.pot = bt->pot;
     a.cell_begin = bt->cell_begin;
-    a.tiles = bt->tiles;
-    a.ntiles = bt->tile_off + L.ncell;
     a.mesh = nullptr;
     a.counters = bt->counters;
     a.queue = reinterpret_cast<int*>(bt->counters + 8);
@@ -1199,6 +1284,39 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
         TPM_HIP(bt, hipGetLastError());
         a.mesh = bt->mesh_force;
     }
+    if (flags & TPM_SKIP_PP) {
+        kick_only_kernel<true><<<cell_grid(L.ncell), 256, 0, bt->stream>>>(a, L.ncell, L.nbox, make_int3(0, 0, 0),
+                                                                            make_int3(0, 0, 0));
+        TPM_HIP(bt, hipGetLastError());
+        return TPM_OK;
+    }
+    // the tiles of every box's active sinks; float positions in the buffer
+    // set that the gather has left, the order in the sort's slot buffer
+    tpm_tile_args t{};
+    t.x = bt->x;
+    t.y = bt->y;
+    t.z = bt->z;
+    t.rung = bt->rung;
+    t.cell_begin = bt->cell_begin;
+    t.ncell = L.ncell;
+    t.nbox = L.nbox;
+    t.boxes = bt->d_boxes;
+    t.ts = bt->tune.tile_sinks;
+    t.cnt = bt->tile_cnt;
+    t.off = bt->tile_off;
+    t.part = bt->scan_part;
+    t.tiles = bt->tiles;
+    t.order = bt->slot;
+    float *fx = reinterpret_cast<float*>(bt->x2), *fy = reinterpret_cast<float*>(bt->y2),
+          *fz = reinterpret_cast<float*>(bt->z2);
+    TPM_TRY(tpm_float_positions(bt->err, bt->stream, t, fx, fy, fz));
+    TPM_TRY(tpm_tiles_make(bt->err, bt->stream, t));
+    a.fx = fx;
+    a.fy = fy;
+    a.fz = fz;
+    a.tiles = bt->tiles;
+    a.ntiles = bt->tile_off + L.ncell;
+    a.order = bt->slot;
     const bool persistent = bt->tune.sched == 1;
     int64_t grid = persistent ? bt->persist_grid : (L.tiles_max + 7) / 8 * 8;
     if (grid < 8) grid = 8;

@@ -22,6 +22,8 @@
 //    c' - d alone (with zeros when that cell is empty), so no two waves
 //    touch the same word, no sum is formed by atomics and nothing is read
 //    back;
+//  * each cell's particles come in the order of compact 32-particle tiles
+//    (tpm_tiles.hip), which is undone in the epilogue;
 //  * the same wave interpolates the mesh force of its particles (the 6^3
 //    stencil split over 4 lanes per particle), so that its memory latency
 //    hides behind the pair work of other waves;
@@ -36,6 +38,7 @@
 #include <vector>
 
 #include "tpm_pp_device.hpp"
+#include "tpm_tiles.hpp"
 
 #pragma clang fp contract(off)
 
@@ -461,6 +464,7 @@ struct SymEpiArgs {
     const float4* __restrict__ gsrc;
     const float4* __restrict__ gmesh;  // nullptr: no mesh term
     int64_t n;
+    const uint32_t* __restrict__ order;  // particle of each sum
     tpm_kick_out o;
     unsigned flags;
     tpm_box_dev box0;
@@ -490,7 +494,8 @@ __global__ __launch_bounds__(256) void pp_sym_epilogue_kernel(SymEpiArgs a) {
     tpm_kick_out o = a.o;
     if (o.counters) o.counters += TPM_COUNTER_STRIDE * (blockIdx.x % TPM_COUNTER_SLOTS);
     int nr = -1;
-    if (valid) nr = kick_epilogue(B, a.flags, o, (int)i, o.rung[i], pm.x, pm.y, pm.z, pm.w, gx, gy, gz, ph);
+    const int p = (int)a.order[ii];
+    if (valid) nr = kick_epilogue(B, a.flags, o, p, o.rung[p], pm.x, pm.y, pm.z, pm.w, gx, gy, gz, ph);
     max_rung_update(o, nr);
 }
 
@@ -524,10 +529,33 @@ tpm_status tpm_pp_kick_sym(tpm_ctx* ctx, double scale, double t0, int first_call
     tpm_box_fill(&box, ctx->p, 0, first_call, t0, scale);
     box.cell0 = 0;
     box.mesh0 = 0;
+    // each cell's particles in the order of 32-particle tiles of compact
+    // boxes (tpm_tiles.hip), in the buffer set the chain mesh left: fewer
+    // sinks in reach of a source tile than in runs of the Morton order
+    tpm_tile_args t{};
+    t.x = ctx->x;
+    t.y = ctx->y;
+    t.z = ctx->z;
+    t.rung = ctx->rung;
+    t.cell_begin = ctx->cell_begin;
+    t.ncell = ctx->C * ctx->C * ctx->C;
+    t.C = ctx->C;
+    t.cell_w = box.cell_w;
+    t.hi = make_int3(ctx->C, ctx->C, ctx->C);
+    t.ts = 32;
+    t.all = 1;
+    t.full = 1;
+    t.cnt = ctx->tile_cnt;
+    t.off = ctx->tile_off;
+    t.part = ctx->tile_part;
+    t.order = ctx->idx;
+    TPM_TRY(tpm_tiles_make(ctx->err, s, t));
+    TPM_TRY(tpm_order_positions(ctx->err, s, n, t, ctx->x2, ctx->y2, ctx->z2));
+    ctx->fpos_epoch = -1;
     SymArgs a{};
-    a.x = ctx->x;
-    a.y = ctx->y;
-    a.z = ctx->z;
+    a.x = ctx->x2;
+    a.y = ctx->y2;
+    a.z = ctx->z2;
     a.cell_begin = ctx->cell_begin;
     a.phi = use_pm ? ctx->phi : nullptr;
     a.gsink = reinterpret_cast<float4*>(ctx->gsink);
@@ -542,6 +570,7 @@ tpm_status tpm_pp_kick_sym(tpm_ctx* ctx, double scale, double t0, int first_call
     b.gsrc = a.gsrc;
     b.gmesh = use_pm ? a.gmesh : nullptr;
     b.n = n;
+    b.order = ctx->idx;
     b.o = tpm_kick_out{ctx->gx, ctx->gy, ctx->gz, ctx->pot, ctx->vx, ctx->vy, ctx->vz, ctx->rung, ctx->counters};
     b.flags = flags & (TPM_SKIP_PP | TPM_SKIP_PM | TPM_SKIP_KICK);
     b.box0 = box;
@@ -567,8 +596,6 @@ tpm_status tpm_pp_kick_sym(tpm_ctx* ctx, double scale, double t0, int first_call
         std::vector<unsigned long long> hw(TPM_COUNTER_WORDS);
         TPM_HIP(ctx, hipMemcpyAsync(hw.data(), ctx->counters, sizeof(unsigned long long) * TPM_COUNTER_WORDS,
                                     hipMemcpyDeviceToHost, s));
-        int32_t nt = 0;
-        TPM_HIP(ctx, hipMemcpyAsync(&nt, ctx->ntiles, sizeof(nt), hipMemcpyDeviceToHost, s));
         TPM_HIP(ctx, hipStreamSynchronize(s));
         float ms = 0.f;
         TPM_HIP(ctx, hipEventElapsedTime(&ms, e0, e1));
@@ -578,7 +605,7 @@ tpm_status tpm_pp_kick_sym(tpm_ctx* ctx, double scale, double t0, int first_call
         stats->max_rung = (int)hc[1];
         stats->candidate_pairs = (double)hc[2];
         stats->ms_pp = ms;
-        stats->n_tiles = nt;
+        stats->n_tiles = (int64_t)hw[TPM_COUNTER_TILES];
     }
     return TPM_OK;
 }

@@ -1,0 +1,398 @@
+// tpm_tiles.hip -- the direct kernel's work items and float positions.
+//
+// The reference takes its sinks in buckets of a per-cell tree (<= 128,
+// tree.cpp:216-245) and compacts the active ones inside the kernel
+// (kick_treepm.cu:476-503).  Here every kick makes tiles of <= ts active
+// sinks of one chain cell, ts the tuning's tile size:
+//   count:  active particles per cell -> tiles per cell;
+//   scan:   tile offsets and their number (on the device, no wait);
+//   build:  per cell, the active particles' order and the tiles.
+// The order splits a cell's active particles in halves at the median of the
+// longest axis until <= ts remain, so a tile's box is near a cube: at 512^3
+// 16-sink tiles stage 1580 sources instead of 1930 with runs of the Morton
+// order (a CPU model of the boxes; kd order and tiles cost 2.0 ms there).
+// Tiles of active sinks only: with an eighth of 256^3 particles active the
+// kernel has an eighth of the tiles.
+#include "tpm_tiles.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace {
+
+__device__ __forceinline__ unsigned count_below(unsigned long long m) {
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+// Tile order: cells are visited in z-major blocks of TILE_BLOCK^3 cells
+// (blocks z-major, cells z-major inside a block), so the tiles the PP kernel
+// runs close together in time share their 27-cell neighbourhoods: a block's
+// sources (10^3 cells at 512^3, ~2 MB) and its stretch of the potential mesh
+// fit one XCD's L2.  rank(c) is this order's position of cell c, a bijection
+// onto [0, C^3) (edge blocks are smaller).  Each tile is computed
+// independently, so the order changes no result.
+#define TILE_BLOCK 8
+// 32-bit arithmetic throughout (C^3 < 2^27): a wave does this for one cell.
+__device__ __forceinline__ int32_t tile_rank(uint32_t c, uint32_t C) {
+    const uint32_t q = c / C;
+    const int x = (int)(c - q * C), z = (int)(q / C), y = (int)(q - (uint32_t)z * C), Ci = (int)C;
+    const int bx = x / TILE_BLOCK, by = y / TILE_BLOCK, bz = z / TILE_BLOCK;
+    const int sy = min(TILE_BLOCK, Ci - by * TILE_BLOCK), sz = min(TILE_BLOCK, Ci - bz * TILE_BLOCK);
+    const int sx = min(TILE_BLOCK, Ci - bx * TILE_BLOCK);
+    const int before = bz * TILE_BLOCK * Ci * Ci + sz * by * TILE_BLOCK * Ci + sz * sy * bx * TILE_BLOCK;
+    const int local = ((z - bz * TILE_BLOCK) * sy + (y - by * TILE_BLOCK)) * sx + (x - bx * TILE_BLOCK);
+    return before + local;
+}
+
+// What a cell's wave needs of its box.
+struct CellBox {
+    int box, cell0, C, min_rung;
+    uint32_t w;
+};
+__device__ __forceinline__ CellBox cell_box(const tpm_tile_args& a, int c) {
+    if (!a.boxes) return CellBox{0, 0, a.C, a.min_rung, a.cell_w};
+    const int b = tpm_upper_index(a.nbox, c, [&](int k) { return (int64_t)a.boxes[k].cell0; });
+    return CellBox{b, a.boxes[b].cell0, a.boxes[b].C, a.boxes[b].min_rung, a.boxes[b].cell_w};
+}
+
+// Float offsets of a cell's particles from the cell's centre, in raw units:
+// rounded to 2^-25 of half a cell, and shared by the 27 x tiles that stage
+// them (three subtractions and three conversions less per staged source).
+__global__ __launch_bounds__(256) void float_positions_kernel(tpm_tile_args a, float* __restrict__ fx,
+                                                              float* __restrict__ fy, float* __restrict__ fz) {
+    const int lane = threadIdx.x & 63;
+    const int wave = (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
+    const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
+    for (int c = wave; c < a.ncell; c += nwave) {
+        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
+        if (b == e) continue;
+        const CellBox B = cell_box(a, c);
+        const uint32_t l = (uint32_t)(c - B.cell0), C = (uint32_t)B.C;
+        const uint32_t qx = (l % C) * B.w + B.w / 2, qy = ((l / C) % C) * B.w + B.w / 2,
+                       qz = (l / (C * C)) * B.w + B.w / 2;
+        for (int i = b + lane; i < e; i += 64) {
+            fx[i] = (float)(int)(a.x[i] - qx);
+            fy[i] = (float)(int)(a.y[i] - qy);
+            fz[i] = (float)(int)(a.z[i] - qz);
+        }
+    }
+}
+
+__global__ void order_positions_kernel(int64_t n, const uint32_t* __restrict__ order, const uint32_t* __restrict__ x,
+                                       const uint32_t* __restrict__ y, const uint32_t* __restrict__ z,
+                                       uint32_t* __restrict__ ox, uint32_t* __restrict__ oy,
+                                       uint32_t* __restrict__ oz) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t j = order[i];
+        ox[i] = x[j];
+        oy[i] = y[j];
+        oz[i] = z[j];
+    }
+}
+
+// Tiles of each cell: ceil(active / ts), zero outside [lo, hi).  16 lanes per
+// cell.
+__global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a) {
+    const int sub = threadIdx.x & 15;
+    const int64_t g = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 4;
+    const int64_t ng = ((int64_t)gridDim.x * blockDim.x) >> 4;
+    for (int64_t c = g; c < a.ncell; c += ng) {
+        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
+        int n = 0;
+        int64_t r = c;
+        bool in = true;
+        if (!a.boxes) {
+            r = tile_rank((uint32_t)c, (uint32_t)a.C);
+            const uint32_t C = (uint32_t)a.C, u = (uint32_t)c;
+            const int x = (int)(u % C), y = (int)((u / C) % C), z = (int)(u / (C * C));
+            in = x >= a.lo.x && x < a.hi.x && y >= a.lo.y && y < a.hi.y && z >= a.lo.z && z < a.hi.z;
+        }
+        if (in) {
+            if (a.all) {
+                n = e - b;
+            } else if (b < e) {
+                const int min_rung = cell_box(a, (int)c).min_rung;
+                for (int i = b + sub; i < e; i += 16) n += a.rung[i] >= min_rung ? 1 : 0;
+#pragma unroll
+                for (int o = 8; o >= 1; o >>= 1) n += __shfl_xor(n, o);
+            }
+        }
+        if (sub == 0) a.cnt[r] = (n + a.ts - 1) / a.ts;
+    }
+}
+
+// The order and the tiles of one cell, by one wave, KD_CHUNK active particles
+// at a time (in chain-mesh order, whose Morton codes keep them together).  A
+// segment of len particles that makes m tiles is split m / 2 : m - m / 2, at
+// the position whose lower side has len (m / 2) / m particles (full tiles: ts
+// (m / 2)), found by
+// bisection of the coordinate with ballot counts; ties go by position, so the
+// split is exact and depends on nothing but the cell's particles.
+constexpr int KD_CHUNK = 256;
+constexpr int KD_STACK = 8;  // pending segments: one per level of at most log2(256 / 8), and the current one
+
+struct KdWave {
+    uint32_t p[3][KD_CHUNK];  // offsets from the cell's centre, + 2^31
+    uint32_t id[KD_CHUNK];    // particles of the chunk
+    uint32_t ord[KD_CHUNK];   // their order
+    int stack[KD_STACK][9];   // first, len, tiles, box
+};
+
+// The LDS words of a KdWave are written and read by the lanes of one wave,
+// whose LDS operations complete in order: the compiler keeps the order, and
+// nothing waits for the tiles' global stores, as a fence would.
+__device__ __forceinline__ void kd_sync() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Minimum and maximum of a wave: DPP within the rows of 16, the rows by
+// scalar operations.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t v, Op op) {
+    const auto dpp = [](uint32_t x, auto ctrl) {
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, decltype(ctrl)::value, 0xf, 0xf, false);
+    };
+    v = op(v, dpp(v, std::integral_constant<int, 0xB1>{}));
+    v = op(v, dpp(v, std::integral_constant<int, 0x4E>{}));
+    v = op(v, dpp(v, std::integral_constant<int, 0x141>{}));
+    v = op(v, dpp(v, std::integral_constant<int, 0x140>{}));
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16),
+                   c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    return op(op(a, b), op(c, d));
+}
+__device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
+    return wave_reduce(v, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+}
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
+    return wave_reduce(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+
+// Splits a.ord[s .. s + len) so that its first `left` entries are the `left`
+// smallest along an axis; returns the split coordinate.  PER: entries per
+// lane, at least len / 64 (most segments have at most 64 entries).
+template <int PER>
+__device__ __forceinline__ uint32_t kd_split(KdWave& w, int lane, int s, int len, int left, int axis, uint32_t lo,
+                                             uint32_t hi) {
+    uint32_t e[PER], key[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        e[i] = 0u;
+        key[i] = ~0u;
+        const int k = lane + 64 * i;
+        if (k < len) {
+            e[i] = w.ord[s + k];
+            key[i] = w.p[axis][e[i]];
+        }
+    }
+    const auto below = [&](uint32_t t) {
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < PER; i++)
+            n += __popcll(__ballot(key[i] < t));
+        return n;
+    };
+    // below(a) <= left < below(b) or the exact split; keys lie in [lo, hi],
+    // hi < 2^32 - 1 (offsets span less than half the box), so padding keys
+    // are above every threshold
+    uint32_t a = lo, b = hi + 1u, t = a;
+    int nt = 0;
+    while (b - a > 1u) {
+        t = a + (b - a) / 2u;
+        nt = below(t);
+        if (nt == left) break;
+        if (nt < left)
+            a = t;
+        else
+            b = t;
+    }
+    if (nt != left) {
+        t = a;
+        nt = below(t);
+    }
+    // keys equal to t fill the lower side up in order
+    int need = left - nt, nl = 0, nr = 0;
+    uint32_t dst[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const bool have = lane + 64 * i < len;
+        const unsigned long long me = __ballot(have && key[i] == t);
+        const bool lower = have && (key[i] < t || (key[i] == t && (int)count_below(me) < need));
+        need = max(need - __popcll(me), 0);
+        const unsigned long long ml = __ballot(lower), mr = __ballot(have && !lower);
+        dst[i] = (uint32_t)(lower ? nl + (int)count_below(ml) : left + nr + (int)count_below(mr));
+        nl += __popcll(ml);
+        nr += __popcll(mr);
+    }
+    kd_sync();
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+        if (lane + 64 * i < len) w.ord[s + (int)dst[i]] = e[i];
+    return t;
+}
+
+__global__ __launch_bounds__(256) void tile_build_kernel(tpm_tile_args a) {
+    __shared__ KdWave s_wave[4];
+    const int lane = threadIdx.x & 63;
+    KdWave& w = s_wave[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)];
+    const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
+    const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
+    const int ts = a.ts;
+    for (int c = wave; c < a.ncell; c += nwave) {
+        const int r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
+        if (a.cnt[r] == 0) continue;
+        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
+        const CellBox B = cell_box(a, c);
+        const uint32_t l = (uint32_t)(c - B.cell0), C = (uint32_t)B.C;
+        const uint32_t q[3] = {(l % C) * B.w + B.w / 2 - 0x80000000u, ((l / C) % C) * B.w + B.w / 2 - 0x80000000u,
+                               (l / (C * C)) * B.w + B.w / 2 - 0x80000000u};
+        int tile = a.off[r];
+        int out = b;  // next slot of the cell's order
+        int i0 = b;   // next particle of the cell
+        while (i0 < e) {
+            // the next chunk of active particles
+            int n = 0;
+            while (i0 < e && n < KD_CHUNK) {
+                const int i = i0 + lane;
+                bool act = i < e && (a.all || a.rung[i] >= B.min_rung);
+                unsigned long long m = __ballot(act);
+                int took = 64;
+                if (n + __popcll(m) > KD_CHUNK) {
+                    // the chunk is full inside this group: take its first ones
+                    act = act && n + (int)count_below(m) < KD_CHUNK;
+                    m = __ballot(act);
+                    took = 64 - __builtin_clzll(m);  // up to the last one taken
+                }
+                if (act) {
+                    const int k = n + (int)count_below(m);
+                    w.id[k] = (uint32_t)i;
+                    w.ord[k] = (uint32_t)k;
+                    w.p[0][k] = a.x[i] - q[0];
+                    w.p[1][k] = a.y[i] - q[1];
+                    w.p[2][k] = a.z[i] - q[2];
+                }
+                n += __popcll(m);
+                i0 += took;
+            }
+            if (n == 0) break;
+            kd_sync();
+            const int m0 = (n + ts - 1) / ts;
+            int sp = 1;
+            uint32_t lo[3], hi[3];
+            if (m0 > 1) {
+                // the chunk's box; from there on halves of it
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    uint32_t mn = ~0u, mx = 0u;
+                    for (int k = lane; k < n; k += 64) {
+                        const uint32_t v = w.p[d][k];
+                        mn = min(mn, v);
+                        mx = max(mx, v);
+                    }
+                    lo[d] = wave_umin(mn);
+                    hi[d] = wave_umax(mx);
+                }
+            } else {
+                lo[0] = lo[1] = lo[2] = hi[0] = hi[1] = hi[2] = 0u;
+            }
+            if (lane == 0) {
+                w.stack[0][0] = 0;
+                w.stack[0][1] = n;
+                w.stack[0][2] = m0;
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    w.stack[0][3 + d] = (int)lo[d];
+                    w.stack[0][6 + d] = (int)hi[d];
+                }
+            }
+            kd_sync();
+            while (sp > 0) {
+                sp--;
+                const int s = __builtin_amdgcn_readfirstlane(w.stack[sp][0]);
+                const int len = __builtin_amdgcn_readfirstlane(w.stack[sp][1]);
+                const int m = __builtin_amdgcn_readfirstlane(w.stack[sp][2]);
+                if (m == 1) {
+                    if (lane == 0 && a.tiles) a.tiles[tile] = make_int4(c, out + s, out + s + len, B.box);
+                    tile++;
+                    continue;
+                }
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    lo[d] = (uint32_t)__builtin_amdgcn_readfirstlane(w.stack[sp][3 + d]);
+                    hi[d] = (uint32_t)__builtin_amdgcn_readfirstlane(w.stack[sp][6 + d]);
+                }
+                int axis = 0;
+                uint32_t span = hi[0] - lo[0], l0 = lo[0], h0 = hi[0];
+                if (hi[1] - lo[1] > span) {
+                    axis = 1;
+                    span = hi[1] - lo[1];
+                    l0 = lo[1];
+                    h0 = hi[1];
+                }
+                if (hi[2] - lo[2] > span) {
+                    axis = 2;
+                    l0 = lo[2];
+                    h0 = hi[2];
+                }
+                const int m1 = m / 2, left = a.full ? ts * m1 : len * m1 / m;
+                const uint32_t t = len <= 64    ? kd_split<1>(w, lane, s, len, left, axis, l0, h0)
+                                   : len <= 128 ? kd_split<2>(w, lane, s, len, left, axis, l0, h0)
+                                                : kd_split<KD_CHUNK / 64>(w, lane, s, len, left, axis, l0, h0);
+                kd_sync();
+                if (lane == 0) {
+                    // the upper side waits below the lower one
+                    int* up = w.stack[sp];
+                    int* dn = w.stack[sp + 1];
+                    up[0] = s + left;
+                    up[1] = len - left;
+                    up[2] = m - m1;
+                    dn[0] = s;
+                    dn[1] = left;
+                    dn[2] = m1;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        dn[3 + d] = (int)lo[d];
+                        up[6 + d] = (int)hi[d];
+                        up[3 + d] = (int)(d == axis ? t : lo[d]);
+                        dn[6 + d] = (int)(d == axis ? t : hi[d]);
+                    }
+                }
+                sp += 2;
+                kd_sync();
+            }
+            for (int k = lane; k < n; k += 64) a.order[out + k] = w.id[w.ord[k]];
+            out += n;
+            kd_sync();
+        }
+    }
+}
+
+}  // namespace
+
+// One wave per cell up to a grid that fills the chip many times over.
+static unsigned wave_grid(int64_t ncell) { return (unsigned)std::min<int64_t>((ncell + 3) / 4, 65536); }
+
+tpm_status tpm_float_positions(std::string& err, hipStream_t s, const tpm_tile_args& a, float* fx, float* fy,
+                               float* fz) {
+    if (a.ncell == 0) return TPM_OK;
+    float_positions_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a, fx, fy, fz);
+    TPM_HIPE(err, hipGetLastError());
+    return TPM_OK;
+}
+
+tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const tpm_tile_args& a, uint32_t* x,
+                               uint32_t* y, uint32_t* z) {
+    order_positions_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, a.order, a.x, a.y, a.z, x, y, z);
+    TPM_HIPE(err, hipGetLastError());
+    return TPM_OK;
+}
+
+tpm_status tpm_tiles_make(std::string& err, hipStream_t s, const tpm_tile_args& a) {
+    if (a.ncell == 0) return TPM_OK;
+    tile_count_kernel<<<(unsigned)std::min<int64_t>(((int64_t)a.ncell + 15) / 16, 65536), 256, 0, s>>>(a);
+    TPM_HIPE(err, hipGetLastError());
+    TPM_TRY(tpm_scan_i32(err, s, a.cnt, a.ncell, a.part, a.off));
+    tile_build_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a);
+    TPM_HIPE(err, hipGetLastError());
+    return TPM_OK;
+}
