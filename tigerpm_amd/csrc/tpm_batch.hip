@@ -96,6 +96,8 @@ tpm_status build_layout(tpm_batch* bt, tpm_batch_layout* L) {
     int64_t cell = 0, dep = 0, q = 0, tiles = 0;
     int lds = 0, nk = 0, mfw = 0;
     const int nb = (int)bt->boxes.size();
+    int64_t n_all = 0;
+    for (const tpm_batch_box& b : bt->boxes) n_all += b.live ? b.n : 0;
     for (int i = 0; i < nb; i++) {
         const tpm_batch_box& b = bt->boxes[i];
         tpm_box_dev& d = bt->h_boxes[i];
@@ -114,7 +116,8 @@ tpm_status build_layout(tpm_batch* bt, tpm_batch_layout* L) {
             d.B = b.B;
             d.nb = b.nb;
             cell += cells_of(b.C);
-            dep += (int64_t)b.nb * b.nb * b.nb;
+            d.parts = tpm_deposit_parts(b.n, b.nb, n_all);
+            dep += (int64_t)b.nb * b.nb * b.nb * d.parts;
             q += b.n;
             tiles += b.n / ts + cells_of(b.C) + 1;
             lds = std::max(lds, b.wmax * b.wmax * b.wmax * 8);

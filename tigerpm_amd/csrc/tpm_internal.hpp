@@ -101,6 +101,7 @@ struct tpm_box_dev {
     double ninv;         // 1.0 / C (split planes fixed32(k * ninv))
     int32_t dep0;        // first deposit work item of the box
     int32_t B, nb;       // deposit block edge (chain cells) and blocks per axis
+    int32_t parts;       // deposit work items per block
     int32_t min_rung, first_call, do_phi, cull;
     // pair constants in 2^-32 box units
     float rcut2s, cull2s, inv2rs_s, tsp, h2s, h2inv_s, hinv_s, h3inv_s;
@@ -629,3 +630,4 @@ tpm_status tpm_green_table(std::string& err, hipStream_t s, int M, double rs, in
 #define TPM_DEPOSIT_LDS_AUTO (80 * 1024)  // automatic block edge: 2 workgroups per CU
 tpm_status tpm_deposit_lds_setup(std::string& err);  // allow the deposit kernels their LDS
 void tpm_deposit_blocking(int C, int M, int interlace, int want, int* B, int* wmax);
+int tpm_deposit_parts(int64_t n, int nb, int64_t n_all);

@@ -104,6 +104,7 @@ struct BlockedDepositArgs {
     unsigned long long* __restrict__ grid;
     uint64_t shift;
     int C, M, B, nb;                      // nb = ceil(C / B) blocks per axis
+    int parts;                            // workgroups per block
 };
 
 // Mesh nodes [lo, lo + w) touched by particles of chain cells [c0, c1].
@@ -115,13 +116,15 @@ __host__ __device__ __forceinline__ void block_nodes(uint64_t xlo, uint64_t xhi_
     *w = h - l + 1;
 }
 
-// The deposit of block bid (of nb^3) of one box; plane(k) gives split plane
-// k < C of the box's chain mesh, cell0 its first global cell.
+// Part `part` of `parts` of the deposit of block bid (of nb^3) of one box;
+// plane(k) gives split plane k < C of the box's chain mesh, cell0 its first
+// global cell.  The parts of a block take every parts-th of its particles,
+// each with its own copy of the footprint in LDS.
 template <int ORDER, class Plane>
 __device__ __forceinline__ void deposit_block(const uint32_t* __restrict__ x, const uint32_t* __restrict__ y,
                                               const uint32_t* __restrict__ z, const int32_t* __restrict__ cell_begin,
                                               int cell0, unsigned long long* __restrict__ grid, uint64_t shift, int C,
-                                              int M, int B, int nb, int bid, Plane plane,
+                                              int M, int B, int nb, int bid, int part, int parts, Plane plane,
                                               unsigned long long* __restrict__ sg) {
     constexpr int NP = ORDER;
     const int bx = bid % nb, by = (bid / nb) % nb, bz = bid / (nb * nb);
@@ -157,8 +160,9 @@ __device__ __forceinline__ void deposit_block(const uint32_t* __restrict__ x, co
     }
     __syncthreads();
     const int total = row_pre[nrows];
+    if (part >= total) return;
     int row = 0;
-    for (int k = threadIdx.x; k < total; k += blockDim.x) {
+    for (int k = part + parts * (int)threadIdx.x; k < total; k += parts * (int)blockDim.x) {
         while (k >= row_pre[row + 1]) row++;
         const int i = row_first[row] + (k - row_pre[row]);
         int bxn, byn, bzn;
@@ -190,7 +194,8 @@ template <int ORDER>
 __global__ __launch_bounds__(TPM_DEPOSIT_THREADS) void deposit_blocked_kernel(BlockedDepositArgs a) {
     extern __shared__ unsigned long long sg[];
     const uint32_t* bounds = a.bounds;
-    deposit_block<ORDER>(a.x, a.y, a.z, a.cell_begin, 0, a.grid, a.shift, a.C, a.M, a.B, a.nb, (int)blockIdx.x,
+    deposit_block<ORDER>(a.x, a.y, a.z, a.cell_begin, 0, a.grid, a.shift, a.C, a.M, a.B, a.nb,
+                         (int)blockIdx.x / a.parts, (int)blockIdx.x % a.parts, a.parts,
                          [&](int k) { return bounds[k]; }, sg);
 }
 
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(TPM_DEPOSIT_THREADS) void bdeposit_kernel(const uin
     const tpm_box_dev& bx = boxes[b];
     const double ninv = bx.ninv;
     deposit_block<ORDER>(x, y, z, cell_begin, bx.cell0, grid + bx.mesh0, shift, bx.C, bx.M, bx.B, bx.nb,
-                         item - bx.dep0, [&](int k) { return tpm_split_plane(k, ninv); }, sg);
+                         (item - bx.dep0) / bx.parts, (item - bx.dep0) % bx.parts, bx.parts, [&](int k) { return tpm_split_plane(k, ninv); }, sg);
 }
 
 // Unit masses per node: float(double(sum) * 2^-32).
@@ -601,6 +606,21 @@ void tpm_deposit_blocking(int C, int M, int interlace, int want, int* Bout, int*
     }
 }
 
+// Workgroups per deposit block of a box of n particles in nb^3 blocks, n_all
+// particles being deposited by the launch: enough for about 768 equal shares
+// of n_all, but no share below 512 particles (a share clears and writes back
+// the block's whole footprint, a few thousand nodes).  The sums are integers,
+// so the grid does not depend on it.  Small and coarse boxes have few blocks:
+// with one workgroup per block the reference's ratios took 2.34 ms for 120^3
+// particles (27 blocks) and 2.17 ms for 60^3 (8 blocks); now 0.09 and 0.03 ms.
+// Interleaved shares put neighbouring particles, which add to the same nodes,
+// into different workgroups: contiguous ones take 0.20 and 0.10 ms.
+int tpm_deposit_parts(int64_t n, int nb, int64_t n_all) {
+    const int64_t share = std::max<int64_t>(512, n_all / 768);
+    const int64_t block = n / ((int64_t)nb * nb * nb);
+    return (int)std::min<int64_t>(std::max<int64_t>(block / share, 1), 1024);
+}
+
 // Integer deposit (grid displaced by shift / 2^32 cells) into rho_q and,
 // with to_float, its float image into rho.
 static tpm_status deposit_density(tpm_ctx* ctx, uint64_t shift, bool to_float = true) {
@@ -625,7 +645,8 @@ static tpm_status deposit_density(tpm_ctx* ctx, uint64_t shift, bool to_float = 
         da.M = M;
         da.B = B;
         da.nb = (ctx->C + B - 1) / B;
-        const unsigned nblk = (unsigned)((int64_t)da.nb * da.nb * da.nb);
+        da.parts = tpm_deposit_parts(ctx->n, da.nb, ctx->n);
+        const unsigned nblk = (unsigned)((int64_t)da.nb * da.nb * da.nb * da.parts);
         const size_t lds = sizeof(unsigned long long) * (size_t)wmax * wmax * wmax;
         switch (ctx->p.order) {
             case 2: deposit_blocked_kernel<2><<<nblk, TPM_DEPOSIT_THREADS, lds, s>>>(da); break;
