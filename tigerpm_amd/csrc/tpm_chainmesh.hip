@@ -568,6 +568,25 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_apply_kernel(const int32_t*
     }
 }
 
+// The whole scan in one block (few entries: one launch instead of three).
+constexpr int64_t SCAN_SMALL = 8 * SCAN_CHUNK;
+__global__ __launch_bounds__(SCAN_THREADS) void scan_small_kernel(const int32_t* __restrict__ in, int n,
+                                                                  int32_t* __restrict__ out) {
+    __shared__ int32_t sh[SCAN_THREADS];
+    const int per = (n + SCAN_THREADS - 1) / SCAN_THREADS;
+    const int b0 = (int)threadIdx.x * per, b1 = min(b0 + per, n);
+    int32_t s = 0;
+    for (int k = b0; k < b1; k++) s += in[k];
+    int32_t tot;
+    int32_t run = block_exclusive_scan(s, sh, &tot);
+    for (int k = b0; k < b1; k++) {
+        const int32_t v = in[k];
+        out[k] = run;
+        run += v;
+    }
+    if (threadIdx.x == 0) out[n] = tot;
+}
+
 __global__ void bscatter_kernel(int64_t n, const uint32_t* __restrict__ key, const uint32_t* __restrict__ slot,
                                 const int32_t* __restrict__ cell_begin, uint32_t* __restrict__ tmp) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
@@ -673,6 +692,11 @@ tpm_status tpm_scan_i32(std::string& err, hipStream_t s, const int32_t* in, int6
     if (nchunk < 1 || nchunk > INT32_MAX) {
         err = "scan: bad size";
         return TPM_ERR_INVALID;
+    }
+    if (n <= SCAN_SMALL) {
+        scan_small_kernel<<<1, SCAN_THREADS, 0, s>>>(in, (int)n, out);
+        TPM_HIPE(err, hipGetLastError());
+        return TPM_OK;
     }
     scan_partials_kernel<<<(unsigned)nchunk, SCAN_THREADS, 0, s>>>(in, n, part);
     scan_part_kernel<<<1, SCAN_THREADS, 0, s>>>(part, nchunk, out + n);

@@ -1176,6 +1176,7 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
         t.ncell = (int32_t)ncell;
         t.C = ctx->C;
         t.min_rung = min_rung;
+        t.n = t.n_all = ctx->n;
         t.cell_w = a.box0.cell_w;
         t.lo = blo;
         t.hi = bhi;
@@ -1188,11 +1189,9 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
         t.order = ctx->idx;
         float *fx = reinterpret_cast<float*>(ctx->x2), *fy = reinterpret_cast<float*>(ctx->y2),
               *fz = reinterpret_cast<float*>(ctx->z2);
-        if (ctx->fpos_epoch != ctx->chain_epoch) {
-            TPM_TRY(tpm_float_positions(ctx->err, s, t, fx, fy, fz));
-            ctx->fpos_epoch = ctx->chain_epoch;
-        }
-        TPM_TRY(tpm_tiles_make(ctx->err, s, t));
+        const bool made = ctx->fpos_epoch == ctx->chain_epoch;
+        TPM_TRY(tpm_tiles_make(ctx->err, s, t, made ? nullptr : fx, fy, fz));
+        ctx->fpos_epoch = ctx->chain_epoch;
         a.fx = fx;
         a.fy = fy;
         a.fz = fz;
@@ -1301,6 +1300,7 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
     t.ncell = L.ncell;
     t.nbox = L.nbox;
     t.boxes = bt->d_boxes;
+    t.n_all = L.n_live;
     t.ts = bt->tune.tile_sinks;
     t.cnt = bt->tile_cnt;
     t.off = bt->tile_off;
@@ -1309,8 +1309,7 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
     t.order = bt->slot;
     float *fx = reinterpret_cast<float*>(bt->x2), *fy = reinterpret_cast<float*>(bt->y2),
           *fz = reinterpret_cast<float*>(bt->z2);
-    TPM_TRY(tpm_float_positions(bt->err, bt->stream, t, fx, fy, fz));
-    TPM_TRY(tpm_tiles_make(bt->err, bt->stream, t));
+    TPM_TRY(tpm_tiles_make(bt->err, bt->stream, t, fx, fy, fz));
     a.fx = fx;
     a.fy = fy;
     a.fz = fz;

@@ -47,29 +47,42 @@ __device__ __forceinline__ int32_t tile_rank(uint32_t c, uint32_t C) {
 // What a cell's wave needs of its box.
 struct CellBox {
     int box, cell0, C, min_rung;
+    int64_t n;
     uint32_t w;
 };
 __device__ __forceinline__ CellBox cell_box(const tpm_tile_args& a, int c) {
-    if (!a.boxes) return CellBox{0, 0, a.C, a.min_rung, a.cell_w};
+    if (!a.boxes) return CellBox{0, 0, a.C, a.min_rung, a.n, a.cell_w};
     const int b = tpm_upper_index(a.nbox, c, [&](int k) { return (int64_t)a.boxes[k].cell0; });
-    return CellBox{b, a.boxes[b].cell0, a.boxes[b].C, a.boxes[b].min_rung, a.boxes[b].cell_w};
+    return CellBox{b, a.boxes[b].cell0, a.boxes[b].C, a.boxes[b].min_rung, a.boxes[b].n, a.boxes[b].cell_w};
 }
 
-// Float offsets of a cell's particles from the cell's centre, in raw units:
-// rounded to 2^-25 of half a cell, and shared by the 27 x tiles that stage
-// them (three subtractions and three conversions less per staged source).
-__global__ __launch_bounds__(256) void float_positions_kernel(tpm_tile_args a, float* __restrict__ fx,
-                                                              float* __restrict__ fy, float* __restrict__ fz) {
+// One wave per cell: its number of tiles, ceil(active / ts) (zero outside [lo,
+// hi)), and where wanted (fx) the float offsets of its particles from its
+// centre, in raw units: rounded to 2^-25 of half a cell, and shared by the
+// tiles of 27 cells that stage them (three subtractions and three
+// conversions less per staged source).
+__global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a, float* __restrict__ fx,
+                                                         float* __restrict__ fy, float* __restrict__ fz) {
     const int lane = threadIdx.x & 63;
-    const int wave = (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
     for (int c = wave; c < a.ncell; c += nwave) {
         const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
-        if (b == e) continue;
         const CellBox B = cell_box(a, c);
         const uint32_t l = (uint32_t)(c - B.cell0), C = (uint32_t)B.C;
-        const uint32_t qx = (l % C) * B.w + B.w / 2, qy = ((l / C) % C) * B.w + B.w / 2,
-                       qz = (l / (C * C)) * B.w + B.w / 2;
+        const uint32_t x = l % C, y = (l / C) % C, z = l / (C * C);
+        int n = 0;
+        if (a.boxes || ((int)x >= a.lo.x && (int)x < a.hi.x && (int)y >= a.lo.y && (int)y < a.hi.y &&
+                        (int)z >= a.lo.z && (int)z < a.hi.z)) {
+            if (a.all)
+                n = e - b;
+            else
+                for (int i = b; i < e; i += 64)
+                    n += __popcll(__ballot(i + lane < e && a.rung[min(i + lane, e - 1)] >= B.min_rung));
+        }
+        if (lane == 0) a.cnt[a.boxes ? c : tile_rank(l, C)] = (n + a.ts - 1) / a.ts;
+        if (!fx) continue;
+        const uint32_t qx = x * B.w + B.w / 2, qy = y * B.w + B.w / 2, qz = z * B.w + B.w / 2;
         for (int i = b + lane; i < e; i += 64) {
             fx[i] = (float)(int)(a.x[i] - qx);
             fy[i] = (float)(int)(a.y[i] - qy);
@@ -90,45 +103,18 @@ __global__ void order_positions_kernel(int64_t n, const uint32_t* __restrict__ o
     }
 }
 
-// Tiles of each cell: ceil(active / ts), zero outside [lo, hi).  16 lanes per
-// cell.
-__global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a) {
-    const int sub = threadIdx.x & 15;
-    const int64_t g = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 4;
-    const int64_t ng = ((int64_t)gridDim.x * blockDim.x) >> 4;
-    for (int64_t c = g; c < a.ncell; c += ng) {
-        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
-        int n = 0;
-        int64_t r = c;
-        bool in = true;
-        if (!a.boxes) {
-            r = tile_rank((uint32_t)c, (uint32_t)a.C);
-            const uint32_t C = (uint32_t)a.C, u = (uint32_t)c;
-            const int x = (int)(u % C), y = (int)((u / C) % C), z = (int)(u / (C * C));
-            in = x >= a.lo.x && x < a.hi.x && y >= a.lo.y && y < a.hi.y && z >= a.lo.z && z < a.hi.z;
-        }
-        if (in) {
-            if (a.all) {
-                n = e - b;
-            } else if (b < e) {
-                const int min_rung = cell_box(a, (int)c).min_rung;
-                for (int i = b + sub; i < e; i += 16) n += a.rung[i] >= min_rung ? 1 : 0;
-#pragma unroll
-                for (int o = 8; o >= 1; o >>= 1) n += __shfl_xor(n, o);
-            }
-        }
-        if (sub == 0) a.cnt[r] = (n + a.ts - 1) / a.ts;
-    }
-}
-
-// The order and the tiles of one cell, by one wave, KD_CHUNK active particles
-// at a time (in chain-mesh order, whose Morton codes keep them together).  A
+// The order and the tiles of a chunk of a cell's active particles, by one
+// wave: KD_CHUNK of them in chain-mesh order, whose Morton codes keep them
+// together, half as many in boxes below KD_SMALL particles, where the waves
+// are few and the splits of a chunk, one after the other, are the kernel's
+// time.  a.per_cell waves share a cell's chunks.  A
 // segment of len particles that makes m tiles is split m / 2 : m - m / 2, at
 // the position whose lower side has len (m / 2) / m particles (full tiles: ts
 // (m / 2)), found by
 // bisection of the coordinate with ballot counts; ties go by position, so the
 // split is exact and depends on nothing but the cell's particles.
 constexpr int KD_CHUNK = 256;
+constexpr int KD_SMALL = 1 << 19;
 constexpr int KD_STACK = 8;  // pending segments: one per level of at most log2(256 / 8), and the current one
 
 struct KdWave {
@@ -238,41 +224,41 @@ __global__ __launch_bounds__(256) void tile_build_kernel(tpm_tile_args a) {
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
     const int ts = a.ts;
-    for (int c = wave; c < a.ncell; c += nwave) {
+    for (int u = wave; u < a.ncell * a.per_cell; u += nwave) {
+        const int c = u / a.per_cell, k0 = u - c * a.per_cell;
         const int r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
-        if (a.cnt[r] == 0) continue;
+        const int ntile = a.cnt[r];
+        if (ntile == 0) continue;
         const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
         const CellBox B = cell_box(a, c);
+        const int chunk = B.n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK;
         const uint32_t l = (uint32_t)(c - B.cell0), C = (uint32_t)B.C;
         const uint32_t q[3] = {(l % C) * B.w + B.w / 2 - 0x80000000u, ((l / C) % C) * B.w + B.w / 2 - 0x80000000u,
                                (l / (C * C)) * B.w + B.w / 2 - 0x80000000u};
-        int tile = a.off[r];
-        int out = b;  // next slot of the cell's order
-        int i0 = b;   // next particle of the cell
-        while (i0 < e) {
-            // the next chunk of active particles
+        int seen = 0, i0 = b;  // active particles before particle i0 of the cell
+        for (int k = k0; k * (chunk / ts) < ntile; k += a.per_cell) {
+            const int first = k * chunk;  // active particles before the chunk
+            int tile = a.off[r] + k * (chunk / ts);
+            const int out = b + first;  // its place in the order
             int n = 0;
-            while (i0 < e && n < KD_CHUNK) {
+            while (i0 < e && n < chunk) {
                 const int i = i0 + lane;
-                bool act = i < e && (a.all || a.rung[i] >= B.min_rung);
-                unsigned long long m = __ballot(act);
-                int took = 64;
-                if (n + __popcll(m) > KD_CHUNK) {
-                    // the chunk is full inside this group: take its first ones
-                    act = act && n + (int)count_below(m) < KD_CHUNK;
-                    m = __ballot(act);
-                    took = 64 - __builtin_clzll(m);  // up to the last one taken
-                }
+                bool act = i < e && (a.all || a.rung[min(i, e - 1)] >= B.min_rung);
+                const unsigned long long m = __ballot(act);
+                const int rank = seen + (int)count_below(m) - first;
+                act = act && rank >= 0 && rank < chunk;
+                const unsigned long long mt = __ballot(act);
                 if (act) {
-                    const int k = n + (int)count_below(m);
-                    w.id[k] = (uint32_t)i;
-                    w.ord[k] = (uint32_t)k;
-                    w.p[0][k] = a.x[i] - q[0];
-                    w.p[1][k] = a.y[i] - q[1];
-                    w.p[2][k] = a.z[i] - q[2];
+                    w.id[rank] = (uint32_t)i;
+                    w.ord[rank] = (uint32_t)rank;
+                    w.p[0][rank] = a.x[i] - q[0];
+                    w.p[1][rank] = a.y[i] - q[1];
+                    w.p[2][rank] = a.z[i] - q[2];
                 }
-                n += __popcll(m);
-                i0 += took;
+                n += __popcll(mt);
+                if (n == chunk) break;  // the next chunk may begin inside this group
+                seen += __popcll(m);
+                i0 += 64;
             }
             if (n == 0) break;
             kd_sync();
@@ -360,8 +346,7 @@ __global__ __launch_bounds__(256) void tile_build_kernel(tpm_tile_args a) {
                 sp += 2;
                 kd_sync();
             }
-            for (int k = lane; k < n; k += 64) a.order[out + k] = w.id[w.ord[k]];
-            out += n;
+            for (int i = lane; i < n; i += 64) a.order[out + i] = w.id[w.ord[i]];
             kd_sync();
         }
     }
@@ -369,16 +354,8 @@ __global__ __launch_bounds__(256) void tile_build_kernel(tpm_tile_args a) {
 
 }  // namespace
 
-// One wave per cell up to a grid that fills the chip many times over.
-static unsigned wave_grid(int64_t ncell) { return (unsigned)std::min<int64_t>((ncell + 3) / 4, 65536); }
-
-tpm_status tpm_float_positions(std::string& err, hipStream_t s, const tpm_tile_args& a, float* fx, float* fy,
-                               float* fz) {
-    if (a.ncell == 0) return TPM_OK;
-    float_positions_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a, fx, fy, fz);
-    TPM_HIPE(err, hipGetLastError());
-    return TPM_OK;
-}
+// Workgroups of 4 waves, up to a grid that fills the chip many times over.
+static unsigned wave_grid(int64_t waves) { return (unsigned)std::min<int64_t>((waves + 3) / 4, 65536); }
 
 tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const tpm_tile_args& a, uint32_t* x,
                                uint32_t* y, uint32_t* z) {
@@ -387,12 +364,14 @@ tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const
     return TPM_OK;
 }
 
-tpm_status tpm_tiles_make(std::string& err, hipStream_t s, const tpm_tile_args& a) {
+tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a, float* fx, float* fy, float* fz) {
     if (a.ncell == 0) return TPM_OK;
-    tile_count_kernel<<<(unsigned)std::min<int64_t>(((int64_t)a.ncell + 15) / 16, 65536), 256, 0, s>>>(a);
+    tile_count_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a, fx, fy, fz);
     TPM_HIPE(err, hipGetLastError());
     TPM_TRY(tpm_scan_i32(err, s, a.cnt, a.ncell, a.part, a.off));
-    tile_build_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a);
+    // as many waves as an average cell has chunks
+    a.per_cell = (int)std::min<int64_t>(std::max<int64_t>(a.n_all / a.ncell / (KD_CHUNK / 2), 1), 32);
+    tile_build_kernel<<<wave_grid((int64_t)a.ncell * a.per_cell), 256, 0, s>>>(a);
     TPM_HIPE(err, hipGetLastError());
     return TPM_OK;
 }

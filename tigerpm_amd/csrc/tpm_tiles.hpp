@@ -15,6 +15,9 @@ struct tpm_tile_args {
     int32_t nbox;
     const tpm_box_dev* boxes;
     int C, min_rung;
+    int64_t n;        // particles of the box (boxes: in the table)
+    int64_t n_all;    // particles of all cells
+    int per_cell;     // waves per cell of the build (set by tpm_tiles_make)
     uint32_t cell_w;
     int3 lo, hi;
     int ts;
@@ -27,11 +30,9 @@ struct tpm_tile_args {
     uint32_t* order;  // particles, cell by cell
 };
 
-// Float offsets of every particle from its cell's centre (raw units).
-tpm_status tpm_float_positions(std::string& err, hipStream_t s, const tpm_tile_args& a, float* fx, float* fy,
-                               float* fz);
 // The raw positions in the order of the tiles.
 tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const tpm_tile_args& a, uint32_t* x,
                                uint32_t* y, uint32_t* z);
-// Tiles of at most ts active sinks of one cell, in spatial order.
-tpm_status tpm_tiles_make(std::string& err, hipStream_t s, const tpm_tile_args& a);
+// Tiles of at most ts active sinks of one cell, in spatial order; with fx also
+// the float offset of every particle from its cell's centre (raw units).
+tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a, float* fx, float* fy, float* fz);
