@@ -1,4 +1,5 @@
 // tpm_api.hip -- the C ABI (include/tigerpm_hip.h).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -7,16 +8,94 @@
 
 tpm_status tpm_fft_release(tpm_ctx* ctx);
 
-// dst[r] = src[map[r]]: device arrays in the caller's order.
-__global__ static void gather_u32_kernel(int64_t n, const uint32_t* __restrict__ map, const uint32_t* __restrict__ src,
-                                         uint32_t* __restrict__ dst) {
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
-        dst[r] = src[map[r]];
+// Arrays to the host: entry r of each is src[r], or src[map[r]] (the
+// caller's order).  Page-locked destinations of up to READBACK_KERNEL bytes
+// together are written by one kernel for all arrays: a copy call costs the
+// host about 10 us.  Eight arrays (29 B per particle) of 32^3 particles take
+// 30 us against 97, of 64^3 149 against 218, of 93^3 432 against 490; at 256^3
+// (487 MB) the copies' 56.5 GB/s beat the kernel's 55.3.  Larger reads and
+// pageable destinations take one copy per array, through the staging buffer
+// where there is a map.
+constexpr int64_t READBACK_KERNEL = 64 << 20;
+struct ReadbackArgs {
+    const void* src[11];
+    void* dst[11];
+    int bytes[11];
+    const uint32_t* map;
+    int64_t n;
+};
+template <class V>
+__device__ __forceinline__ void readback_array(const ReadbackArgs& a, int k) {
+    const V* __restrict__ src = static_cast<const V*>(a.src[k]);
+    V* __restrict__ dst = static_cast<V*>(a.dst[k]);
+    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < a.n; r += (int64_t)gridDim.x * blockDim.x)
+        dst[r] = src[a.map ? (int64_t)a.map[r] : r];
 }
-__global__ static void gather_u8_kernel(int64_t n, const uint32_t* __restrict__ map, const uint8_t* __restrict__ src,
-                                        uint8_t* __restrict__ dst) {
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
-        dst[r] = src[map[r]];
+__global__ __launch_bounds__(256) static void readback_kernel(ReadbackArgs a) {
+    const int k = blockIdx.y;
+    if (a.bytes[k] == 4)
+        readback_array<uint32_t>(a, k);
+    else
+        readback_array<uint8_t>(a, k);
+}
+
+// The device address of [p, p + bytes) when it is page-locked host memory, else nullptr.
+static void* device_view(void* p, size_t bytes) {
+    hipPointerAttribute_t lo{}, hi{};
+    char* const last = static_cast<char*>(p) + bytes - 1;
+    if (hipPointerGetAttributes(&lo, p) != hipSuccess || hipPointerGetAttributes(&hi, last) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (lo.type != hipMemoryTypeHost || hi.type != hipMemoryTypeHost || !lo.devicePointer || !hi.devicePointer)
+        return nullptr;
+    if (static_cast<char*>(hi.devicePointer) - static_cast<char*>(lo.devicePointer) != (ptrdiff_t)(bytes - 1))
+        return nullptr;
+    return lo.devicePointer;
+}
+
+tpm_status tpm_readback(std::string& err, hipStream_t s, int64_t n, const tpm_copy* cp, int count,
+                        const uint32_t* map, uint32_t* staging) {
+    ReadbackArgs a{};
+    a.map = map;
+    a.n = n;
+    int used = 0;
+    int64_t each = 0;
+    for (int k = 0; k < count; k++) each += cp[k].dst ? cp[k].bytes : 0;
+    bool kernel = each * n <= READBACK_KERNEL;
+    for (int k = 0; k < count && kernel; k++) {
+        if (!cp[k].dst) continue;
+        a.src[used] = cp[k].src;
+        a.bytes[used] = cp[k].bytes;
+        a.dst[used] = device_view(cp[k].dst, (size_t)cp[k].bytes * n);
+        kernel = a.dst[used] != nullptr;
+        used++;
+    }
+    if (kernel) {
+        if (used == 0) return TPM_OK;
+        readback_kernel<<<dim3(std::min(grid_for(n, 256), 256u), (unsigned)used), 256, 0, s>>>(a);
+        TPM_HIPE(err, hipGetLastError());
+        return TPM_OK;
+    }
+    for (int k = 0; k < count; k++) {
+        if (!cp[k].dst) continue;
+        const void* src = cp[k].src;
+        if (map) {
+            // into the staging buffer first (stream order keeps its copy
+            // ahead of the next array's)
+            ReadbackArgs g{};
+            g.map = map;
+            g.n = n;
+            g.src[0] = src;
+            g.dst[0] = staging;
+            g.bytes[0] = cp[k].bytes;
+            readback_kernel<<<dim3(grid_for(n, 256), 1), 256, 0, s>>>(g);
+            TPM_HIPE(err, hipGetLastError());
+            src = staging;
+        }
+        TPM_HIPE(err, hipMemcpyAsync(cp[k].dst, src, (size_t)cp[k].bytes * n, hipMemcpyDeviceToHost, s));
+    }
+    return TPM_OK;
 }
 
 static std::once_flag g_fft_once;
@@ -243,31 +322,12 @@ extern "C" tpm_status tpm_particles_download(tpm_ctx* ctx, uint32_t* x, uint32_t
     const int64_t n = ctx->n;
     hipStream_t s = ctx->stream;
     if (n > 0) {
-        struct {
-            void* dst;
-            const void* src;
-            size_t bytes;
-        } cp[] = {{x, ctx->x, 4}, {y, ctx->y, 4}, {z, ctx->z, 4},   {vx, ctx->vx, 4},   {vy, ctx->vy, 4},   {vz, ctx->vz, 4},
-                  {rung, ctx->rung, 1}, {gx, ctx->gx, 4}, {gy, ctx->gy, 4}, {gz, ctx->gz, 4}, {pot, ctx->pot, 4}};
-        // The caller's order differs from the device's: gather each array
-        // through h2d into a staging buffer first (stream order keeps the
-        // staging buffer's copy ahead of the next gather).
+        const tpm_copy cp[] = {{x, ctx->x, 4},       {y, ctx->y, 4},   {z, ctx->z, 4},   {vx, ctx->vx, 4},
+                               {vy, ctx->vy, 4},     {vz, ctx->vz, 4}, {rung, ctx->rung, 1}, {gx, ctx->gx, 4},
+                               {gy, ctx->gy, 4},     {gz, ctx->gz, 4}, {pot, ctx->pot, 4}};
+        // the caller's order, where it differs from the device's
         const bool mapped = ctx->host_order == TPM_ORDER_REFERENCE && !ctx->h2d_identity;
-        for (auto& c : cp) {
-            if (!c.dst) continue;
-            const void* src = c.src;
-            if (mapped) {
-                if (c.bytes == 4)
-                    gather_u32_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, ctx->h2d, (const uint32_t*)c.src,
-                                                                       ctx->ref_cid2);
-                else
-                    gather_u8_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, ctx->h2d, (const uint8_t*)c.src,
-                                                                      (uint8_t*)ctx->ref_cid2);
-                TPM_HIP(ctx, hipGetLastError());
-                src = ctx->ref_cid2;
-            }
-            TPM_HIP(ctx, hipMemcpyAsync(c.dst, src, c.bytes * n, hipMemcpyDeviceToHost, s));
-        }
+        TPM_TRY(tpm_readback(ctx->err, s, n, cp, 11, mapped ? ctx->h2d : nullptr, ctx->ref_cid2));
     }
     TPM_HIP(ctx, hipStreamSynchronize(s));
     return TPM_OK;

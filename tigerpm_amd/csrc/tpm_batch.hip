@@ -610,16 +610,10 @@ extern "C" tpm_status tpm_batch_download(tpm_batch* bt, int id, uint32_t* x, uin
     (void)hipSetDevice(bt->device);
     const int64_t o = b->p0, n = b->n;
     hipStream_t s = bt->stream;
-    struct {
-        void* dst;
-        const void* src;
-        size_t bytes;
-    } cp[] = {{x, bt->x + o, 4 * (size_t)n},    {y, bt->y + o, 4 * (size_t)n},   {z, bt->z + o, 4 * (size_t)n},
-              {vx, bt->vx + o, 4 * (size_t)n},  {vy, bt->vy + o, 4 * (size_t)n}, {vz, bt->vz + o, 4 * (size_t)n},
-              {rung, bt->rung + o, (size_t)n},  {gx, bt->gx + o, 4 * (size_t)n}, {gy, bt->gy + o, 4 * (size_t)n},
-              {gz, bt->gz + o, 4 * (size_t)n},  {pot, bt->pot + o, 4 * (size_t)n}};
-    for (auto& c : cp)
-        if (c.dst) TPM_HIP(bt, hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, s));
+    const tpm_copy cp[] = {{x, bt->x + o, 4},     {y, bt->y + o, 4},   {z, bt->z + o, 4},       {vx, bt->vx + o, 4},
+                           {vy, bt->vy + o, 4},   {vz, bt->vz + o, 4}, {rung, bt->rung + o, 1}, {gx, bt->gx + o, 4},
+                           {gy, bt->gy + o, 4},   {gz, bt->gz + o, 4}, {pot, bt->pot + o, 4}};
+    TPM_TRY(tpm_readback(bt->err, s, n, cp, 11, nullptr, nullptr));
     TPM_HIP(bt, hipStreamSynchronize(s));
     return TPM_OK;
 }

@@ -595,6 +595,16 @@ tpm_status tpm_ewald_noalloc_run(tpm_ctx* ctx, int64_t ns, const uint32_t* spx, 
                                  const uint32_t* spz, double alpha, double* phi, double* gx, double* gy, double* gz);
 tpm_status tpm_ic_zeldovich_run(tpm_ctx* ctx, int n_side, uint64_t seed, double rms_disp, double spectral_index);
 tpm_status tpm_ic_uniform_run(tpm_ctx* ctx, int64_t n, uint64_t seed);
+// One particle array for the host: n entries of 4 or 1 bytes (dst nullptr: not wanted).
+struct tpm_copy {
+    void* dst;
+    const void* src;
+    int bytes;
+};
+// Enqueues the copies (n >= 1, count <= 11), in the order of map unless it is
+// nullptr; staging: n words on the device, needed with a map.
+tpm_status tpm_readback(std::string& err, hipStream_t s, int64_t n, const tpm_copy* cp, int count,
+                        const uint32_t* map, uint32_t* staging);
 // Exclusive scan (tpm_chainmesh.hip).
 tpm_status tpm_scan_i32(std::string& err, hipStream_t s, const int32_t* in, int64_t n, int32_t* part, int32_t* out);
 tpm_status tpm_fill_u64(tpm_ctx* ctx, unsigned long long* p, int64_t n);
