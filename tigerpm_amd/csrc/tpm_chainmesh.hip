@@ -23,10 +23,13 @@ namespace {
 // Onesweep radix sort with 9-bit digits: the 512^3 keys (26 bits) take three
 // passes instead of four (6.0 vs 6.5 ms for the whole chain mesh, same
 // permutation: the sort is stable, so the digit width cannot change it).
+// Onesweep at every size: rocPRIM's merge sort below 2^20 keys takes 16
+// launches for a 64^3 box, onesweep 6 (27 us of its 0.72 ms step).
 using ChainSortConfig = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<512, 12>, rocprim::kernel_config<512, 12>, 9,
-                                        rocprim::block_radix_rank_algorithm::match>>;
+                                        rocprim::block_radix_rank_algorithm::match>,
+    0>;
 
 __global__ void key_kernel(int64_t n, const uint32_t* __restrict__ x, const uint32_t* __restrict__ y,
                            const uint32_t* __restrict__ z, int C, const uint32_t* __restrict__ bnd,
