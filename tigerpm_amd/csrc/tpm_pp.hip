@@ -323,15 +323,13 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
                 for (int k = 0; k < 4; k++) s[k] = fbuf[q + k * SPLIT + stream];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
-                    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                    float e = __builtin_amdgcn_exp2f(-u);
-                    if (!PME) {
-                        const bool in = u < ulo;
-                        window |= __ballot(u < uhi) & ~__ballot(in);
-                        e = in ? e : 0.f;
+                    if constexpr (PME) {
+                        const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
+                        const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                        pp_far(dx, dy, dz, u, __builtin_amdgcn_exp2f(-u), gx, gy, gz, ph);
+                    } else {
+                        pp_far_cut(s[k], fox, foy, foz, ulo, uhi, window, gx, gy, gz, ph);
                     }
-                    pp_far(dx, dy, dz, u, e, gx, gy, gz, ph);
                 }
             }
             if (!PME && window) {

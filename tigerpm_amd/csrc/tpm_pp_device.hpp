@@ -173,6 +173,19 @@ __device__ __forceinline__ void pp_far(float dx, float dy, float dz, float u, fl
     ph = fmaf(ew, p, ph);
 }
 
+// pp_far with the cutoff of a source s and a sink (fox, foy, foz): pairs
+// with u below ulo are inside, at or above uhi outside, and where any lane's
+// lies between (added as if outside) its bit in window is set.
+__device__ __forceinline__ void pp_far_cut(const float4& s, float fox, float foy, float foz, float ulo, float uhi,
+                                           unsigned long long& window, float& gx, float& gy, float& gz, float& ph) {
+    const float dx = s.x - fox, dy = s.y - foy, dz = s.z - foz;
+    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    const bool in = u < ulo;
+    window |= __ballot(u < uhi) & ~__ballot(in);
+    const float e = __builtin_amdgcn_exp2f(-u);
+    pp_far(dx, dy, dz, u, in ? e : 0.f, gx, gy, gz, ph);
+}
+
 // 6-point quintic weights (kick_treepm.cu:527-549) in Horner form.
 __device__ __forceinline__ void interp6_weights(float x, float w[6], float dw[6]) {
     w[0] = x * ((1.f / 12.f) + x * (-(1.f / 24.f) + x * (-(3.f / 8.f) + x * ((13.f / 24.f) + x * -(5.f / 24.f)))));

@@ -47,15 +47,7 @@ __global__ __launch_bounds__(64, 8) void pair_rate_kernel(tpm_box_dev B, int ite
 #pragma unroll
             for (int k = 0; k < 4; k++) s[k] = fbuf[q + k * PROBE_SPLIT + stream];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
-                const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                float e = __builtin_amdgcn_exp2f(-u);
-                const bool in = u < ulo;
-                window |= __ballot(u < uhi) & ~__ballot(in);
-                e = in ? e : 0.f;
-                pp_far(dx, dy, dz, u, e, gx, gy, gz, ph);
-            }
+            for (int k = 0; k < 4; k++) pp_far_cut(s[k], fox, foy, foz, ulo, uhi, window, gx, gy, gz, ph);
         }
     }
     if (window) ph += 1e-30f;
