@@ -5,7 +5,7 @@
 // FFTW r2c (fft.cpp:51-67), apply_laplacian (:201-245), inverse FFT
 // normalised by 1/N^3 (fft.cpp:468, 512).  Here the deposit accumulates
 // integer Q32 weights with 64-bit atomics (order-independent, so the grid is
-// bit-exact and deterministic), the 3-D transforms run in rocFFT, and the
+// bit-exact and deterministic), the 3-D transforms run in tpm_fft.hip or rocFFT, and the
 // deposit factor 4 pi M, the PME filter, the assignment deconvolution and the
 // 1/M^3 normalisation live in one FP32 Green's table built in FP64.
 // Optionally (interlace) a second deposit onto the grid displaced by half a
@@ -686,7 +686,7 @@ tpm_status tpm_pm_solve(tpm_ctx* ctx) {
         ctx->green_order = ctx->p.order;
         ctx->green_t_valid = false;
     }
-    if (ctx->fft.plans->tw && !ctx->p.interlace) {
+    if (ctx->fft.plans->tw && tpm_lds_fft_pow2(M) && !ctx->p.interlace) {
         // LDS-tiled transform: the Q32 conversion inside its first pass, the
         // Green's multiply between the forward and inverse x transforms of
         // one pass (same arithmetic as the separate kernels), its factors
