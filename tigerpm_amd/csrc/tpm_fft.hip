@@ -494,8 +494,13 @@ void launch_pm(hipStream_t st, const unsigned long long* q, float* phi, float2* 
 // component.  Bound by LDS reads: a thread makes NM outputs and their
 // mirrors from each pair that it reads (Poisson solve of a 97^3 mesh: 1 output
 // 171 us, 2 155, 4 143; with eight rows per workgroup instead of sixteen, whose
-// smaller LDS lets more of them share a CU, 2 outputs 124, 4 139).
+// smaller LDS lets more of them share a CU, 2 outputs 124, 4 139).  The
+// terms are summed in blocks of SUM_BLK: a density's mean makes the partial
+// sums of one long chain grow to p / 2 terms before they cancel, and its rounding
+// is the PM force's error (97^3, rms of the force: one chain 8.5e-6, blocks of 8
+// 4.2e-6, rocFFT 5.6e-6; no change in time, nor blocks of 4 or 6 in either).
 constexpr int NM = 2;
+constexpr int SUM_BLK = 8;
 struct GenPlan {
     int M;
     int nstage;
@@ -623,20 +628,31 @@ __device__ __forceinline__ void gen_stage_prime(float2* __restrict__ x, float2* 
             m[u] = min(g * NM + u, Q);  // past the last: it again
             q[u] = 0;
         }
+        for (int r0 = 1; r0 <= Q; r0 += SUM_BLK) {
+            float2 cb[NM], db[NM];
+#pragma unroll
+            for (int u = 0; u < NM; u++) cb[u] = db[u] = make_float2(0.f, 0.f);
+            const int r1 = min(r0 + SUM_BLK, Q + 1);
 #pragma unroll 2
-        for (int r = 1; r <= Q; r++) {
-            i1 += mr;
-            i2 -= mr;
-            const float2 xa = x[lds_at<T>(t, i1)], xb = x[lds_at<T>(t, i2)];
+            for (int r = r0; r < r1; r++) {
+                i1 += mr;
+                i2 -= mr;
+                const float2 xa = x[lds_at<T>(t, i1)], xb = x[lds_at<T>(t, i2)];
+#pragma unroll
+                for (int u = 0; u < NM; u++) {
+                    q[u] += m[u];
+                    q[u] -= q[u] >= p ? p : 0;
+                    const float2 w = tw[q[u] * mr];
+                    cb[u].x = fmaf(xa.x, w.x, cb[u].x);
+                    cb[u].y = fmaf(xa.y, w.x, cb[u].y);
+                    db[u].x = fmaf(xb.x, -w.y, db[u].x);
+                    db[u].y = fmaf(xb.y, -w.y, db[u].y);
+                }
+            }
 #pragma unroll
             for (int u = 0; u < NM; u++) {
-                q[u] += m[u];
-                q[u] -= q[u] >= p ? p : 0;
-                const float2 w = tw[q[u] * mr];
-                c[u].x = fmaf(xa.x, w.x, c[u].x);
-                c[u].y = fmaf(xa.y, w.x, c[u].y);
-                d[u].x = fmaf(xb.x, -w.y, d[u].x);
-                d[u].y = fmaf(xb.y, -w.y, d[u].y);
+                c[u] = cadd(c[u], cb[u]);
+                d[u] = cadd(d[u], db[u]);
             }
         }
         const int i0 = (j - k) * p + k;
@@ -861,11 +877,10 @@ bool tpm_lds_fft_pow2(int M) { return M >= 16 && M <= 1024 && (M & (M - 1)) == 0
 // transforms, transposes: 30 to 60 launches for a solve).  Poisson solve, general kernels
 // against rocFFT, in us: 38^3 50 / 102, 61^3 66 / 139, 93^3 86 / 212,
 // 101^3 126 / 226, 155^3 189 / 501, 217^3 343 / 973, 244^3 591 / 719, 279^3
-// 751 / 2968, 332^3 1871 / 2171, 380^3 2078 / 3085.  The rounding error of the
-// direct prime stage grows with p but stays below the convolution's (relative
-// rms of a 93^3 transform 1.6e-7 / 3.2e-7, 101^3 2.3e-7 / 3.5e-7).
-// The lines: for p > 101 even sizes gain nothing (226 = 2 113: 648 / 614) and from
-// p = 200 or so the inverse's error passes rocFFT's (211: 3.7e-7 / 3.3e-7);
+// 751 / 2968, 332^3 1871 / 2171, 380^3 2078 / 3085.  The rounding error is
+// below the convolution's: the PM force's over 14 sizes from 38 to 155, uniform
+// and Zel'dovich boxes, is 3.1e-6 / 4.6e-6 (rms), 0.66 of it in the mean.
+// The lines: for p > 101 even sizes lose (202 = 2 101 is a draw, 226 = 2 113 648 / 614);
 // above 384 large p lose (404 = 4 101: 5129 / 3710); without a factor
 // above 17 rocFFT is faster (100^3: 110 / 66).
 bool tpm_lds_fft_size(int M) {
