@@ -141,8 +141,7 @@ typedef struct {
                       240 B per particle of device memory), 0 = from each
                       end as the reference does, -1 = default */
     int fft;       /* mesh FFTs: 0 = this library's LDS-tiled transform for
-                      power-of-two meshes 16..1024 and for meshes up to 384
-                      whose largest prime factor is 19..101, rocFFT otherwise,
+                      power-of-two meshes 16..1024 and rocFFT otherwise,
                       1 = rocFFT for every size.  Both agree to FP32
                       rounding; a batch uses the default. */
 } tpm_tuning;

@@ -1,5 +1,5 @@
-// tpm_fft.hip -- 3-D real FFTs of cubic meshes whose size is a power of two
-// (16 .. 1024) or has a prime factor that rocFFT has no kernel for, LDS-tiled, in the layouts of fft3d_execute / fft3d_inv_execute
+// tpm_fft.hip -- 3-D real FFTs of power-of-two cubic meshes (16 .. 1024),
+// LDS-tiled, in the layouts of fft3d_execute / fft3d_inv_execute
 // (fft.cpp:51-84): R2C unnormalised, C2R unnormalised (the PM folds 1/M^3
 // into its Green's function, fft.cpp:468, 512).
 //
@@ -483,412 +483,9 @@ void launch_pm(hipStream_t st, const unsigned long long* q, float* phi, float2* 
     fft_z_c2r_kernel<M, T><<<M * (M / T), FFT_THREADS, 0, st>>>(spec, phi, tf);
 }
 
-
-// ---- Sizes with a larger prime factor (runtime M) ---------------------------
-// The same passes and layouts for M = product of the plan's radices.  Z and
-// Z' take two real rows as one complex row of M points, which needs no even
-// M.  A stage reads one LDS buffer and writes the other; radices up to 8 go
-// through registers, a larger prime p pairs its inputs r and p - r in place
-// (sum and difference) and makes outputs m and p - m together from
-// p / 2 terms each, so that a row costs p fused multiply-adds per point and
-// component.  Bound by LDS reads: a thread makes NM outputs and their
-// mirrors from each pair that it reads (Poisson solve of a 97^3 mesh: 1 output
-// 171 us, 2 155, 4 143; with eight rows per workgroup instead of sixteen, whose
-// smaller LDS lets more of them share a CU, 2 outputs 124, 4 139).  The
-// terms are summed in blocks of SUM_BLK: a density's mean makes the partial
-// sums of one long chain grow to p / 2 terms before they cancel, and its rounding
-// is the PM force's error (97^3, rms of the force: one chain 8.5e-6, blocks of 8
-// 4.2e-6, rocFFT 5.6e-6; no change in time, nor blocks of 4 or 6 in either).
-constexpr int NM = 2;
-constexpr int SUM_BLK = 8;
-struct GenPlan {
-    int M;
-    int nstage;
-    int radix[10];
-};
-
-__device__ __forceinline__ constexpr float odd_cos(int P, int q) {
-    // cos(2 pi q / P), q <= P / 2
-    constexpr float c3[2] = {1.f, -0.5f}, c5[3] = {1.f, 0.30901699437494742f, -0.80901699437494742f},
-                    c7[4] = {1.f, 0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f};
-    return P == 3 ? c3[q] : P == 5 ? c5[q] : c7[q];
-}
-__device__ __forceinline__ constexpr float odd_sin(int P, int q) {
-    constexpr float s3[2] = {0.f, 0.86602540378443865f}, s5[3] = {0.f, 0.95105651629515357f, 0.58778525229247313f},
-                    s7[4] = {0.f, 0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f};
-    return P == 3 ? s3[q] : P == 5 ? s5[q] : s7[q];
-}
-
-// DFT of odd length P in registers.
-template <int P, int DIR>
-__device__ __forceinline__ void dft_odd(float2* v) {
-    constexpr int Q = (P - 1) / 2;
-    float2 a[Q], b[Q];
-#pragma unroll
-    for (int r = 0; r < Q; r++) {
-        a[r] = cadd(v[r + 1], v[P - 1 - r]);
-        b[r] = csub(v[r + 1], v[P - 1 - r]);
-    }
-    const float2 x0 = v[0];
-#pragma unroll
-    for (int r = 0; r < Q; r++) v[0] = cadd(v[0], a[r]);
-#pragma unroll
-    for (int m = 1; m <= Q; m++) {
-        float2 c = x0, d = make_float2(0.f, 0.f);
-#pragma unroll
-        for (int r = 1; r <= Q; r++) {
-            const int q = (r * m) % P;
-            const float co = odd_cos(P, q > Q ? P - q : q);
-            const float si = q > Q ? -odd_sin(P, P - q) : odd_sin(P, q);
-            c.x = fmaf(a[r - 1].x, co, c.x);
-            c.y = fmaf(a[r - 1].y, co, c.y);
-            d.x = fmaf(b[r - 1].x, si, d.x);
-            d.y = fmaf(b[r - 1].y, si, d.y);
-        }
-        d = mul_i<DIR>(d);
-        v[m] = cadd(c, d);
-        v[P - m] = csub(c, d);
-    }
-}
-
-template <int R, int DIR>
-__device__ __forceinline__ void dft_any(float2* v) {
-    if constexpr (R == 2 || R == 4 || R == 8)
-        Dft<R, DIR>::run(v);
-    else
-        dft_odd<R, DIR>(v);
-}
-
-// e / d for e d < 2^32, by the multiplier ceil(2^32 / d); d = 1 has none.
-struct FastDiv {
-    unsigned d, mul;
-    __device__ explicit FastDiv(unsigned d_) : d(d_), mul(0xffffffffu / d_ + 1u) {}
-    __device__ unsigned div(unsigned e) const { return d == 1 ? e : __umulhi(e, mul); }
-};
-
-template <int T, int R, int DIR>
-__device__ __forceinline__ void gen_stage(const float2* __restrict__ x, float2* __restrict__ y,
-                                          const float2* __restrict__ tw, int M, int Ns) {
-    const int mr = M / R, ws = mr / Ns;
-    const FastDiv ns((unsigned)Ns);
-    for (int b = (int)threadIdx.x; b < T * mr; b += FFT_THREADS) {
-        const int t = b % T, j = b / T;
-        const int k = j - (int)ns.div((unsigned)j) * Ns;
-        float2 v[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = x[lds_at<T>(t, j + r * mr)];
-        if (Ns > 1) {
-#pragma unroll
-            for (int r = 1; r < R; r++) {
-                const float2 w = tw[r * k * ws];
-                v[r] = cmul(v[r], DIR < 0 ? w : conjc(w));
-            }
-        }
-        dft_any<R, DIR>(v);
-        const int i0 = (j - k) * R + k;
-#pragma unroll
-        for (int r = 0; r < R; r++) y[lds_at<T>(t, i0 + r * Ns)] = v[r];
-    }
-}
-
-// A prime p > 7; x is overwritten.  A thread makes NM outputs m and their
-// mirrors p - m from each pair of inputs that it reads.
-template <int T, int DIR>
-__device__ __forceinline__ void gen_stage_prime(float2* __restrict__ x, float2* __restrict__ y,
-                                                const float2* __restrict__ tw, int M, int Ns, int p) {
-    const int mr = M / p, ws = mr / Ns, Q = (p - 1) / 2;
-    const FastDiv ns((unsigned)Ns), dm((unsigned)mr);
-    for (int b = (int)threadIdx.x; b < T * mr * Q; b += FFT_THREADS) {
-        const int t = b % T, c = b / T;
-        const int r0 = (int)dm.div((unsigned)c), j = c - r0 * mr, r = r0 + 1;
-        const int i1 = lds_at<T>(t, j + r * mr), i2 = lds_at<T>(t, j + (p - r) * mr);
-        float2 u = x[i1], v = x[i2];
-        if (Ns > 1) {
-            const int k = j - (int)ns.div((unsigned)j) * Ns;
-            const float2 w1 = tw[r * k * ws], w2 = tw[(p - r) * k * ws];
-            u = cmul(u, DIR < 0 ? w1 : conjc(w1));
-            v = cmul(v, DIR < 0 ? w2 : conjc(w2));
-        }
-        x[i1] = cadd(u, v);
-        x[i2] = csub(u, v);
-    }
-    __syncthreads();
-    const int mg = (Q + NM) / NM;  // groups of the Q + 1 outputs m <= Q
-    for (int b = (int)threadIdx.x; b < T * mr * mg; b += FFT_THREADS) {
-        const int t = b % T, e = b / T;
-        const int g = (int)dm.div((unsigned)e), j = e - g * mr;
-        const int k = j - (int)ns.div((unsigned)j) * Ns;
-        const float2 x0 = x[lds_at<T>(t, j)];
-        float2 c[NM], d[NM];
-        int m[NM], q[NM], i1 = j, i2 = j + M;
-#pragma unroll
-        for (int u = 0; u < NM; u++) {
-            c[u] = x0;
-            d[u] = make_float2(0.f, 0.f);
-            m[u] = min(g * NM + u, Q);  // past the last: it again
-            q[u] = 0;
-        }
-        for (int r0 = 1; r0 <= Q; r0 += SUM_BLK) {
-            float2 cb[NM], db[NM];
-#pragma unroll
-            for (int u = 0; u < NM; u++) cb[u] = db[u] = make_float2(0.f, 0.f);
-            const int r1 = min(r0 + SUM_BLK, Q + 1);
-#pragma unroll 2
-            for (int r = r0; r < r1; r++) {
-                i1 += mr;
-                i2 -= mr;
-                const float2 xa = x[lds_at<T>(t, i1)], xb = x[lds_at<T>(t, i2)];
-#pragma unroll
-                for (int u = 0; u < NM; u++) {
-                    q[u] += m[u];
-                    q[u] -= q[u] >= p ? p : 0;
-                    const float2 w = tw[q[u] * mr];
-                    cb[u].x = fmaf(xa.x, w.x, cb[u].x);
-                    cb[u].y = fmaf(xa.y, w.x, cb[u].y);
-                    db[u].x = fmaf(xb.x, -w.y, db[u].x);
-                    db[u].y = fmaf(xb.y, -w.y, db[u].y);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < NM; u++) {
-                c[u] = cadd(c[u], cb[u]);
-                d[u] = cadd(d[u], db[u]);
-            }
-        }
-        const int i0 = (j - k) * p + k;
-#pragma unroll
-        for (int u = 0; u < NM; u++) {
-            const float2 di = mul_i<DIR>(d[u]);
-            y[lds_at<T>(t, i0 + m[u] * Ns)] = cadd(c[u], di);
-            if (m[u] > 0) y[lds_at<T>(t, i0 + (p - m[u]) * Ns)] = csub(c[u], di);
-        }
-    }
-}
-
-// The T rows of length M in s (s2: a second buffer); returns the buffer that
-// holds the result.  Begins and ends with a barrier.
-template <int T, int DIR>
-__device__ __forceinline__ float2* gen_rows(float2* s, float2* s2, const float2* tw, const GenPlan& P) {
-    int Ns = 1;
-    __syncthreads();
-    for (int i = 0; i < P.nstage; i++) {
-        const int R = P.radix[i];
-        switch (R) {
-            case 2: gen_stage<T, 2, DIR>(s, s2, tw, P.M, Ns); break;
-            case 3: gen_stage<T, 3, DIR>(s, s2, tw, P.M, Ns); break;
-            case 4: gen_stage<T, 4, DIR>(s, s2, tw, P.M, Ns); break;
-            case 5: gen_stage<T, 5, DIR>(s, s2, tw, P.M, Ns); break;
-            case 7: gen_stage<T, 7, DIR>(s, s2, tw, P.M, Ns); break;
-            case 8: gen_stage<T, 8, DIR>(s, s2, tw, P.M, Ns); break;
-            default: gen_stage_prime<T, DIR>(s, s2, tw, P.M, Ns, R); break;
-        }
-        Ns *= R;
-        float2* const t = s;
-        s = s2;
-        s2 = t;
-        __syncthreads();
-    }
-    return s;
-}
-
-__device__ __forceinline__ void gen_twiddles(float2* tw, const float2* __restrict__ tf, int M) {
-    for (int q = (int)threadIdx.x; q < M; q += FFT_THREADS) tw[q] = tf[q];
-}
-
-extern __shared__ __align__(16) float2 gen_lds[];
-
-// Z: real rows r[ix][iy0 + 0 .. 2T)[*], a pair per complex row.  Grid
-// M * ceil(M / 2T).
-template <int T>
-__global__ __launch_bounds__(FFT_THREADS) void gen_z_r2c_kernel(const float* __restrict__ in, float2* __restrict__ A,
-                                                               const float2* __restrict__ tf, GenPlan P) {
-    const int M = P.M, H = M / 2 + 1, nt = (M + 2 * T - 1) / (2 * T);
-    float2 *s = gen_lds, *s2 = s + T * M, *tw = s2 + T * M;
-    const int64_t ix = blockIdx.x / nt;
-    const int iy0 = (int)(blockIdx.x % nt) * 2 * T, tn = min(2 * T, M - iy0);
-    const float* src = in + (ix * M + iy0) * M;
-    const FastDiv dm((unsigned)M);
-    gen_twiddles(tw, tf, M);
-#pragma unroll 4
-    for (int e = (int)threadIdx.x; e < 2 * T * M; e += FFT_THREADS) {
-        const int row = (int)dm.div((unsigned)e), i = e - row * M;
-        const float v = row < tn ? src[e] : 0.f;
-        reinterpret_cast<float*>(&s[lds_at<T>(row >> 1, i)])[row & 1] = v;
-    }
-    const float2* z = gen_rows<T, -1>(s, s2, tw, P);
-    float2* dst = A + ix * H * M + iy0;
-    for (int e = (int)threadIdx.x; e < 2 * T * H; e += FFT_THREADS) {
-        const int k = e / (2 * T), tt = e % (2 * T);
-        if (tt >= tn) continue;
-        const float2 a = z[lds_at<T>(tt >> 1, k)], b = conjc(z[lds_at<T>(tt >> 1, k ? M - k : 0)]);
-        // first row (a + b) / 2, second (a - b) / 2i
-        const float2 d = tt & 1 ? mul_i<-1>(csub(a, b)) : cadd(a, b);
-        dst[(int64_t)k * M + tt] = make_float2(0.5f * d.x, 0.5f * d.y);
-    }
-}
-
-// Z': the reverse.  The imaginary parts of modes 0 and M / 2, which a real
-// row does not have, are left out.
-template <int T>
-__global__ __launch_bounds__(FFT_THREADS) void gen_z_c2r_kernel(const float2* __restrict__ A, float* __restrict__ out,
-                                                               const float2* __restrict__ tf, GenPlan P) {
-    const int M = P.M, H = M / 2 + 1, nt = (M + 2 * T - 1) / (2 * T);
-    float2 *s = gen_lds, *s2 = s + T * M, *tw = s2 + T * M;
-    const int64_t ix = blockIdx.x / nt;
-    const int iy0 = (int)(blockIdx.x % nt) * 2 * T, tn = min(2 * T, M - iy0);
-    const float2* src = A + ix * H * M + iy0;
-    gen_twiddles(tw, tf, M);
-#pragma unroll 4
-    for (int e = (int)threadIdx.x; e < T * H; e += FFT_THREADS) {
-        const int k = e / T, t = e % T;
-        const float2 zero = make_float2(0.f, 0.f);
-        float2 a = 2 * t < tn ? src[(int64_t)k * M + 2 * t] : zero;
-        float2 b = 2 * t + 1 < tn ? src[(int64_t)k * M + 2 * t + 1] : zero;
-        const int mk = k ? M - k : 0;
-        if (mk == k) a.y = b.y = 0.f;
-        s[lds_at<T>(t, k)] = make_float2(a.x - b.y, a.y + b.x);
-        if (mk != k) s[lds_at<T>(t, mk)] = make_float2(a.x + b.y, b.x - a.y);
-    }
-    const float2* z = gen_rows<T, 1>(s, s2, tw, P);
-    float* dst = out + (ix * M + iy0) * M;
-    const FastDiv dm((unsigned)M);
-    for (int e = (int)threadIdx.x; e < tn * M; e += FFT_THREADS) {
-        const int row = (int)dm.div((unsigned)e), i = e - row * M;
-        dst[e] = reinterpret_cast<const float*>(&z[lds_at<T>(row >> 1, i)])[row & 1];
-    }
-}
-
-// Y (FWD): A[ix0 + t][kz][*] -> B[kz][ky][ix0 + t];  Y' (!FWD): the reverse.
-// Grid H * ceil(M / T).
-template <int T, bool FWD>
-__global__ __launch_bounds__(FFT_THREADS) void gen_y_kernel(const float2* __restrict__ in, float2* __restrict__ out,
-                                                           const float2* __restrict__ tf, GenPlan P) {
-    const int M = P.M, H = M / 2 + 1, nt = (M + T - 1) / T;
-    float2 *s = gen_lds, *s2 = s + T * M, *tw = s2 + T * M;
-    const int64_t kz = blockIdx.x / nt;
-    const int ix0 = (int)(blockIdx.x % nt) * T, tn = min(T, M - ix0);
-    const FastDiv dm((unsigned)M);
-    const float2 zero = make_float2(0.f, 0.f);
-    gen_twiddles(tw, tf, M);
-#pragma unroll 4
-    for (int e = (int)threadIdx.x; e < T * M; e += FFT_THREADS) {
-        if (FWD) {
-            const int t = (int)dm.div((unsigned)e), i = e - t * M;
-            s[lds_at<T>(t, i)] = t < tn ? in[((int64_t)(ix0 + t) * H + kz) * M + i] : zero;
-        } else {
-            const int i = e / T, t = e % T;
-            s[lds_at<T>(t, i)] = t < tn ? in[(kz * M + i) * M + ix0 + t] : zero;
-        }
-    }
-    const float2* z = gen_rows<T, FWD ? -1 : 1>(s, s2, tw, P);
-    for (int e = (int)threadIdx.x; e < T * M; e += FFT_THREADS) {
-        if (FWD) {
-            const int i = e / T, t = e % T;
-            if (t < tn) out[(kz * M + i) * M + ix0 + t] = z[lds_at<T>(t, i)];
-        } else {
-            const int t = (int)dm.div((unsigned)e), i = e - t * M;
-            if (t < tn) out[((int64_t)(ix0 + t) * H + kz) * M + i] = z[lds_at<T>(t, i)];
-        }
-    }
-}
-
-// X (FWD): B[kz0 + t][ky][*] -> S[kx][ky][kz0 + t];  X' (!FWD): the reverse.
-// Grid M * ceil(H / T).
-template <int T, bool FWD>
-__global__ __launch_bounds__(FFT_THREADS) void gen_x_kernel(const float2* __restrict__ in, float2* __restrict__ out,
-                                                           const float2* __restrict__ tf, GenPlan P) {
-    const int M = P.M, H = M / 2 + 1, nt = (H + T - 1) / T;
-    float2 *s = gen_lds, *s2 = s + T * M, *tw = s2 + T * M;
-    const int64_t ky = blockIdx.x / nt;
-    const int kz0 = (int)(blockIdx.x % nt) * T, tn = min(T, H - kz0);
-    const FastDiv dm((unsigned)M);
-    const float2 zero = make_float2(0.f, 0.f);
-    gen_twiddles(tw, tf, M);
-#pragma unroll 4
-    for (int e = (int)threadIdx.x; e < T * M; e += FFT_THREADS) {
-        if (FWD) {
-            const int t = (int)dm.div((unsigned)e), i = e - t * M;
-            s[lds_at<T>(t, i)] = t < tn ? in[((int64_t)(kz0 + t) * M + ky) * M + i] : zero;
-        } else {
-            const int i = e / T, t = e % T;
-            s[lds_at<T>(t, i)] = t < tn ? in[((int64_t)i * M + ky) * H + kz0 + t] : zero;
-        }
-    }
-    const float2* z = gen_rows<T, FWD ? -1 : 1>(s, s2, tw, P);
-    for (int e = (int)threadIdx.x; e < T * M; e += FFT_THREADS) {
-        if (FWD) {
-            const int i = e / T, t = e % T;
-            if (t < tn) out[((int64_t)i * M + ky) * H + kz0 + t] = z[lds_at<T>(t, i)];
-        } else {
-            const int t = (int)dm.div((unsigned)e), i = e - t * M;
-            if (t < tn) out[((int64_t)(kz0 + t) * M + ky) * M + i] = z[lds_at<T>(t, i)];
-        }
-    }
-}
-
-// Radices of M: primes above 7 first (no twiddles there), then 7 .. 3, 8, 4
-// and 2.  Returns the largest radix.
-int gen_plan(int M, GenPlan* P) {
-    P->M = M;
-    P->nstage = 0;
-    int rest = M, big = 1;
-    for (int p = 11; p <= rest; p += 2)
-        while (rest % p == 0) {
-            P->radix[P->nstage++] = p;
-            rest /= p;
-            big = std::max(big, p);
-        }
-    for (int R : {7, 5, 3, 8, 4, 2})
-        while (rest % R == 0) {
-            P->radix[P->nstage++] = R;
-            rest /= R;
-            big = std::max(big, R);
-        }
-    return big;
-}
-
-template <int T>
-void gen_r2c(hipStream_t st, const GenPlan& P, const float* in, float2* out, float2* work, const float2* tf) {
-    const int M = P.M, H = M / 2 + 1;
-    const size_t lds = sizeof(float2) * (size_t)(2 * T + 1) * M;
-    gen_z_r2c_kernel<T><<<M * ((M + 2 * T - 1) / (2 * T)), FFT_THREADS, lds, st>>>(in, out, tf, P);
-    gen_y_kernel<T, true><<<H * ((M + T - 1) / T), FFT_THREADS, lds, st>>>(out, work, tf, P);
-    gen_x_kernel<T, true><<<M * ((H + T - 1) / T), FFT_THREADS, lds, st>>>(work, out, tf, P);
-}
-
-template <int T>
-void gen_c2r(hipStream_t st, const GenPlan& P, float2* in, float* out, float2* work, const float2* tf) {
-    const int M = P.M, H = M / 2 + 1;
-    const size_t lds = sizeof(float2) * (size_t)(2 * T + 1) * M;
-    gen_x_kernel<T, false><<<M * ((H + T - 1) / T), FFT_THREADS, lds, st>>>(in, work, tf, P);
-    gen_y_kernel<T, false><<<H * ((M + T - 1) / T), FFT_THREADS, lds, st>>>(work, in, tf, P);
-    gen_z_c2r_kernel<T><<<M * ((M + 2 * T - 1) / (2 * T)), FFT_THREADS, lds, st>>>(in, out, tf, P);
-}
-
-#define GEN_T 8      // complex rows per workgroup
-#define GEN_MAX 384  // two buffers of them and the twiddles: 51 KiB of LDS
-
 }  // namespace
 
-bool tpm_lds_fft_pow2(int M) { return M >= 16 && M <= 1024 && (M & (M - 1)) == 0; }
-
-// rocFFT has kernels for the radices up to 17; a larger prime factor it
-// transforms as a convolution of twice the length or more (chirps, two
-// transforms, transposes: 30 to 60 launches for a solve).  Poisson solve, general kernels
-// against rocFFT, in us: 38^3 50 / 102, 61^3 66 / 139, 93^3 86 / 212,
-// 101^3 126 / 226, 155^3 189 / 501, 217^3 343 / 973, 244^3 591 / 719, 279^3
-// 751 / 2968, 332^3 1871 / 2171, 380^3 2078 / 3085.  The rounding error is
-// below the convolution's: the PM force's over 14 sizes from 38 to 155, uniform
-// and Zel'dovich boxes, is 3.1e-6 / 4.6e-6 (rms), 0.66 of it in the mean.
-// The lines: for p > 101 even sizes lose (202 = 2 101 is a draw, 226 = 2 113 648 / 614);
-// above 384 large p lose (404 = 4 101: 5129 / 3710); without a factor
-// above 17 rocFFT is faster (100^3: 110 / 66).
-bool tpm_lds_fft_size(int M) {
-    if (tpm_lds_fft_pow2(M)) return true;
-    GenPlan P;
-    const int p = M >= 16 && M <= GEN_MAX ? gen_plan(M, &P) : 0;
-    return p >= 19 && p <= 101;
-}
+bool tpm_lds_fft_size(int M) { return M >= 16 && M <= 1024 && (M & (M - 1)) == 0; }
 
 tpm_status tpm_lds_fft_twiddles(std::string& err, int M, float2** tf) {
     std::vector<float2> h(M);
@@ -911,15 +508,7 @@ tpm_status tpm_lds_fft_r2c(std::string& err, hipStream_t st, int M, const void* 
         case 256: launch_r2c<256>(st, in, q32, out, work, tf, green); break;
         case 512: launch_r2c<512>(st, in, q32, out, work, tf, green); break;
         case 1024: launch_r2c<1024>(st, in, q32, out, work, tf, green); break;
-        default: {
-            if (!tpm_lds_fft_size(M) || q32 || green) {
-                err = "LDS FFT: unsupported size " + std::to_string(M);
-                return TPM_ERR_FFT;
-            }
-            GenPlan P;
-            gen_plan(M, &P);
-            gen_r2c<GEN_T>(st, P, static_cast<const float*>(in), out, work, tf);
-        }
+        default: err = "LDS FFT: unsupported size " + std::to_string(M); return TPM_ERR_FFT;
     }
     TPM_HIPE(err, hipGetLastError());
     return TPM_OK;
@@ -935,15 +524,7 @@ tpm_status tpm_lds_fft_c2r(std::string& err, hipStream_t st, int M, float2* in, 
         case 256: launch_c2r<256>(st, in, out, work, tf); break;
         case 512: launch_c2r<512>(st, in, out, work, tf); break;
         case 1024: launch_c2r<1024>(st, in, out, work, tf); break;
-        default: {
-            if (!tpm_lds_fft_size(M)) {
-                err = "LDS FFT: unsupported size " + std::to_string(M);
-                return TPM_ERR_FFT;
-            }
-            GenPlan P;
-            gen_plan(M, &P);
-            gen_c2r<GEN_T>(st, P, in, out, work, tf);
-        }
+        default: err = "LDS FFT: unsupported size " + std::to_string(M); return TPM_ERR_FFT;
     }
     TPM_HIPE(err, hipGetLastError());
     return TPM_OK;

@@ -43,7 +43,7 @@ inline void tpm_reduce_counters(const unsigned long long* h, unsigned long long 
 // Plans of one cubic size (single precision, out of place), shared by every
 // context and batch on the device: made once per (device, M, backend) and
 // kept until the process ends.  Backend: rocFFT, or this library's LDS-tiled
-// transform (tpm_fft.hip) for the sizes of tpm_lds_fft_size, whose plan is its
+// transform (tpm_fft.hip) for power-of-two M in [16, 1024], whose plan is its
 // twiddle table.
 struct tpm_fft_plans {
     rocfft_plan fwd = nullptr;  // R2C
@@ -66,8 +66,7 @@ struct tpm_fft {
     void* work = nullptr;
     size_t work_bytes = 0;
 };
-bool tpm_lds_fft_pow2(int M);  // the power-of-two kernels (all of the passes below)
-bool tpm_lds_fft_size(int M);  // those and the general ones (float input, no Green's factors: r2c and c2r)
+bool tpm_lds_fft_size(int M);
 tpm_status tpm_lds_fft_twiddles(std::string& err, int M, float2** tf);
 // in: M^3 floats, or with q32 the int64 Q32 density grid; green: the PM's
 // Green's table applied to the spectrum as it is stored (nullptr: none).

@@ -686,7 +686,7 @@ tpm_status tpm_pm_solve(tpm_ctx* ctx) {
         ctx->green_order = ctx->p.order;
         ctx->green_t_valid = false;
     }
-    if (ctx->fft.plans->tw && tpm_lds_fft_pow2(M) && !ctx->p.interlace) {
+    if (ctx->fft.plans->tw && !ctx->p.interlace) {
         // LDS-tiled transform: the Q32 conversion inside its first pass, the
         // Green's multiply between the forward and inverse x transforms of
         // one pass (same arithmetic as the separate kernels), its factors
