@@ -110,14 +110,15 @@ struct tpm_box_dev {
     // inside the softening length: 1 / (2 rs)^2 in 2^-64 units (x^2 = r2 *
     // inv4rs2_s) and 4 / (3 sqrt(pi)) / (2 rs)^3 in 2^-96 units
     float inv4rs2_s, k3_s;
-    // far pairs (pp_far): lengths times far_s are x sqrt(log2 e), x = r / (2 rs)
-    float far_s;                // per 2^-32 unit
-    float far_near2, far_cull2; // squared distances from a tile's box, far_s units: below the first a source's
+    // far pairs (pp_far), offsets in 2^-32 units
+    float far_u;                // x^2 log2(e) = squared offset * far_u, x = r / (2 rs)
+    float far_near2, far_cull2; // squared distances from a tile's box: below the first a source's
                                 // pairs take the general law, at or beyond the second it is dropped
+    float far_wide, far_all2;   // a tile of a larger half width uses far_all2 for far_near2: no far source
     float far_ulo, far_uhi;     // the cutoff as u, less and more than any rounding of u
     float far_wrap;             // largest |offset| + box half width whose differences cannot wrap
     float far_g, far_ph;        // sums of pp_far -> box units
-    uint32_t cell_w;            // 2^32 / C: cell k's float positions are offsets from k cell_w + cell_w / 2
+    uint32_t cell_w;            // 2^32 / C: cell k's centre is near k cell_w + cell_w / 2
     uint64_t rcut2i;            // a pair is inside the cutoff when its squared raw offset is below this
     // kick epilogue
     float GM, phi0, eta, t0, scale, hsoft;
@@ -165,16 +166,14 @@ struct tpm_ctx {
     uint32_t* bounds = nullptr;  // C split planes (raw values)
     int32_t* cell_begin = nullptr;
     int64_t cells_cap = 0;
-    // The direct kernel's sink tiles, made by every kick (tpm_pp_tiles):
+    // The direct kernel's sink tiles, made by every kick (tpm_tiles_make):
     // tile t holds the particles order[begin .. end) (order: the sort's idx
-    // buffer) of one cell.  The float positions lie in the second buffer set
-    // (x2, y2, z2), free between chain-mesh builds.
+    // buffer) of one cell.
     int32_t* tile_cnt = nullptr;   // tiles per cell
     int32_t* tile_off = nullptr;   // exclusive scan of tile_cnt, then their number
     int32_t* tile_part = nullptr;  // scan scratch
     int4* tiles = nullptr;         // (cell id, begin, end, 0)
     int64_t tiles_cap = 0;
-    int64_t fpos_epoch = -1;       // the chain-mesh build whose float positions are there
     bool chain_valid = false;
     int chain_C = 0;
     int tile = 16;        // sinks per PP tile: 16, 32 or 64 (tuning)

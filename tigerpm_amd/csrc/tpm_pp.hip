@@ -33,6 +33,7 @@
 #include "tpm_pp_device.hpp"
 #include "tpm_tiles.hpp"
 
+#include <cfloat>
 #include <climits>
 
 // Staged sources of a wave: far ones (float offsets) and near ones (int32
@@ -69,9 +70,6 @@ struct PPArgs {
     float* __restrict__ gz;
     float* __restrict__ pot;
     const int32_t* __restrict__ cell_begin;
-    const float* __restrict__ fx;   // float offsets from the cells' centres (tpm_float_positions)
-    const float* __restrict__ fy;
-    const float* __restrict__ fz;
     const int4* __restrict__ tiles;
     const int32_t* __restrict__ ntiles;
     const uint32_t* __restrict__ order;  // the particles of a tile: order[tile.y .. tile.z)
@@ -179,16 +177,31 @@ __device__ __forceinline__ int tile_max(int v) {
 
 // The short-range sums of one tile, by one wave: lane l has sink l % TS (raw
 // position px, py, pz) and walks stream l / TS.  The sources are those of the
-// 27 cells around cell (cx, cy, cz), 64 at a time, as float offsets from
-// their cell's centre: one FMA per axis makes them offsets from the centre of
-// the tile's box in far_s units.  Each source is tested against that box:
+// 27 cells around cell (cx, cy, cz), 64 at a time, as int32 offsets from the
+// centre of the tile's box, rounded to float once (2^-24 of the offset, which
+// is at most the pair's distance and half the box).  Each source is tested
+// against that box:
 //   beyond the cutoff (far_cull2, a margin of 2048 raw units over rcut, float
 //     rounding stays below 600): dropped;
-//   within far_near2 of the box: near list, as int32 offsets from the centre
-//     (made from the raw positions), evaluated with the general law (pp_pair);
+//   within far_near2 of the box: near list, as int32 offsets, evaluated with
+//     the general law (pp_pair);
 //   else: far list, as float offsets, evaluated with pp_far.  Every pair of a
 //     far source is at least FAR_X0 2 rs and h apart.
 // At 512^3 nine pairs of ten are far ones.
+// The float offsets' rounding grows with the box's half width H: a pair at
+// distance d is off by up to 2^-23 (d + H) per axis, where an exact difference
+// is rounded by 2^-24 d.  H is 1.1 rs in a full cell and at most 2.5 rs in the
+// sparsest at the usual ratios (half a cell); a wider box (few sinks in a
+// chain mesh much coarser than rcut) keeps the exact integer differences: its
+// sources all take the near list.  Error of a sink's pair sum against FP64
+// relative to the rms force, median over the sinks, exact differences and the
+// general law for every pair / this: 64^3 particles C = 11 1.9e-7 / 1.4e-7,
+// C = 5 2.0e-7 / 1.5e-7, 93^3 C = 5 3.1e-7 / 2.3e-7, 128^3 C = 5 2.3e-7 / 1.8e-7,
+// 20^3 on a 128^3 mesh, C = 5, 2.4e-8 for both.
+// (Offsets from the cells' centres stored once per chain mesh save the
+// conversions, but their rounding is that of a cell's width: 2.6e-7 at 128^3
+// C = 5, and a close pair is off by 2e-6 in cells of 160 rs.  Kicks at the
+// reference's ratios are 3 % slower without them, 120^3 25.6 -> 26.5 ms, the others the same.)
 // The cutoff of a far pair: float offsets are rounded by up to a few raw
 // units, and a pair on the wrong side of the cutoff is an error of
 // 5e-4 of a typical force, larger than all rounding together.  So u is
@@ -210,7 +223,6 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
     const int stream = lane / TS;
     const int C = B.C;
     const bool cull = B.cull != 0;
-    const float fs = B.far_s;
     // the box of the sinks with inbox: centre (raw) and half widths
     int ox = (int)(px - rx), oy = (int)(py - ry), oz = (int)(pz - rz);
     const int lox = tile_min<TS>(inbox ? ox : INT_MAX), hix = tile_max<TS>(inbox ? ox : INT_MIN);
@@ -220,19 +232,18 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
     // half the box, which C >= 3 rules out, but lo + hi may not fit
     const int mx = lox + (hix - lox) / 2, my = loy + (hiy - loy) / 2, mz = loz + (hiz - loz) / 2;
     const uint32_t qx = rx + (uint32_t)mx, qy = ry + (uint32_t)my, qz = rz + (uint32_t)mz;
-    const float hx = (float)max(hix - mx, mx - lox) * fs, hy = (float)max(hiy - my, my - loy) * fs,
-                hz = (float)max(hiz - mz, mz - loz) * fs;
+    const float hx = (float)max(hix - mx, mx - lox), hy = (float)max(hiy - my, my - loy),
+                hz = (float)max(hiz - mz, mz - loz);
+    const float near2 = fmaxf(hx, fmaxf(hy, hz)) > B.far_wide ? B.far_all2 : B.far_near2;
     ox -= mx;
     oy -= my;
     oz -= mz;
-    const float fox = (float)ox * fs, foy = (float)oy * fs, foz = (float)oz * fs;
+    const float fox = (float)ox, foy = (float)oy, foz = (float)oz;
     // kept in vector registers: an SGPR operand costs a VALU instruction half its rate
-    float ulo = B.far_ulo, uhi = B.far_uhi;
-    asm volatile("" : "+v"(ulo), "+v"(uhi));
-    // lane l < 27: neighbour cell l, its particles and its centre's offset
-    // from the box's
+    float ulo = B.far_ulo, uhi = B.far_uhi, fu = B.far_u;
+    asm volatile("" : "+v"(ulo), "+v"(uhi), "+v"(fu));
+    // lane l < 27: neighbour cell l's particles
     int rb = 0, re = 0;
-    float lx = 0.f, ly = 0.f, lz = 0.f;
     if (lane < 27) {
         int jx = cx + lane % 3 - 1, jy = cy + (lane / 3) % 3 - 1, jz = cz + lane / 9 - 1;
         jx += jx < 0 ? C : (jx >= C ? -C : 0);
@@ -241,19 +252,12 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
         const int c2 = B.cell0 + (jz * C + jy) * C + jx;
         rb = a.cell_begin[c2];
         re = a.cell_begin[c2 + 1];
-        const uint32_t w = B.cell_w;
-        lx = (float)(int)((uint32_t)jx * w + w / 2 - qx) * fs;
-        ly = (float)(int)((uint32_t)jy * w + w / 2 - qy) * fs;
-        lz = (float)(int)((uint32_t)jz * w + w / 2 - qz) * fs;
     }
     const uint32_t lane4 = 4u * (uint32_t)lane;
-    float fsv = fs;
-    asm volatile("" : "+v"(fsv));
     gx = gy = gz = ph = 0.f;
     float ngx = 0.f, ngy = 0.f, ngz = 0.f, nph = 0.f;
     int nfar = 0, nnear = 0;
     int cell = -1, j0 = 0, je = 0;
-    float cxo = 0.f, cyo = 0.f, czo = 0.f;
     for (;;) {
         // 64 sources, or after the last cell none
         bool more = true;
@@ -264,22 +268,20 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
             }
             j0 = __builtin_amdgcn_readlane(rb, cell);
             je = __builtin_amdgcn_readlane(re, cell);
-            cxo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lx), cell));
-            cyo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ly), cell));
-            czo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lz), cell));
         }
         if (more) {
             // lanes past the cell's end read its last particle and are masked
             const int left = je - j0;
             const unsigned long long valid = left >= 64 ? ~0ull : (1ull << left) - 1ull;
             const uint32_t off = min(lane4, 4u * (uint32_t)(left - 1));
-            const float fx = fmaf(*(const float*)((const char*)(a.fx + j0) + off), fsv, cxo);
-            const float fy = fmaf(*(const float*)((const char*)(a.fy + j0) + off), fsv, cyo);
-            const float fz = fmaf(*(const float*)((const char*)(a.fz + j0) + off), fsv, czo);
+            const int ix = (int)(*(const uint32_t*)((const char*)(a.x + j0) + off) - qx);
+            const int iy = (int)(*(const uint32_t*)((const char*)(a.y + j0) + off) - qy);
+            const int iz = (int)(*(const uint32_t*)((const char*)(a.z + j0) + off) - qz);
+            const float fx = (float)ix, fy = (float)iy, fz = (float)iz;
             const float ex = fmaxf(fabsf(fx) - hx, 0.f), ey = fmaxf(fabsf(fy) - hy, 0.f),
                         ez = fmaxf(fabsf(fz) - hz, 0.f);
             const float d2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
-            unsigned long long mn = __ballot(d2 < B.far_near2), mf;
+            unsigned long long mn = __ballot(d2 < near2), mf;
             if (cull) {
                 mf = __ballot(d2 < B.far_cull2) & ~mn & valid;
             } else {
@@ -299,14 +301,14 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
                 if (__builtin_amdgcn_inverse_ballot_w64(mn))
                     nbuf[__builtin_amdgcn_mbcnt_hi((unsigned)(mn >> 32),
                                                    __builtin_amdgcn_mbcnt_lo((unsigned)mn, nnear))] =
-                        make_int4((int)(a.x[j] - qx), (int)(a.y[j] - qy), (int)(a.z[j] - qz), j);
+                        make_int4(ix, iy, iz, j);
                 nnear += __popcll(mn);
             }
             j0 += 64;
         }
         if (nfar > FAR_AT || (!more && nfar > 0)) {
-            // Whole blocks of 4 rounds (four pairs in flight per lane: 83
-            // cycles per 64 pairs, 95 with two); the rest stays in the list,
+            // Whole blocks of 4 rounds (four pairs in flight per lane: 85
+            // cycles per 64 pairs, some 12 more with two); the rest stays in the list,
             // and after the last source is filled up with padding sources
             // beyond any cutoff (e = 0).
             int nblk = nfar / BLK * BLK;
@@ -325,10 +327,10 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
                 for (int k = 0; k < 4; k++) {
                     if constexpr (PME) {
                         const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
-                        const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                        const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) * fu;
                         pp_far(dx, dy, dz, u, __builtin_amdgcn_exp2f(-u), gx, gy, gz, ph);
                     } else {
-                        pp_far_cut(s[k], fox, foy, foz, ulo, uhi, window, gx, gy, gz, ph);
+                        pp_far_cut(s[k], fox, foy, foz, fu, ulo, uhi, window, gx, gy, gz, ph);
                     }
                 }
             }
@@ -336,7 +338,7 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
                 for (int q = 0; q < nblk; q += SPLIT) {
                     const float4 s = fbuf[q + stream];
                     const float dx = s.x - fox, dy = s.y - foy, dz = s.z - foz;
-                    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) * fu;
                     if (u >= ulo && u < uhi) {
                         const int j = __float_as_int(s.w);
                         if (pp_inside(B, (int)((qx + (uint32_t)ox) - a.x[j]), (int)((qy + (uint32_t)oy) - a.y[j]),
@@ -369,7 +371,7 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
         }
         if (!more) break;
     }
-    // box units: pp_pair's sums are in 2^-32 units, pp_far's in far_s units
+    // box units: pp_pair's sums and pp_far's offsets are in 2^-32 units
     gx = fmaf(ngx, 0x1p64f, gx * B.far_g);
     gy = fmaf(ngy, 0x1p64f, gy * B.far_g);
     gz = fmaf(ngz, 0x1p64f, gz * B.far_g);
@@ -998,27 +1000,29 @@ void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_c
     b->hinv_s = hinv / S;
     b->h2inv_s = (hinv * hinv) / (S * S);
     b->h3inv_s = ((hinv * hinv * hinv) / (S * S)) / S;
-    // pp_far: lengths in far_s units are x sqrt(log2 e).  Offsets span at
-    // most two cells (half a box); a source's float offset is rounded when it
-    // is converted and when it is scaled, a sink's likewise and their
-    // difference once more: 2^-22.5 of the span bounds the sum per axis, and
-    // u's own arithmetic adds less than 2^-22.
+    // pp_far.  far_wide bounds the half width H of a box with far sources.
+    // The window: an offset s of a source, o of a sink and their difference d
+    // are rounded to 2^-24 of themselves, |s| <= |d| + H, |o| <= H, so an axis
+    // of a pair at rcut is off by up to 2^-23 (rcut + H), r^2 by 2 sqrt(3)
+    // times that over rcut, and its own arithmetic, u's product and the
+    // second-order terms add less than 8 roundings of 2^-24.
     {
         const double two32 = 4294967296.0, l2e = 1.4426950408889634;
-        const float fs = (float)(std::sqrt(l2e) / (2.0 * p.rs) / two32);
-        const double fsd = fs;
-        b->far_s = fs;
-        const double nr = (std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * two32 + 2048.0) * fsd;
+        const float fu = (float)(l2e / (4.0 * p.rs * p.rs) / (two32 * two32));
+        b->far_u = fu;
+        const double nr = std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * two32 + 2048.0;
         b->far_near2 = (float)(nr * nr * (1.0 + 1e-6));
-        const double cr = (p.rcut * two32 + 2048.0) * fsd;
+        const double cr = p.rcut * two32 + 2048.0;
         b->far_cull2 = (float)(cr * cr * (1.0 + 1e-6));
-        const double rc = p.rcut * two32, uc = rc * rc * fsd * fsd;
-        const double span = std::min(2.0 / p.chain_dim, 0.5) * two32;
-        const double rel = 2.0 * std::sqrt(3.0) * std::exp2(-22.5) * span / rc + std::exp2(-22.0);
-        b->far_ulo = (float)(uc * (1.0 - rel) * (1.0 - 1e-7));
-        b->far_uhi = (float)(uc * (1.0 + rel) * (1.0 + 1e-7));
-        b->far_wrap = (float)(0x1p31 * fsd * (1.0 - 1e-5));
-        b->far_g = (float)(std::sqrt(l2e) / (4.0 * p.rs * p.rs));
+        const double wide = std::min(FAR_WIDE * p.rs, 0.5) * two32;
+        b->far_wide = (float)wide;
+        b->far_all2 = b->cull ? std::max(b->far_near2, b->far_cull2) : FLT_MAX;
+        const double rc = p.rcut * two32, uc = rc * rc * (double)fu;
+        const double rel = 2.0 * std::sqrt(3.0) * std::exp2(-23.0) * (rc + wide) / rc + std::exp2(-21.0);
+        b->far_ulo = (float)(uc * (1.0 - rel));
+        b->far_uhi = (float)(uc * (1.0 + rel));
+        b->far_wrap = (float)(0x1p31 * (1.0 - 1e-5));
+        b->far_g = (float)(l2e / (8.0 * p.rs * p.rs * p.rs) / two32);
         b->far_ph = (float)(1.0 / (2.0 * p.rs));
         b->rcut2i = (uint64_t)std::ceil(rc * rc);
     }
@@ -1108,6 +1112,7 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
     if (pme) {
         // kick_pme: every pair of the 27 cells counts, and phi starts at 0
         a.box0.cull = 0;
+        a.box0.far_all2 = FLT_MAX;
         a.box0.phi0 = 0.f;
     }
     a.flags = flags & (TPM_SKIP_PP | TPM_SKIP_PM | TPM_SKIP_KICK);
@@ -1156,8 +1161,7 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
         TPM_HIP(ctx, hipGetLastError());
     } else if (ctx->n > 0 && blocks > 0) {
         // the tiles of the active sinks (kick_pme: of every sink, so that its
-        // sums do not depend on which are active) and, once per chain mesh,
-        // the float positions
+        // sums do not depend on which are active)
         if (tiles_all > ctx->tiles_cap) {
             if (ctx->tiles) TPM_HIP(ctx, hipFree(ctx->tiles));
             ctx->tiles = nullptr;
@@ -1185,14 +1189,7 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
         t.part = ctx->tile_part;
         t.tiles = ctx->tiles;
         t.order = ctx->idx;
-        float *fx = reinterpret_cast<float*>(ctx->x2), *fy = reinterpret_cast<float*>(ctx->y2),
-              *fz = reinterpret_cast<float*>(ctx->z2);
-        const bool made = ctx->fpos_epoch == ctx->chain_epoch;
-        TPM_TRY(tpm_tiles_make(ctx->err, s, t, made ? nullptr : fx, fy, fz));
-        ctx->fpos_epoch = ctx->chain_epoch;
-        a.fx = fx;
-        a.fy = fy;
-        a.fz = fz;
+        TPM_TRY(tpm_tiles_make(ctx->err, s, t));
         a.tiles = ctx->tiles;
         a.ntiles = ctx->tile_off + ncell;
         a.order = ctx->idx;
@@ -1287,8 +1284,7 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
         TPM_HIP(bt, hipGetLastError());
         return TPM_OK;
     }
-    // the tiles of every box's active sinks; float positions in the buffer
-    // set that the gather has left, the order in the sort's slot buffer
+    // the tiles of every box's active sinks, their order in the sort's slot buffer
     tpm_tile_args t{};
     t.x = bt->x;
     t.y = bt->y;
@@ -1305,12 +1301,7 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
     t.part = bt->scan_part;
     t.tiles = bt->tiles;
     t.order = bt->slot;
-    float *fx = reinterpret_cast<float*>(bt->x2), *fy = reinterpret_cast<float*>(bt->y2),
-          *fz = reinterpret_cast<float*>(bt->z2);
-    TPM_TRY(tpm_tiles_make(bt->err, bt->stream, t, fx, fy, fz));
-    a.fx = fx;
-    a.fy = fy;
-    a.fz = fz;
+    TPM_TRY(tpm_tiles_make(bt->err, bt->stream, t));
     a.tiles = bt->tiles;
     a.ntiles = bt->tile_off + L.ncell;
     a.order = bt->slot;

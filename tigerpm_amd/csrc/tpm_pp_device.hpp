@@ -141,8 +141,9 @@ __device__ __forceinline__ void pp_pair_exact(const tpm_box_dev& a, int ox, int 
 }
 
 // The same law for a pair at least FAR_X0 * 2 rs and h apart: no softening,
-// and erfc by one polynomial instead of A&S 7.1.26.  Lengths come scaled so
-// that u = x^2 log2(e), x = r / (2 rs): e = exp2(-u) = exp(-x^2) and
+// and erfc by one polynomial instead of A&S 7.1.26.  dx, dy, dz: source - sink
+// in 2^-32 units, u = x^2 log2(e), x = r / (2 rs): e = exp2(-u) = exp(-x^2),
+// which the caller gates by the cutoff, and
 // y = rsq(u).  erfc(x) / x = e y^2 P(y), P a polynomial of degree 6 in 1 / x
 // (the factors log2(e)^(k/2) are in its coefficients) fitted to erfcx(x) x
 // over x >= 0.71 to 5e-8 of erfc, a third of 7.1.26's error, and valid to
@@ -150,11 +151,11 @@ __device__ __forceinline__ void pp_pair_exact(const tpm_box_dev& a, int ox, int 
 // int-to-float conversions and constants that are literals: measured issue
 // cycles per wave64 on gfx950 are 2 to 2.7 for multiplies, adds and FMAs, 4.3
 // for the conversion, 8.2 for exp / rsq / rcp and 4.5 for an FMA with an SGPR
-// operand, so 83 cycles per 64 pairs here against 116 for pp_pair (PP stage of a
-// 256^3 kick 25.1 -> 22.2 ms, kick_pme 60^3 16.5 -> 12.8 ms).
-// (dx, dy, dz): source - sink; the caller gates e by the cutoff.
-// Sums: g += (source - sink) F, ph += erfc(x) / x, in far_s units.
+// operand, so 85 cycles per 64 pairs here against 112 for pp_pair
+// (the far loop alone, 8 waves per SIMD).
+// Sums: g += (source - sink) F, ph += erfc(x) / x, to be scaled by far_g and far_ph.
 #define FAR_X0 0.72
+#define FAR_WIDE 3.0  // rs: half width of a box of sinks whose far sources pp_far takes (pp_sum)
 __device__ __forceinline__ void pp_far(float dx, float dy, float dz, float u, float e, float& gx, float& gy,
                                        float& gz, float& ph) {
     const float y = __builtin_amdgcn_rsqf(u);
@@ -176,10 +177,10 @@ __device__ __forceinline__ void pp_far(float dx, float dy, float dz, float u, fl
 // pp_far with the cutoff of a source s and a sink (fox, foy, foz): pairs
 // with u below ulo are inside, at or above uhi outside, and where any lane's
 // lies between (added as if outside) its bit in window is set.
-__device__ __forceinline__ void pp_far_cut(const float4& s, float fox, float foy, float foz, float ulo, float uhi,
-                                           unsigned long long& window, float& gx, float& gy, float& gz, float& ph) {
+__device__ __forceinline__ void pp_far_cut(const float4& s, float fox, float foy, float foz, float fu, float ulo,
+                                           float uhi, unsigned long long& window, float& gx, float& gy, float& gz, float& ph) {
     const float dx = s.x - fox, dy = s.y - foy, dz = s.z - foz;
-    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) * fu;
     const bool in = u < ulo;
     window |= __ballot(u < uhi) & ~__ballot(in);
     const float e = __builtin_amdgcn_exp2f(-u);

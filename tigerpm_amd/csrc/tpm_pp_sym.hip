@@ -550,9 +550,8 @@ tpm_status tpm_pp_kick_sym(tpm_ctx* ctx, double scale, double t0, int first_call
     t.off = ctx->tile_off;
     t.part = ctx->tile_part;
     t.order = ctx->idx;
-    TPM_TRY(tpm_tiles_make(ctx->err, s, t, nullptr, nullptr, nullptr));
+    TPM_TRY(tpm_tiles_make(ctx->err, s, t));
     TPM_TRY(tpm_order_positions(ctx->err, s, n, t, ctx->x2, ctx->y2, ctx->z2));
-    ctx->fpos_epoch = -1;
     SymArgs a{};
     a.x = ctx->x2;
     a.y = ctx->y2;

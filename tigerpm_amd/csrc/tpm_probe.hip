@@ -34,10 +34,9 @@ __global__ __launch_bounds__(64, 8) void pair_rate_kernel(tpm_box_dev B, int ite
         fbuf[k] = make_float4(c[0], c[1], c[2], 0.f);
     }
     __syncthreads();
-    const float fox = (slot * 4099 - 32768) * B.far_s, foy = (20011 - slot * 3001) * B.far_s,
-                foz = slot * 1777 * B.far_s;
-    float ulo = B.far_ulo, uhi = B.far_uhi;
-    asm volatile("" : "+v"(ulo), "+v"(uhi));
+    const float fox = slot * 4099 - 32768, foy = 20011 - slot * 3001, foz = slot * 1777;
+    float ulo = B.far_ulo, uhi = B.far_uhi, fu = B.far_u;
+    asm volatile("" : "+v"(ulo), "+v"(uhi), "+v"(fu));
     float gx = 0.f, gy = 0.f, gz = 0.f, ph = 0.f;
     unsigned long long window = 0ull;
     for (int it = 0; it < iters; it++) {
@@ -47,7 +46,7 @@ __global__ __launch_bounds__(64, 8) void pair_rate_kernel(tpm_box_dev B, int ite
 #pragma unroll
             for (int k = 0; k < 4; k++) s[k] = fbuf[q + k * PROBE_SPLIT + stream];
 #pragma unroll
-            for (int k = 0; k < 4; k++) pp_far_cut(s[k], fox, foy, foz, ulo, uhi, window, gx, gy, gz, ph);
+            for (int k = 0; k < 4; k++) pp_far_cut(s[k], fox, foy, foz, fu, ulo, uhi, window, gx, gy, gz, ph);
         }
     }
     if (window) ph += 1e-30f;

@@ -1,4 +1,4 @@
-// tpm_tiles.hip -- the direct kernel's work items and float positions.
+// tpm_tiles.hip -- the direct kernel's work items.
 //
 // The reference takes its sinks in buckets of a per-cell tree (<= 128,
 // tree.cpp:216-245) and compacts the active ones inside the kernel
@@ -58,12 +58,8 @@ __device__ __forceinline__ CellBox cell_box(const tpm_tile_args& a, int c) {
 }
 
 // One wave per cell: its number of tiles, ceil(active / ts) (zero outside [lo,
-// hi)), and where wanted (fx) the float offsets of its particles from its
-// centre, in raw units: rounded to 2^-25 of half a cell, and shared by the
-// tiles of 27 cells that stage them (three subtractions and three
-// conversions less per staged source).
-__global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a, float* __restrict__ fx,
-                                                         float* __restrict__ fy, float* __restrict__ fz) {
+// hi)).
+__global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
@@ -82,13 +78,6 @@ __global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a, float*
                     n += __popcll(__ballot(i + lane < e && a.rung[min(i + lane, e - 1)] >= B.min_rung));
         }
         if (lane == 0) a.cnt[a.boxes ? c : tile_rank(l, C)] = (n + a.ts - 1) / a.ts;
-        if (!fx) continue;
-        const uint32_t qx = x * B.w + B.w / 2, qy = y * B.w + B.w / 2, qz = z * B.w + B.w / 2;
-        for (int i = b + lane; i < e; i += 64) {
-            fx[i] = (float)(int)(a.x[i] - qx);
-            fy[i] = (float)(int)(a.y[i] - qy);
-            fz[i] = (float)(int)(a.z[i] - qz);
-        }
     }
 }
 
@@ -365,9 +354,9 @@ tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const
     return TPM_OK;
 }
 
-tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a, float* fx, float* fy, float* fz) {
+tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a) {
     if (a.ncell == 0) return TPM_OK;
-    tile_count_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a, fx, fy, fz);
+    tile_count_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a);
     TPM_HIPE(err, hipGetLastError());
     TPM_TRY(tpm_scan_i32(err, s, a.cnt, a.ncell, a.part, a.off));
     // as many waves as an average cell has chunks

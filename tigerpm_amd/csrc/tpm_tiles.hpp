@@ -33,6 +33,5 @@ struct tpm_tile_args {
 // The raw positions in the order of the tiles.
 tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const tpm_tile_args& a, uint32_t* x,
                                uint32_t* y, uint32_t* z);
-// Tiles of at most ts active sinks of one cell, in spatial order; with fx also
-// the float offset of every particle from its cell's centre (raw units).
-tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a, float* fx, float* fy, float* fz);
+// Tiles of at most ts active sinks of one cell, in spatial order.
+tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a);

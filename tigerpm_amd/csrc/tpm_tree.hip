@@ -896,13 +896,17 @@ __device__ __forceinline__ void walk_bucket(const WalkArgs& a, const tpm_tree_bu
                     const float lx = sh.box[k][0], hx = sh.box[k][1], ly = sh.box[k][2];
                     const float hy = sh.box[k][3], lz = sh.box[k][4], hz = sh.box[k][5];
                     // Sources at least the near radius from the block's box
-                    // take the law without softening (pp_far), on float
-                    // offsets, as in the direct kernel; the others, and all
-                    // of them where float differences could wrap (C < 5),
+                    // take the law without softening (pp_far), on int32
+                    // offsets from the box's centre rounded to float, as in
+                    // the direct kernel (pp_sum); the others, and all
+                    // of them where the box is wide or float differences
+                    // could wrap (C < 5),
                     // the general one (walk 4.64 -> 4.03 ms at 128^3).
                     const bool hb = HALF && k == K - 1;
                     const int S = hb ? 4 : 2, st = hb ? s4 : stream;  // source streams
-                    const float fs = B.far_s;
+                    const int mx = (int)(0.5f * (lx + hx)), my = (int)(0.5f * (ly + hy)), mz = (int)(0.5f * (lz + hz));
+                    const float near2 =
+                        0.5f * fmaxf(hx - lx, fmaxf(hy - ly, hz - lz)) > B.far_wide ? B.far_all2 : B.far_near2;
                     int m = 0, mf = 0;  // near, far sources
                     for (int i0 = 0; i0 < nbuf; i0 += 64) {
                         const int i = i0 + lane;
@@ -917,13 +921,14 @@ __device__ __forceinline__ void walk_bucket(const WalkArgs& a, const tpm_tree_bu
                             const float ez = fmaxf(fmaxf(lz - fz, fz - hz), 0.f);
                             const float d2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
                             keep = !B.cull || d2 < B.cull2s;
-                            close = !B.cull || d2 * (fs * fs) < B.far_near2;
+                            close = !B.cull || d2 < near2;
                         }
                         const unsigned long long mk = __ballot(keep && close), ml = __ballot(keep && !close);
                         if (keep && close) sh.cbuf[WALK_SBUF + 15 - m - (int)count_below(mk)] = sv;
                         if (keep && !close)
                             reinterpret_cast<float4*>(sh.cbuf)[mf + (int)count_below(ml)] =
-                                make_float4(fx * fs, fy * fs, fz * fs, __int_as_float(i));
+                                make_float4((float)(sv.x - mx), (float)(sv.y - my), (float)(sv.z - mz),
+                                            __int_as_float(i));
                         m += __popcll(mk);
                         mf += __popcll(ml);
                     }
@@ -935,9 +940,9 @@ __device__ __forceinline__ void walk_bucket(const WalkArgs& a, const tpm_tree_bu
                         if (lane < nblk - mf)
                             reinterpret_cast<float4*>(sh.cbuf)[mf + lane] = make_float4(1e15f, 1e15f, 1e15f, 0.f);
                         __syncthreads();
-                        const float fox = (float)ox[k] * fs, foy = (float)oy[k] * fs, foz = (float)oz[k] * fs;
-                        float ulo = B.far_ulo, uhi = B.far_uhi;
-                        asm volatile("" : "+v"(ulo), "+v"(uhi));
+                        const float fox = (float)(ox[k] - mx), foy = (float)(oy[k] - my), foz = (float)(oz[k] - mz);
+                        float ulo = B.far_ulo, uhi = B.far_uhi, fu = B.far_u;
+                        asm volatile("" : "+v"(ulo), "+v"(uhi), "+v"(fu));
                         float gx = 0.f, gy = 0.f, gz = 0.f, ph = 0.f;
                         unsigned long long window = 0ull;
 #pragma unroll 1
@@ -946,13 +951,14 @@ __device__ __forceinline__ void walk_bucket(const WalkArgs& a, const tpm_tree_bu
 #pragma unroll
                             for (int u = 0; u < 4; u++) v[u] = fbuf[j + u * S];
 #pragma unroll
-                            for (int u = 0; u < 4; u++) pp_far_cut(v[u], fox, foy, foz, ulo, uhi, window, gx, gy, gz, ph);
+                            for (int u = 0; u < 4; u++)
+                                pp_far_cut(v[u], fox, foy, foz, fu, ulo, uhi, window, gx, gy, gz, ph);
                         }
                         if (window) {
                             for (int j = st; j < nblk; j += S) {
                                 const float4 v = fbuf[j];
                                 const float dx = v.x - fox, dy = v.y - foy, dz = v.z - foz;
-                                const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                                const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) * fu;
                                 if (u >= ulo && u < uhi) {
                                     const int4 sv = sh.sbuf[__float_as_int(v.w)];
                                     if (pp_inside(B, ox[k] - sv.x, oy[k] - sv.y, oz[k] - sv.z))
