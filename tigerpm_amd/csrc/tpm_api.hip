@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "tpm_internal.hpp"
+#include "tpm_readback.hpp"
 
 tpm_status tpm_fft_release(tpm_ctx* ctx);
 
@@ -12,10 +13,11 @@ tpm_status tpm_fft_release(tpm_ctx* ctx);
 // caller's order).  Page-locked destinations of up to READBACK_KERNEL bytes
 // together are written by one kernel for all arrays: a copy call costs the
 // host about 10 us.  Eight arrays (29 B per particle) of 32^3 particles take
-// 30 us against 97, of 64^3 149 against 218, of 93^3 432 against 490; at 256^3
-// (487 MB) the copies' 56.5 GB/s beat the kernel's 55.3.  Larger reads and
-// pageable destinations take one copy per array, through the staging buffer
-// where there is a map.
+// 32 us against 99, of 64^3 151 against 220, of 93^3 434 against 495, of 128^3
+// (61 MB) 1110 against 1152, of 160^3 (119 MB) 2151 against 2173; at 200^3 (232
+// MB) the copies win by 1 % and at 256^3 by 2 %.  Larger reads and other
+// destinations (tpm_readback_direct) take one copy per array, through the
+// staging buffer where there is a map.
 constexpr int64_t READBACK_KERNEL = 64 << 20;
 struct ReadbackArgs {
     const void* src[11];
@@ -39,19 +41,28 @@ __global__ __launch_bounds__(256) static void readback_kernel(ReadbackArgs a) {
         readback_array<uint8_t>(a, k);
 }
 
-// The device address of [p, p + bytes) when it is page-locked host memory, else nullptr.
-static void* device_view(void* p, size_t bytes) {
-    hipPointerAttribute_t lo{}, hi{};
-    char* const last = static_cast<char*>(p) + bytes - 1;
-    if (hipPointerGetAttributes(&lo, p) != hipSuccess || hipPointerGetAttributes(&hi, last) != hipSuccess) {
+// What the runtime knows of a destination whose entries have so many bytes:
+// its allocation's base and size are asked for, since the ends of a range say
+// nothing of what lies between them.
+static tpm_readback_dst readback_dst(void* p, int bytes) {
+    tpm_readback_dst d{bytes, false, 0, 0, 0};
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        return d;
     }
-    if (lo.type != hipMemoryTypeHost || hi.type != hipMemoryTypeHost || !lo.devicePointer || !hi.devicePointer)
-        return nullptr;
-    if (static_cast<char*>(hi.devicePointer) - static_cast<char*>(lo.devicePointer) != (ptrdiff_t)(bytes - 1))
-        return nullptr;
-    return lo.devicePointer;
+    if (at.type != hipMemoryTypeHost || !at.devicePointer) return d;
+    if (hipMemGetAddressRange(&base, &size, at.devicePointer) != hipSuccess) {
+        (void)hipGetLastError();
+        return d;
+    }
+    d.host = true;
+    d.dev = reinterpret_cast<uintptr_t>(at.devicePointer);
+    d.base = reinterpret_cast<uintptr_t>(base);
+    d.size = size;
+    return d;
 }
 
 tpm_status tpm_readback(std::string& err, hipStream_t s, int64_t n, const tpm_copy* cp, int count,
@@ -63,14 +74,16 @@ tpm_status tpm_readback(std::string& err, hipStream_t s, int64_t n, const tpm_co
     int64_t each = 0;
     for (int k = 0; k < count; k++) each += cp[k].dst ? cp[k].bytes : 0;
     bool kernel = each * n <= READBACK_KERNEL;
+    tpm_readback_dst d[11];
     for (int k = 0; k < count && kernel; k++) {
         if (!cp[k].dst) continue;
+        d[used] = readback_dst(cp[k].dst, cp[k].bytes);
         a.src[used] = cp[k].src;
         a.bytes[used] = cp[k].bytes;
-        a.dst[used] = device_view(cp[k].dst, (size_t)cp[k].bytes * n);
-        kernel = a.dst[used] != nullptr;
+        a.dst[used] = reinterpret_cast<void*>(d[used].dev);
         used++;
     }
+    kernel = kernel && tpm_readback_direct(d, used, n);
     if (kernel) {
         if (used == 0) return TPM_OK;
         readback_kernel<<<dim3(std::min(grid_for(n, 256), 256u), (unsigned)used), 256, 0, s>>>(a);
