@@ -661,11 +661,16 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
 }
 
 // The kick alone (TPM_SKIP_PP): the epilogue of every active particle of the
-// cells in [lo, hi) from its mesh term, one wave per cell and one lane per
-// particle (through 16-sink tiles, with a quarter of the lanes, it took
-// 0.44 ms at 256^3).
+// cells in [lo, hi) from its mesh term, one lane per particle (through
+// 16-sink tiles, with a quarter of the lanes, it took 0.44 ms at 256^3).  One
+// wave per cell for its first KO_RUN particles; those beyond, of crowded
+// cells, KO_RUN at a time by further waves, one per KO_RUN particles of all:
+// wave v looks at the cell that holds particle v KO_RUN.  (10^5 particles in
+// one cell took one wave 314 us, now 10; 1024 instead of 2048 costs 256^3
+// uniform ones 8 us of 115.)
+#define KO_RUN 2048
 template <bool BATCH>
-__global__ __launch_bounds__(256) void kick_only_kernel(PPArgs a, int ncell, int nbox, int3 lo, int3 hi) {
+__global__ __launch_bounds__(256) void kick_only_kernel(PPArgs a, int ncell, int nrun, int nbox, int3 lo, int3 hi) {
     const int lane = (int)lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
@@ -673,9 +678,19 @@ __global__ __launch_bounds__(256) void kick_only_kernel(PPArgs a, int ncell, int
         a.counters ? a.counters + TPM_COUNTER_STRIDE * (blockIdx.x % TPM_COUNTER_SLOTS) : nullptr;
     const tpm_kick_out o{a.gx, a.gy, a.gz, a.pot, a.vx, a.vy, a.vz, a.rung, cnt};
     int nr = -1;
-    for (int c = wave; c < ncell; c += nwave) {
-        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
-        if (b == e) continue;
+    for (int u = wave; u < ncell + nrun; u += nwave) {
+        int c = u, b, e;
+        if (u < ncell) {
+            b = a.cell_begin[c];
+            e = min(a.cell_begin[c + 1], b + KO_RUN);
+        } else {
+            const int i0 = (u - ncell) * KO_RUN;
+            if (i0 >= a.cell_begin[ncell]) continue;
+            c = tpm_upper_index(ncell, i0, [&](int k) { return (int64_t)a.cell_begin[k]; });
+            b = max(i0, a.cell_begin[c] + KO_RUN);
+            e = min(i0 + KO_RUN, a.cell_begin[c + 1]);
+        }
+        if (b >= e) continue;
         int box = 0;
         if constexpr (BATCH) box = tpm_upper_index(nbox, c, [&](int k) { return (int64_t)a.boxes[k].cell0; });
         const tpm_box_dev B = tile_box<BATCH>(a, box);
@@ -964,9 +979,8 @@ static void pp_launch(int ts, bool persistent, unsigned grid, hipStream_t s, con
 
 }  // namespace
 
-// One wave per cell, 4 per workgroup, up to a grid that fills the chip many
-// times over.
-static unsigned cell_grid(int64_t ncell) { return (unsigned)std::min<int64_t>((ncell + 3) / 4, 65536); }
+// Waves, 4 per workgroup, up to a grid that fills the chip many times over.
+static unsigned wave_grid(int64_t waves) { return (unsigned)std::min<int64_t>((waves + 3) / 4, 65536); }
 
 void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_call, double t0, double scale) {
     b->C = p.chain_dim;
@@ -1157,7 +1171,8 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
         TPM_HIP(ctx, hipGetLastError());
     }
     if (ctx->n > 0 && (flags & TPM_SKIP_PP)) {
-        kick_only_kernel<false><<<cell_grid(ncell), 256, 0, s>>>(a, (int)ncell, 1, blo, bhi);
+        const int nrun = (int)((ctx->n + KO_RUN - 1) / KO_RUN);
+        kick_only_kernel<false><<<wave_grid(ncell + nrun), 256, 0, s>>>(a, (int)ncell, nrun, 1, blo, bhi);
         TPM_HIP(ctx, hipGetLastError());
     } else if (ctx->n > 0 && blocks > 0) {
         // the tiles of the active sinks (kick_pme: of every sink, so that its
@@ -1279,8 +1294,9 @@ tpm_status tpm_batch_pp(tpm_batch* bt, const tpm_batch_layout& L, unsigned flags
         a.mesh = bt->mesh_force;
     }
     if (flags & TPM_SKIP_PP) {
-        kick_only_kernel<true><<<cell_grid(L.ncell), 256, 0, bt->stream>>>(a, L.ncell, L.nbox, make_int3(0, 0, 0),
-                                                                            make_int3(0, 0, 0));
+        const int nrun = (int)((L.n_live + KO_RUN - 1) / KO_RUN);
+        kick_only_kernel<true><<<wave_grid((int64_t)L.ncell + nrun), 256, 0, bt->stream>>>(
+            a, L.ncell, nrun, L.nbox, make_int3(0, 0, 0), make_int3(0, 0, 0));
         TPM_HIP(bt, hipGetLastError());
         return TPM_OK;
     }

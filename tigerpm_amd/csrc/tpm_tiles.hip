@@ -15,34 +15,16 @@
 // Tiles of active sinks only: with an eighth of 256^3 particles active the
 // kernel has an eighth of the tiles (11.9 -> 4.7 ms).
 #include "tpm_tiles.hpp"
+#include "tpm_tile_order.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 namespace {
 
 __device__ __forceinline__ unsigned count_below(unsigned long long m) {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-
-// Tile order: cells are visited in z-major blocks of TILE_BLOCK^3 cells
-// (blocks z-major, cells z-major inside a block), so the tiles the PP kernel
-// runs close together in time share their 27-cell neighbourhoods: a block's
-// sources (10^3 cells at 512^3, ~2 MB) and its stretch of the potential mesh
-// fit one XCD's L2.  rank(c) is this order's position of cell c, a bijection
-// onto [0, C^3) (edge blocks are smaller).  Each tile is computed
-// independently, so the order changes no result.
-#define TILE_BLOCK 8
-// 32-bit arithmetic throughout (C^3 < 2^27): a wave does this for one cell.
-__device__ __forceinline__ int32_t tile_rank(uint32_t c, uint32_t C) {
-    const uint32_t q = c / C;
-    const int x = (int)(c - q * C), z = (int)(q / C), y = (int)(q - (uint32_t)z * C), Ci = (int)C;
-    const int bx = x / TILE_BLOCK, by = y / TILE_BLOCK, bz = z / TILE_BLOCK;
-    const int sy = min(TILE_BLOCK, Ci - by * TILE_BLOCK), sz = min(TILE_BLOCK, Ci - bz * TILE_BLOCK);
-    const int sx = min(TILE_BLOCK, Ci - bx * TILE_BLOCK);
-    const int before = bz * TILE_BLOCK * Ci * Ci + sz * by * TILE_BLOCK * Ci + sz * sy * bx * TILE_BLOCK;
-    const int local = ((z - bz * TILE_BLOCK) * sy + (y - by * TILE_BLOCK)) * sx + (x - bx * TILE_BLOCK);
-    return before + local;
 }
 
 // What a cell's wave needs of its box.
@@ -57,9 +39,41 @@ __device__ __forceinline__ CellBox cell_box(const tpm_tile_args& a, int c) {
     return CellBox{b, a.boxes[b].cell0, a.boxes[b].C, a.boxes[b].min_rung, a.boxes[b].n, a.boxes[b].cell_w};
 }
 
+// Counts the active particles of [i, e) from i on, in pieces that end at
+// multiples of 16, while at least COUNT_STEP particles are left and the count cannot
+// exceed most; i moves to the first particle not counted.  Four 16-byte loads
+// are in flight per lane (a cell of 10^5 particles: 28 us, 314 with one byte a lane).
+constexpr int COUNT_STEP = 4096;
+__device__ __forceinline__ int count_active(const int8_t* __restrict__ rung, int& i, int e, int most, int lane,
+                                            int min_rung) {
+    int n = 0;
+    while (true) {
+        const int i0 = i & ~15;
+        if (i0 + COUNT_STEP > e || COUNT_STEP > most - n) break;
+        int4 v[4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) v[p] = *reinterpret_cast<const int4*>(rung + i0 + 1024 * p + 16 * lane);
+        int mine = 0;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int w[4] = {v[p].x, v[p].y, v[p].z, v[p].w};
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int r = (int)(int8_t)(w[k / 4] >> (8 * (k % 4)));
+                mine += r >= min_rung && (p > 0 || 16 * lane + k >= i - i0) ? 1 : 0;
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o);
+        n += __builtin_amdgcn_readfirstlane(mine);
+        i = i0 + COUNT_STEP;
+    }
+    return n;
+}
+
 // One wave per cell: its number of tiles, ceil(active / ts) (zero outside [lo,
 // hi)).
-__global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a) {
+__global__ __launch_bounds__(256, 8) void tile_count_kernel(tpm_tile_args a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
@@ -73,9 +87,12 @@ __global__ __launch_bounds__(256) void tile_count_kernel(tpm_tile_args a) {
                         (int)z >= a.lo.z && (int)z < a.hi.z)) {
             if (a.all)
                 n = e - b;
-            else
-                for (int i = b; i < e; i += 64)
+            else {
+                int i = b;
+                n = count_active(a.rung, i, e, INT_MAX, lane, B.min_rung);
+                for (; i < e; i += 64)
                     n += __popcll(__ballot(i + lane < e && a.rung[min(i + lane, e - 1)] >= B.min_rung));
+            }
         }
         if (lane == 0) a.cnt[a.boxes ? c : tile_rank(l, C)] = (n + a.ts - 1) / a.ts;
     }
@@ -97,7 +114,12 @@ __global__ void order_positions_kernel(int64_t n, const uint32_t* __restrict__ o
 // wave: KD_CHUNK of them in chain-mesh order, whose Morton codes keep them
 // together, half as many in boxes below KD_SMALL particles, where the waves
 // are few and the splits of a chunk, one after the other, are the kernel's
-// time.  a.per_cell waves share a cell's chunks.  A
+// time.  a.per_cell waves share a cell's first KD_RUN a.per_cell chunks; the
+// chunks beyond, of cells far more crowded than the average, are found one by
+// one from the tile list by further waves (tile_slot_chunk), so that a halo's
+// cell is made by the whole chip: one cell of 10^5 particles among 64^3
+// uniform ones takes 0.10 ms (11^3 cells) and 0.13 ms (45^3), where its chunks
+// were the work of one wave or two 3.9 and 7.5 ms.  A
 // segment of len particles that makes m tiles is split m / 2 : m - m / 2, at
 // the position whose lower side has len (m / 2) / m particles (full tiles: ts
 // (m / 2)), found by
@@ -105,6 +127,8 @@ __global__ void order_positions_kernel(int64_t n, const uint32_t* __restrict__ o
 // split is exact and depends on nothing but the cell's particles.
 constexpr int KD_CHUNK = 256;
 constexpr int KD_SMALL = 1 << 19;
+constexpr int KD_RUN = 4;
+constexpr int KD_SLOTS = 8;  // slots of the tile list that a wave looks at
 constexpr int KD_STACK = 8;  // pending segments: one per level of at most log2(256 / 8), and the current one
 
 struct KdWave {
@@ -207,137 +231,199 @@ __device__ __forceinline__ uint32_t kd_split(KdWave& w, int lane, int s, int len
     return t;
 }
 
-__global__ __launch_bounds__(256) void tile_build_kernel(tpm_tile_args a) {
+// A cell whose tiles are made.
+struct KdCell {
+    int c, b, e, chunk, first_tile;
+    CellBox B;
+    uint32_t q[3];  // its centre - 2^31
+};
+__device__ __forceinline__ KdCell kd_cell(const tpm_tile_args& a, int c, int first_tile) {
+    KdCell x;
+    x.c = c;
+    x.b = a.cell_begin[c];
+    x.e = a.cell_begin[c + 1];
+    x.B = cell_box(a, c);
+    x.chunk = x.B.n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK;
+    x.first_tile = first_tile;
+    const uint32_t l = (uint32_t)(c - x.B.cell0), C = (uint32_t)x.B.C;
+    x.q[0] = (l % C) * x.B.w + x.B.w / 2 - 0x80000000u;
+    x.q[1] = ((l / C) % C) * x.B.w + x.B.w / 2 - 0x80000000u;
+    x.q[2] = (l / (C * C)) * x.B.w + x.B.w / 2 - 0x80000000u;
+    return x;
+}
+
+// Chunk k of a cell.  seen: active particles before particle i0 of the cell,
+// at most those before the chunk; both move on.
+__device__ __forceinline__ void kd_chunk(const tpm_tile_args& a, KdWave& w, int lane, const KdCell& x, int k, int& seen,
+                                         int& i0) {
+    const int ts = a.ts, e = x.e;
+    const int first = k * x.chunk;  // active particles before the chunk
+    int tile = x.first_tile + k * (x.chunk / ts);
+    const int out = x.b + first;  // its place in the order
+    if (a.all) {
+        seen = first;
+        i0 = out;
+    }
+    seen += count_active(a.rung, i0, e, first - seen, lane, x.B.min_rung);
+    int n = 0;
+    while (i0 < e && n < x.chunk) {
+        const int i = i0 + lane;
+        bool act = i < e && (a.all || a.rung[min(i, e - 1)] >= x.B.min_rung);
+        const unsigned long long m = __ballot(act);
+        const int rank = seen + (int)count_below(m) - first;
+        act = act && rank >= 0 && rank < x.chunk;
+        const unsigned long long mt = __ballot(act);
+        if (act) {
+            w.id[rank] = (uint32_t)i;
+            w.ord[rank] = (uint32_t)rank;
+            w.p[0][rank] = a.x[i] - x.q[0];
+            w.p[1][rank] = a.y[i] - x.q[1];
+            w.p[2][rank] = a.z[i] - x.q[2];
+        }
+        n += __popcll(mt);
+        if (n == x.chunk) break;  // the next chunk may begin inside this group
+        seen += __popcll(m);
+        i0 += 64;
+    }
+    if (n == 0) return;
+    kd_sync();
+    const int m0 = (n + ts - 1) / ts;
+    int sp = 1;
+    uint32_t lo[3], hi[3];
+    if (m0 > 1) {
+        // the chunk's box; from there on halves of it
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            uint32_t mn = ~0u, mx = 0u;
+            for (int k = lane; k < n; k += 64) {
+                const uint32_t v = w.p[d][k];
+                mn = min(mn, v);
+                mx = max(mx, v);
+            }
+            lo[d] = wave_umin(mn);
+            hi[d] = wave_umax(mx);
+        }
+    } else {
+        lo[0] = lo[1] = lo[2] = hi[0] = hi[1] = hi[2] = 0u;
+    }
+    if (lane == 0) {
+        w.stack[0][0] = 0;
+        w.stack[0][1] = n;
+        w.stack[0][2] = m0;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            w.stack[0][3 + d] = (int)lo[d];
+            w.stack[0][6 + d] = (int)hi[d];
+        }
+    }
+    kd_sync();
+    while (sp > 0) {
+        sp--;
+        const int s = __builtin_amdgcn_readfirstlane(w.stack[sp][0]);
+        const int len = __builtin_amdgcn_readfirstlane(w.stack[sp][1]);
+        const int m = __builtin_amdgcn_readfirstlane(w.stack[sp][2]);
+        if (m == 1) {
+            if (lane == 0 && a.tiles) a.tiles[tile] = make_int4(x.c, out + s, out + s + len, x.B.box);
+            tile++;
+            continue;
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = (uint32_t)__builtin_amdgcn_readfirstlane(w.stack[sp][3 + d]);
+            hi[d] = (uint32_t)__builtin_amdgcn_readfirstlane(w.stack[sp][6 + d]);
+        }
+        int axis = 0;
+        uint32_t span = hi[0] - lo[0], l0 = lo[0], h0 = hi[0];
+        if (hi[1] - lo[1] > span) {
+            axis = 1;
+            span = hi[1] - lo[1];
+            l0 = lo[1];
+            h0 = hi[1];
+        }
+        if (hi[2] - lo[2] > span) {
+            axis = 2;
+            l0 = lo[2];
+            h0 = hi[2];
+        }
+        const int m1 = m / 2, left = a.full ? ts * m1 : len * m1 / m;
+        const uint32_t t = len <= 64    ? kd_split<1>(w, lane, s, len, left, axis, l0, h0)
+                           : len <= 128 ? kd_split<2>(w, lane, s, len, left, axis, l0, h0)
+                                        : kd_split<KD_CHUNK / 64>(w, lane, s, len, left, axis, l0, h0);
+        kd_sync();
+        if (lane == 0) {
+            // the upper side waits below the lower one
+            int* up = w.stack[sp];
+            int* dn = w.stack[sp + 1];
+            up[0] = s + left;
+            up[1] = len - left;
+            up[2] = m - m1;
+            dn[0] = s;
+            dn[1] = left;
+            dn[2] = m1;
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                dn[3 + d] = (int)lo[d];
+                up[6 + d] = (int)hi[d];
+                up[3 + d] = (int)(d == axis ? t : lo[d]);
+                dn[6 + d] = (int)(d == axis ? t : hi[d]);
+            }
+        }
+        sp += 2;
+        kd_sync();
+    }
+    for (int i = lane; i < n; i += 64) a.order[out + i] = w.id[w.ord[i]];
+    kd_sync();
+}
+
+__global__ __launch_bounds__(256, 7) void tile_build_kernel(tpm_tile_args a) {
     __shared__ KdWave s_wave[4];
     const int lane = threadIdx.x & 63;
     KdWave& w = s_wave[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)];
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
-    const int ts = a.ts;
-    for (int u = wave; u < a.ncell * a.per_cell; u += nwave) {
-        const int c = u / a.per_cell, k0 = u - c * a.per_cell;
-        const int r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
-        const int ntile = a.cnt[r];
-        if (ntile == 0) continue;
-        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
-        const CellBox B = cell_box(a, c);
-        const int chunk = B.n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK;
-        const uint32_t l = (uint32_t)(c - B.cell0), C = (uint32_t)B.C;
-        const uint32_t q[3] = {(l % C) * B.w + B.w / 2 - 0x80000000u, ((l / C) % C) * B.w + B.w / 2 - 0x80000000u,
-                               (l / (C * C)) * B.w + B.w / 2 - 0x80000000u};
-        int seen = 0, i0 = b;  // active particles before particle i0 of the cell
-        for (int k = k0; k * (chunk / ts) < ntile; k += a.per_cell) {
-            const int first = k * chunk;  // active particles before the chunk
-            int tile = a.off[r] + k * (chunk / ts);
-            const int out = b + first;  // its place in the order
-            int n = 0;
-            while (i0 < e && n < chunk) {
-                const int i = i0 + lane;
-                bool act = i < e && (a.all || a.rung[min(i, e - 1)] >= B.min_rung);
-                const unsigned long long m = __ballot(act);
-                const int rank = seen + (int)count_below(m) - first;
-                act = act && rank >= 0 && rank < chunk;
-                const unsigned long long mt = __ballot(act);
-                if (act) {
-                    w.id[rank] = (uint32_t)i;
-                    w.ord[rank] = (uint32_t)rank;
-                    w.p[0][rank] = a.x[i] - q[0];
-                    w.p[1][rank] = a.y[i] - q[1];
-                    w.p[2][rank] = a.z[i] - q[2];
-                }
-                n += __popcll(mt);
-                if (n == chunk) break;  // the next chunk may begin inside this group
-                seen += __popcll(m);
-                i0 += 64;
+    const int run = KD_RUN * a.per_cell, cell_units = a.ncell * a.per_cell;
+    for (int u = wave; u < cell_units + a.slot_waves; u += nwave) {
+        const bool slots = u >= cell_units;
+        KdCell x{};
+        int k = 0, k1 = 0;                    // chunks of x: every per_cell-th of [k, k1)
+        int vr = 0, vc = 0, vk = -1;          // slots: chunk vk of cell vc, whose rank is vr, of each lane
+        unsigned long long found = 0ull;      // lanes with a chunk
+        if (!slots) {
+            const int c = u / a.per_cell;
+            const int r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
+            const int ntile = a.cnt[r];
+            if (ntile == 0) continue;
+            x = kd_cell(a, c, a.off[r]);
+            k = u - c * a.per_cell;
+            k1 = min(run, (ntile * a.ts + x.chunk - 1) / x.chunk);
+            if (k >= k1) continue;
+        } else {
+            // slots apart by the number of these waves, so that neighbouring
+            // chunks of a cell go to different ones
+            const int space = KD_CHUNK / 2 / a.ts;
+            const int64_t v = (u - cell_units) + (int64_t)lane * a.slot_waves;
+            if (lane < KD_SLOTS && v * space < a.off[a.ncell]) {
+                vr = tpm_upper_index(a.ncell, v * space, [&](int j) { return (int64_t)a.off[j]; });
+                vc = a.boxes ? vr : tile_cell((uint32_t)vr, (uint32_t)a.C);
+                const int64_t n = cell_box(a, vc).n;
+                vk = tile_slot_chunk(v, space, (n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK) / a.ts, a.off[vr], a.off[vr + 1]);
             }
-            if (n == 0) break;
-            kd_sync();
-            const int m0 = (n + ts - 1) / ts;
-            int sp = 1;
-            uint32_t lo[3], hi[3];
-            if (m0 > 1) {
-                // the chunk's box; from there on halves of it
-#pragma unroll
-                for (int d = 0; d < 3; d++) {
-                    uint32_t mn = ~0u, mx = 0u;
-                    for (int k = lane; k < n; k += 64) {
-                        const uint32_t v = w.p[d][k];
-                        mn = min(mn, v);
-                        mx = max(mx, v);
-                    }
-                    lo[d] = wave_umin(mn);
-                    hi[d] = wave_umax(mx);
-                }
-            } else {
-                lo[0] = lo[1] = lo[2] = hi[0] = hi[1] = hi[2] = 0u;
+            found = __ballot(vk >= run);
+            if (!found) continue;
+        }
+        int seen = 0, i0 = x.b;
+        for (;;) {
+            if (slots) {
+                const int l = __builtin_ctzll(found);
+                x = kd_cell(a, __builtin_amdgcn_readlane(vc, l), a.off[__builtin_amdgcn_readlane(vr, l)]);
+                k = __builtin_amdgcn_readlane(vk, l);
+                seen = 0;
+                i0 = x.b;
             }
-            if (lane == 0) {
-                w.stack[0][0] = 0;
-                w.stack[0][1] = n;
-                w.stack[0][2] = m0;
-#pragma unroll
-                for (int d = 0; d < 3; d++) {
-                    w.stack[0][3 + d] = (int)lo[d];
-                    w.stack[0][6 + d] = (int)hi[d];
-                }
-            }
-            kd_sync();
-            while (sp > 0) {
-                sp--;
-                const int s = __builtin_amdgcn_readfirstlane(w.stack[sp][0]);
-                const int len = __builtin_amdgcn_readfirstlane(w.stack[sp][1]);
-                const int m = __builtin_amdgcn_readfirstlane(w.stack[sp][2]);
-                if (m == 1) {
-                    if (lane == 0 && a.tiles) a.tiles[tile] = make_int4(c, out + s, out + s + len, B.box);
-                    tile++;
-                    continue;
-                }
-#pragma unroll
-                for (int d = 0; d < 3; d++) {
-                    lo[d] = (uint32_t)__builtin_amdgcn_readfirstlane(w.stack[sp][3 + d]);
-                    hi[d] = (uint32_t)__builtin_amdgcn_readfirstlane(w.stack[sp][6 + d]);
-                }
-                int axis = 0;
-                uint32_t span = hi[0] - lo[0], l0 = lo[0], h0 = hi[0];
-                if (hi[1] - lo[1] > span) {
-                    axis = 1;
-                    span = hi[1] - lo[1];
-                    l0 = lo[1];
-                    h0 = hi[1];
-                }
-                if (hi[2] - lo[2] > span) {
-                    axis = 2;
-                    l0 = lo[2];
-                    h0 = hi[2];
-                }
-                const int m1 = m / 2, left = a.full ? ts * m1 : len * m1 / m;
-                const uint32_t t = len <= 64    ? kd_split<1>(w, lane, s, len, left, axis, l0, h0)
-                                   : len <= 128 ? kd_split<2>(w, lane, s, len, left, axis, l0, h0)
-                                                : kd_split<KD_CHUNK / 64>(w, lane, s, len, left, axis, l0, h0);
-                kd_sync();
-                if (lane == 0) {
-                    // the upper side waits below the lower one
-                    int* up = w.stack[sp];
-                    int* dn = w.stack[sp + 1];
-                    up[0] = s + left;
-                    up[1] = len - left;
-                    up[2] = m - m1;
-                    dn[0] = s;
-                    dn[1] = left;
-                    dn[2] = m1;
-#pragma unroll
-                    for (int d = 0; d < 3; d++) {
-                        dn[3 + d] = (int)lo[d];
-                        up[6 + d] = (int)hi[d];
-                        up[3 + d] = (int)(d == axis ? t : lo[d]);
-                        dn[6 + d] = (int)(d == axis ? t : hi[d]);
-                    }
-                }
-                sp += 2;
-                kd_sync();
-            }
-            for (int i = lane; i < n; i += 64) a.order[out + i] = w.id[w.ord[i]];
-            kd_sync();
+            kd_chunk(a, w, lane, x, k, seen, i0);
+            found &= found - 1;
+            k += a.per_cell;
+            if (slots ? !found : k >= k1) break;
         }
     }
 }
@@ -361,7 +447,9 @@ tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a) {
     TPM_TRY(tpm_scan_i32(err, s, a.cnt, a.ncell, a.part, a.off));
     // as many waves as an average cell has chunks
     a.per_cell = (int)std::min<int64_t>(std::max<int64_t>(a.n_all / a.ncell / (KD_CHUNK / 2), 1), 32);
-    tile_build_kernel<<<wave_grid((int64_t)a.ncell * a.per_cell), 256, 0, s>>>(a);
+    const int64_t slots = (a.n_all / a.ts + a.ncell) / (KD_CHUNK / 2 / a.ts) + 1;
+    a.slot_waves = (int)((slots + KD_SLOTS - 1) / KD_SLOTS);
+    tile_build_kernel<<<wave_grid((int64_t)a.ncell * a.per_cell + a.slot_waves), 256, 0, s>>>(a);
     TPM_HIPE(err, hipGetLastError());
     return TPM_OK;
 }
