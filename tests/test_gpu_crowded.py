@@ -1,6 +1,6 @@
 """GPU: a chain cell far more crowded than the others.  Its tiles are made by many waves: forces against the oracle's
 FP64 sums with the bound of the other tile tests (2e-5 of the rms force), for every law and subset that makes tiles its own way, and
-the kick alone; and what a kick takes does not grow with the number of chunks that one wave would work through."""
+the kick alone, whose time does not depend on how the particles are spread over the cells."""
 import numpy as np
 import pytest
 
@@ -74,25 +74,17 @@ def test_kick_alone_of_a_crowded_cell(gpu_ctx, n_cell, lo, hi):
     assert np.array_equal(pot != 0, inside & (d["rung"] >= 1))
 
 
-def test_time_of_a_crowded_cell(gpu_ctx):
-    """10^5 particles in one cell against the same number over all 125: each tile of the first stages at most 5 times
-    the candidates, so the pair stage may take about 5 times as long, and the kick alone as long as the other."""
+def test_kick_alone_time_of_a_crowded_cell(gpu_ctx):
+    """10^5 particles in one cell against the same number over all 125: the kick alone does the same work for both."""
     C = 5
     p = T.baseline_params(512, 512, 3, n_total=10 ** 5)
     p.chain_dim = C
-    prev = gpu_ctx.get_tuning()
-    try:
-        gpu_ctx.set_params(p)
-        gpu_ctx.set_tuning()
-        ms = []
-        for n_cell in (10 ** 5, 0):
-            x, y, z = crowded(n_cell, 10 ** 5 - n_cell, C, 3)
-            gpu_ctx.upload(x, y, z)
-            gpu_ctx.chainmesh_create()
-            for flags in (0, T.TPM_SKIP_PP):
-                ms.append(min(gpu_ctx.kick(flags=flags | T.TPM_SKIP_PM | T.TPM_SKIP_KICK).ms_pp for _ in range(5)))
-    finally:
-        gpu_ctx.set_tuning(**prev)
-    print(ms)
-    assert ms[0] < 10 * ms[2]
-    assert ms[1] < 5 * ms[3]
+    gpu_ctx.set_params(p)
+    ms = []
+    for n_cell in (10 ** 5, 0):
+        x, y, z = crowded(n_cell, 10 ** 5 - n_cell, C, 3)
+        gpu_ctx.upload(x, y, z)
+        gpu_ctx.chainmesh_create()
+        flags = T.TPM_SKIP_PP | T.TPM_SKIP_PM | T.TPM_SKIP_KICK
+        ms.append(min(gpu_ctx.kick(flags=flags).ms_pp for _ in range(5)))
+    assert ms[0] < 5 * ms[1]
