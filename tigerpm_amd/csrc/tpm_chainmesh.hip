@@ -572,22 +572,58 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_apply_kernel(const int32_t*
 }
 
 // The whole scan in one block (few entries: one launch instead of three).
+// Every chunk's loads are in flight together; the sums are scanned within the
+// waves by shuffles, across them from LDS.  (8000 entries took 18 us with a
+// stretch of the input per thread, 9 so; three launches
+// 14; up to 2048 3.)
+// NC: chunks.
 constexpr int64_t SCAN_SMALL = 8 * SCAN_CHUNK;
+template <int NC>
 __global__ __launch_bounds__(SCAN_THREADS) void scan_small_kernel(const int32_t* __restrict__ in, int n,
                                                                   int32_t* __restrict__ out) {
-    __shared__ int32_t sh[SCAN_THREADS];
-    const int per = (n + SCAN_THREADS - 1) / SCAN_THREADS;
-    const int b0 = (int)threadIdx.x * per, b1 = min(b0 + per, n);
-    int32_t s = 0;
-    for (int k = b0; k < b1; k++) s += in[k];
-    int32_t tot;
-    int32_t run = block_exclusive_scan(s, sh, &tot);
-    for (int k = b0; k < b1; k++) {
-        const int32_t v = in[k];
-        out[k] = run;
-        run += v;
+    constexpr int NW = SCAN_THREADS / 64;
+    __shared__ int32_t sh[NC][NW];
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    int32_t v[NC][SCAN_ITEMS], incl[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        const int base = c * SCAN_CHUNK + (int)threadIdx.x * SCAN_ITEMS;
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; k++) v[c][k] = base + k < n ? in[base + k] : 0;
     }
-    if (threadIdx.x == 0) out[n] = tot;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        int32_t s = 0;
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; k++) s += v[c][k];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t a = __shfl_up(s, o);
+            s += lane >= o ? a : 0;
+        }
+        incl[c] = s;
+        if (lane == 63) sh[c][wave] = s;
+    }
+    __syncthreads();
+    int32_t before = 0;  // the chunks before, then in each the waves before
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        int32_t mine = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            mine += w < wave ? sh[c][w] : 0;
+            all += sh[c][w];
+        }
+        const int base = c * SCAN_CHUNK + (int)threadIdx.x * SCAN_ITEMS;
+        int32_t run = before + mine + incl[c];
+#pragma unroll
+        for (int k = SCAN_ITEMS - 1; k >= 0; k--) {
+            run -= v[c][k];
+            if (base + k < n) out[base + k] = run;
+        }
+        before += all;
+    }
+    if (threadIdx.x == 0) out[n] = before;
 }
 
 __global__ void bscatter_kernel(int64_t n, const uint32_t* __restrict__ key, const uint32_t* __restrict__ slot,
@@ -697,7 +733,12 @@ tpm_status tpm_scan_i32(std::string& err, hipStream_t s, const int32_t* in, int6
         return TPM_ERR_INVALID;
     }
     if (n <= SCAN_SMALL) {
-        scan_small_kernel<<<1, SCAN_THREADS, 0, s>>>(in, (int)n, out);
+        if (n <= SCAN_CHUNK)
+            scan_small_kernel<1><<<1, SCAN_THREADS, 0, s>>>(in, (int)n, out);
+        else if (n <= 4 * SCAN_CHUNK)
+            scan_small_kernel<4><<<1, SCAN_THREADS, 0, s>>>(in, (int)n, out);
+        else
+            scan_small_kernel<8><<<1, SCAN_THREADS, 0, s>>>(in, (int)n, out);
         TPM_HIPE(err, hipGetLastError());
         return TPM_OK;
     }
