@@ -23,13 +23,16 @@ namespace {
 // Onesweep radix sort with 9-bit digits: the 512^3 keys (26 bits) take three
 // passes instead of four (6.0 vs 6.5 ms for the whole chain mesh, same
 // permutation: the sort is stable, so the digit width cannot change it).
-// Onesweep at every size: rocPRIM's merge sort below 2^20 keys takes 16
-// launches for a 64^3 box, onesweep 6 (27 us of its 0.72 ms step).
+// Below 2^17 keys rocPRIM's merge sort (its own line is at 2^20) takes less time
+// than onesweep, whose passes are bound by launches and gaps there.  Chain mesh in a
+// stream of them, merge sort / onesweep, us: 16^3 keys 21 / 44, 32^3 41 / 48 (13
+// bits) and 53 / 74 (26 bits), 48^3 56 / 52 and 58 / 71, 64^3 90 / 57 and 90 / 78,
+// 100^3 142 / 107.
 using ChainSortConfig = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<512, 12>, rocprim::kernel_config<512, 12>, 9,
                                         rocprim::block_radix_rank_algorithm::match>,
-    0>;
+    1 << 17>;
 
 __global__ void key_kernel(int64_t n, const uint32_t* __restrict__ x, const uint32_t* __restrict__ y,
                            const uint32_t* __restrict__ z, int C, const uint32_t* __restrict__ bnd,
