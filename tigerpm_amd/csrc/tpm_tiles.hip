@@ -71,30 +71,61 @@ __device__ __forceinline__ int count_active(const int8_t* __restrict__ rung, int
     return n;
 }
 
-// One wave per cell: its number of tiles, ceil(active / ts) (zero outside [lo,
-// hi)).
+// The active particles of [b, e), counted by a wave.
+__device__ __forceinline__ int cell_active(const tpm_tile_args& a, int b, int e, int lane, int min_rung) {
+    int i = b, n = count_active(a.rung, i, e, INT_MAX, lane, min_rung);
+    for (; i < e; i += 64) n += __popcll(__ballot(i + lane < e && a.rung[min(i + lane, e - 1)] >= min_rung));
+    return n;
+}
+
+// Whether cell c's sinks are wanted (in [lo, hi)), and its place in the tile
+// list.
+__device__ __forceinline__ bool cell_wanted(const tpm_tile_args& a, int c, int* rank) {
+    *rank = c;
+    if (a.boxes) return true;
+    *rank = tile_rank((uint32_t)c, (uint32_t)a.C);
+    const int x = c % a.C, y = (c / a.C) % a.C, z = c / (a.C * a.C);
+    return x >= a.lo.x && x < a.hi.x && y >= a.lo.y && y < a.hi.y && z >= a.lo.z && z < a.hi.z;
+}
+
+// Number of tiles per cell, ceil(active / ts) (zero outside [lo, hi)): one
+// wave per cell, where cells have few particles one lane, and the wave for a
+// cell of more than 64.
+template <bool LANE>
 __global__ __launch_bounds__(256, 8) void tile_count_kernel(tpm_tile_args a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
-    for (int c = wave; c < a.ncell; c += nwave) {
-        const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
-        const CellBox B = cell_box(a, c);
-        const uint32_t l = (uint32_t)(c - B.cell0), C = (uint32_t)B.C;
-        const uint32_t x = l % C, y = (l / C) % C, z = l / (C * C);
-        int n = 0;
-        if (a.boxes || ((int)x >= a.lo.x && (int)x < a.hi.x && (int)y >= a.lo.y && (int)y < a.hi.y &&
-                        (int)z >= a.lo.z && (int)z < a.hi.z)) {
+    if constexpr (LANE) {
+        for (int64_t c0 = (int64_t)wave * 64; c0 < a.ncell; c0 += (int64_t)nwave * 64) {
+            const int c = (int)c0 + lane;
+            int b = 0, e = 0, r = 0, min_rung = 0, n = 0;
+            if (c < a.ncell) {
+                b = a.cell_begin[c];
+                e = cell_wanted(a, c, &r) ? a.cell_begin[c + 1] : b;
+                if (b < e) min_rung = cell_box(a, c).min_rung;
+            }
             if (a.all)
                 n = e - b;
-            else {
-                int i = b;
-                n = count_active(a.rung, i, e, INT_MAX, lane, B.min_rung);
-                for (; i < e; i += 64)
-                    n += __popcll(__ballot(i + lane < e && a.rung[min(i + lane, e - 1)] >= B.min_rung));
+            else if (e - b <= 64)
+                for (int i = b; i < e; i++) n += a.rung[i] >= min_rung ? 1 : 0;
+            for (unsigned long long m = __ballot(!a.all && e - b > 64); m; m &= m - 1) {
+                const int l = __builtin_ctzll(m);
+                const int k = cell_active(a, __builtin_amdgcn_readlane(b, l), __builtin_amdgcn_readlane(e, l), lane,
+                                          __builtin_amdgcn_readlane(min_rung, l));
+                if (lane == l) n = k;
             }
+            if (c < a.ncell) a.cnt[r] = (n + a.ts - 1) / a.ts;
         }
-        if (lane == 0) a.cnt[a.boxes ? c : tile_rank(l, C)] = (n + a.ts - 1) / a.ts;
+    } else {
+        for (int c = wave; c < a.ncell; c += nwave) {
+            int r, n = 0;
+            if (cell_wanted(a, c, &r)) {
+                const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
+                n = a.all ? e - b : cell_active(a, b, e, lane, cell_box(a, c).min_rung);
+            }
+            if (lane == 0) a.cnt[r] = (n + a.ts - 1) / a.ts;
+        }
     }
 }
 
@@ -231,6 +262,8 @@ __device__ __forceinline__ uint32_t kd_split(KdWave& w, int lane, int s, int len
     return t;
 }
 
+__device__ __forceinline__ int kd_chunk_size(int64_t n) { return n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK; }
+
 // A cell whose tiles are made.
 struct KdCell {
     int c, b, e, chunk, first_tile;
@@ -243,7 +276,7 @@ __device__ __forceinline__ KdCell kd_cell(const tpm_tile_args& a, int c, int fir
     x.b = a.cell_begin[c];
     x.e = a.cell_begin[c + 1];
     x.B = cell_box(a, c);
-    x.chunk = x.B.n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK;
+    x.chunk = kd_chunk_size(x.B.n);
     x.first_tile = first_tile;
     const uint32_t l = (uint32_t)(c - x.B.cell0), C = (uint32_t)x.B.C;
     x.q[0] = (l % C) * x.B.w + x.B.w / 2 - 0x80000000u;
@@ -381,49 +414,60 @@ __global__ __launch_bounds__(256, 7) void tile_build_kernel(tpm_tile_args a) {
     KdWave& w = s_wave[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)];
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6));
     const int nwave = (int)(((int64_t)gridDim.x * blockDim.x) >> 6);
-    const int run = KD_RUN * a.per_cell, cell_units = a.ncell * a.per_cell;
+    const int run = KD_RUN * a.per_cell;
+    const int cell_units = a.group ? (a.ncell + a.group - 1) / a.group : a.ncell * a.per_cell;
     for (int u = wave; u < cell_units + a.slot_waves; u += nwave) {
-        const bool slots = u >= cell_units;
-        KdCell x{};
-        int k = 0, k1 = 0;                    // chunks of x: every per_cell-th of [k, k1)
-        int vr = 0, vc = 0, vk = -1;          // slots: chunk vk of cell vc, whose rank is vr, of each lane
-        unsigned long long found = 0ull;      // lanes with a chunk
-        if (!slots) {
-            const int c = u / a.per_cell;
-            const int r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
-            const int ntile = a.cnt[r];
-            if (ntile == 0) continue;
-            x = kd_cell(a, c, a.off[r]);
-            k = u - c * a.per_cell;
-            k1 = min(run, (ntile * a.ts + x.chunk - 1) / x.chunk);
-            if (k >= k1) continue;
-        } else {
+        // Lanes with k < k1 have every per_cell-th chunk of [k, k1) of cell c,
+        // whose rank is r, for the wave to make.
+        int c = 0, r = 0, k = 0, k1 = 0;
+        if (u >= cell_units) {
             // slots apart by the number of these waves, so that neighbouring
             // chunks of a cell go to different ones
             const int space = KD_CHUNK / 2 / a.ts;
             const int64_t v = (u - cell_units) + (int64_t)lane * a.slot_waves;
             if (lane < KD_SLOTS && v * space < a.off[a.ncell]) {
-                vr = tpm_upper_index(a.ncell, v * space, [&](int j) { return (int64_t)a.off[j]; });
-                vc = a.boxes ? vr : tile_cell((uint32_t)vr, (uint32_t)a.C);
-                const int64_t n = cell_box(a, vc).n;
-                vk = tile_slot_chunk(v, space, (n < KD_SMALL ? KD_CHUNK / 2 : KD_CHUNK) / a.ts, a.off[vr], a.off[vr + 1]);
+                r = tpm_upper_index(a.ncell, v * space, [&](int j) { return (int64_t)a.off[j]; });
+                c = a.boxes ? r : tile_cell((uint32_t)r, (uint32_t)a.C);
+                k = tile_slot_chunk(v, space, kd_chunk_size(cell_box(a, c).n) / a.ts, a.off[r], a.off[r + 1]);
+                k1 = k >= run ? k + 1 : k;
             }
-            found = __ballot(vk >= run);
-            if (!found) continue;
+        } else if (a.group) {
+            // a lane makes the tile of its cell when there is one, of at most
+            // 64 particles; the wave makes the others
+            c = u * a.group + lane;
+            if (lane < a.group && c < a.ncell) {
+                r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
+                const int ntile = a.cnt[r];
+                if (ntile > 0) {
+                    const int b = a.cell_begin[c], e = a.cell_begin[c + 1];
+                    const CellBox B = cell_box(a, c);
+                    if (ntile == 1 && e - b <= 64) {
+                        int n = 0;
+                        for (int i = b; i < e; i++)
+                            if (a.all || a.rung[i] >= B.min_rung) a.order[b + n++] = (uint32_t)i;
+                        if (a.tiles) a.tiles[a.off[r]] = make_int4(c, b, b + n, B.box);
+                    } else {
+                        const int chunk = kd_chunk_size(B.n);
+                        k1 = min(run, (ntile * a.ts + chunk - 1) / chunk);
+                    }
+                }
+            }
+        } else {
+            c = u / a.per_cell;
+            r = a.boxes ? c : tile_rank((uint32_t)c, (uint32_t)a.C);
+            const int ntile = a.cnt[r];
+            if (ntile > 0 && lane == 0) {
+                const int chunk = kd_chunk_size(cell_box(a, c).n);
+                k = u - c * a.per_cell;
+                k1 = min(run, (ntile * a.ts + chunk - 1) / chunk);
+            }
         }
-        int seen = 0, i0 = x.b;
-        for (;;) {
-            if (slots) {
-                const int l = __builtin_ctzll(found);
-                x = kd_cell(a, __builtin_amdgcn_readlane(vc, l), a.off[__builtin_amdgcn_readlane(vr, l)]);
-                k = __builtin_amdgcn_readlane(vk, l);
-                seen = 0;
-                i0 = x.b;
-            }
-            kd_chunk(a, w, lane, x, k, seen, i0);
-            found &= found - 1;
-            k += a.per_cell;
-            if (slots ? !found : k >= k1) break;
+        for (unsigned long long m = __ballot(k < k1); m; m &= m - 1) {
+            const int l = __builtin_ctzll(m);
+            const KdCell x = kd_cell(a, __builtin_amdgcn_readlane(c, l), a.off[__builtin_amdgcn_readlane(r, l)]);
+            const int end = __builtin_amdgcn_readlane(k1, l);
+            int seen = 0, i0 = x.b;
+            for (int j = __builtin_amdgcn_readlane(k, l); j < end; j += a.per_cell) kd_chunk(a, w, lane, x, j, seen, i0);
         }
     }
 }
@@ -440,16 +484,34 @@ tpm_status tpm_order_positions(std::string& err, hipStream_t s, int64_t n, const
     return TPM_OK;
 }
 
+// Where the count takes a lane per cell: below COUNT_LANE_MEAN particles per
+// cell and from COUNT_LANE_CELLS cells on, when a wave per cell is more than
+// one round of the chip (4913 cells: 5 us a wave per cell, 7 a lane).
+// Where the build's waves take several cells each, of which a lane makes
+// those with one tile: where a wave per cell would be more than GROUP_WAVES
+// waves (the chip holds 7168 of them).
+// us, count + build, a wave per cell / so: 32^3 particles in 91^3 cells 426 / 27,
+// 180^3 737 / 78, 200^3 769 / 146, 256^3 1015 / 660, 320^3 1328 / 1025; 64^3 in 45^3
+// 108 / 27, 100^3 117 / 54, 160^3 188 / 152, 256^3 515 / 539.
+constexpr int COUNT_LANE_MEAN = 48, COUNT_LANE_CELLS = 8192, GROUP_WAVES = 16384;
+
 tpm_status tpm_tiles_make(std::string& err, hipStream_t s, tpm_tile_args a) {
     if (a.ncell == 0) return TPM_OK;
-    tile_count_kernel<<<wave_grid(a.ncell), 256, 0, s>>>(a);
+    if (a.n_all < COUNT_LANE_MEAN * (int64_t)a.ncell && a.ncell > COUNT_LANE_CELLS)
+        tile_count_kernel<true><<<wave_grid(((int64_t)a.ncell + 63) / 64), 256, 0, s>>>(a);
+    else
+        tile_count_kernel<false><<<wave_grid(a.ncell), 256, 0, s>>>(a);
     TPM_HIPE(err, hipGetLastError());
     TPM_TRY(tpm_scan_i32(err, s, a.cnt, a.ncell, a.part, a.off));
     // as many waves as an average cell has chunks
     a.per_cell = (int)std::min<int64_t>(std::max<int64_t>(a.n_all / a.ncell / (KD_CHUNK / 2), 1), 32);
-    const int64_t slots = (a.n_all / a.ts + a.ncell) / (KD_CHUNK / 2 / a.ts) + 1;
+    const int64_t slots = (a.n_all / a.ts + std::min<int64_t>(a.ncell, a.n_all)) / (KD_CHUNK / 2 / a.ts) + 1;
     a.slot_waves = (int)((slots + KD_SLOTS - 1) / KD_SLOTS);
-    tile_build_kernel<<<wave_grid((int64_t)a.ncell * a.per_cell + a.slot_waves), 256, 0, s>>>(a);
+    a.group = 0;
+    if (a.per_cell == 1)
+        for (a.group = 1; a.group < 64 && a.ncell / (2 * a.group) >= GROUP_WAVES;) a.group *= 2;
+    const int64_t units = a.group ? ((int64_t)a.ncell + a.group - 1) / a.group : (int64_t)a.ncell * a.per_cell;
+    tile_build_kernel<<<wave_grid(units + a.slot_waves), 256, 0, s>>>(a);
     TPM_HIPE(err, hipGetLastError());
     return TPM_OK;
 }

@@ -17,7 +17,8 @@ struct tpm_tile_args {
     int C, min_rung;
     int64_t n;        // particles of the box (boxes: in the table)
     int64_t n_all;    // particles of all cells
-    int per_cell;     // waves per cell of the build (this and the next set by tpm_tiles_make)
+    int per_cell;     // waves per cell of the build (this and the next two set by tpm_tiles_make)
+    int group;        // cells per wave of the build, of which a lane makes those with one tile; 0: per_cell waves
     int slot_waves;   // waves that find the chunks of crowded cells
     uint32_t cell_w;
     int3 lo, hi;
