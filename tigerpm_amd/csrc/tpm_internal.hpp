@@ -119,6 +119,7 @@ struct tpm_box_dev {
     float far_wrap;             // largest |offset| + box half width whose differences cannot wrap
     float far_g, far_ph;        // sums of pp_far -> box units
     uint32_t cell_w;            // 2^32 / C: cell k's centre is near k cell_w + cell_w / 2
+    float rcut2lo, rcut2hi;     // rcut2s, less and more than any rounding of a squared distance
     uint64_t rcut2i;            // a pair is inside the cutoff when its squared raw offset is below this
     // kick epilogue
     float GM, phi0, eta, t0, scale, hsoft;

@@ -210,8 +210,8 @@ __device__ __forceinline__ int tile_max(int v) {
 // compared with both ends of a window that covers its rounding; a flush that
 // met a pair inside the window (about one in 200 at 512^3) is followed by a
 // pass that adds those of them whose exact squared integer offset is inside;
-// a near pair that close to the cutoff is decided the same way
-// (pp_pair_exact).  The decision is then the same for every tile size and
+// near pairs that close to the cutoff are decided the same way (pp_pair_cut,
+// pp_pair_open).  The decision is then the same for every tile size and
 // order.
 template <int TS, bool PME, class Sync>
 __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, int cx, int cy, int cz, uint32_t px,
@@ -237,6 +237,9 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
     const float hx = (float)max(hix - mx, mx - lox), hy = (float)max(hiy - my, my - loy),
                 hz = (float)max(hiz - mz, mz - loz);
     const float near2 = fmaxf(hx, fmaxf(hy, hz)) > B.far_wide ? B.far_all2 : B.far_near2;
+    // every pair of a near source is closer than rcut: no pair to decide
+    const float reach = sqrtf(near2) + 2.f * sqrtf(fmaf(hx, hx, fmaf(hy, hy, hz * hz))) + 4096.f;
+    const bool near_in = __builtin_amdgcn_readfirstlane(reach * reach < B.rcut2s);
     ox -= mx;
     oy -= my;
     oz -= mz;
@@ -308,10 +311,13 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
             mf &= ~mn & valid;
             mn &= valid;
             const int j = j0 + lane;
-            if (__builtin_amdgcn_inverse_ballot_w64(mf))
-                fbuf[__builtin_amdgcn_mbcnt_hi((unsigned)(mf >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mf, nfar))] =
-                    make_float4(fx, fy, fz, __int_as_float(j));
-            nfar += __popcll(mf);
+            if (mf) {
+                if (__builtin_amdgcn_inverse_ballot_w64(mf))
+                    fbuf[__builtin_amdgcn_mbcnt_hi((unsigned)(mf >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)mf, nfar))] =
+                        make_float4(fx, fy, fz, __int_as_float(j));
+                nfar += __popcll(mf);
+            }
             if (mn) {
                 if (__builtin_amdgcn_inverse_ballot_w64(mn))
                     nbuf[__builtin_amdgcn_mbcnt_hi((unsigned)(mn >> 32),
@@ -374,12 +380,29 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
         }
         if (nnear > NEAR_AT || (!more && nnear > 0)) {
             lds_sync();
-            for (int q = stream; q < nnear; q += SPLIT) {
+            // Whole rounds of SPLIT sources first where no pair is to be
+            // decided (a compact box in a dense region); a loop whose lanes
+            // end at different rounds costs 5 % there, the window 9 % more.
+            // 64^3 particles in 300 halos: 1.55 ms with the general law
+            // alone, 1.67 with every near pair decided in the loop, 1.45 so.
+            int q0 = stream;
+            unsigned long long window = 0ull;
+            if (PME || near_in) {
+                const int full = nnear / SPLIT * SPLIT;
+                const int4* const nl = nbuf + stream;
+#pragma unroll 2
+                for (int q = 0; q < full; q += SPLIT) pp_pair<PME>(B, ox, oy, oz, nl[q], ngx, ngy, ngz, nph);
+                q0 += full;
+            }
+#pragma unroll 2
+            for (int q = q0; q < nnear; q += SPLIT) {
                 if constexpr (PME)
                     pp_pair<true>(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
                 else
-                    pp_pair_exact(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
+                    pp_pair_cut(B, ox, oy, oz, nbuf[q], window, ngx, ngy, ngz, nph);
             }
+            if (!PME && window)
+                for (int q = q0; q < nnear; q += SPLIT) pp_pair_open(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
             executed += (unsigned long long)nnear * (unsigned long long)nact;
             nnear = 0;
             lds_sync();
@@ -1015,6 +1038,12 @@ static void pp_launch(int ts, bool persistent, unsigned grid, hipStream_t s, con
 // Waves, 4 per workgroup, up to a grid that fills the chip many times over.
 static unsigned wave_grid(int64_t waves) { return (unsigned)std::min<int64_t>((waves + 3) / 4, 65536); }
 
+// The squared distance from which a source is a far one, raw units.
+static float far_near2(const tpm_params& p) {
+    const double nr = std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * 4294967296.0 + 2048.0;
+    return (float)(nr * nr * (1.0 + 1e-6));
+}
+
 void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_call, double t0, double scale) {
     b->C = p.chain_dim;
     b->M = p.mesh_dim;
@@ -1057,13 +1086,15 @@ void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_c
         const double two32 = 4294967296.0, l2e = 1.4426950408889634;
         const float fu = (float)(l2e / (4.0 * p.rs * p.rs) / (two32 * two32));
         b->far_u = fu;
-        const double nr = std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * two32 + 2048.0;
-        b->far_near2 = (float)(nr * nr * (1.0 + 1e-6));
-        const double cr = p.rcut * two32 + 2048.0;
+        // (below C = 5 a softened pair beyond rcut, h > rcut, has always counted)
+        const double cr = (b->cull ? p.rcut : std::max(p.rcut, p.hsoft)) * two32 + 2048.0;
         b->far_cull2 = (float)(cr * cr * (1.0 + 1e-6));
+        b->far_near2 = std::min(far_near2(p), b->far_cull2);
         const double wide = std::min(FAR_WIDE * p.rs, 0.5) * two32;
         b->far_wide = (float)wide;
-        b->far_all2 = std::max(b->far_near2, b->far_cull2);
+        b->far_all2 = b->far_cull2;
+        b->rcut2lo = b->rcut2s * (1.f - 1e-6f);
+        b->rcut2hi = b->rcut2s * (1.f + 1e-6f);
         const double rc = p.rcut * two32, uc = rc * rc * (double)fu;
         const double rel = 2.0 * std::sqrt(3.0) * std::exp2(-23.0) * (rc + wide) / rc + std::exp2(-21.0);
         b->far_ulo = (float)(uc * (1.0 - rel));
@@ -1159,6 +1190,7 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
     if (pme) {
         // kick_pme: every pair of the 27 cells counts, and phi starts at 0
         a.box0.cull = 0;
+        a.box0.far_near2 = far_near2(ctx->p);
         a.box0.far_all2 = FLT_MAX;
         a.box0.phi0 = 0.f;
     }

@@ -122,22 +122,40 @@ __device__ __forceinline__ bool pp_inside(const tpm_box_dev& a, int ix, int iy, 
     return (uint64_t)(x * x) + (uint64_t)(y * y) + (uint64_t)(z * z) < a.rcut2i;
 }
 
-// pp_pair with the cutoff decided on the integer offset where the rounding
-// of r2 (four of 2^-24, and rcut2s's own) leaves it open.
-__device__ __forceinline__ void pp_pair_exact(const tpm_box_dev& a, int ox, int oy, int oz, int4 s, float& gx,
-                                              float& gy, float& gz, float& ph) {
-    const int ix = (int)((unsigned)ox - (unsigned)s.x), iy = (int)((unsigned)oy - (unsigned)s.y),
-              iz = (int)((unsigned)oz - (unsigned)s.z);
-    const float fx = (float)ix, fy = (float)iy, fz = (float)iz;
-    const float r2 = fmaf(fx, fx, fmaf(fy, fy, fz * fz));
-    float cut2s = a.rcut2s;
-    if (fabsf(r2 - cut2s) < cut2s * 1e-6f) cut2s = pp_inside(a, ix, iy, iz) ? 2.f * cut2s : 0.f;
+// pp_pair with a window round the cutoff that covers the rounding of r2 (four
+// of 2^-24, and rcut2s's own): pairs below it are inside, at or above its upper
+// end outside, and where any lane's lies between (added as if outside) its bit in window is
+// set; pp_pair_open then adds what those whose exact squared integer offset is inside
+// lack.  (Deciding each pair within the loop costs 8 % where all sources are near.)
+__device__ __forceinline__ void pp_pair_cut(const tpm_box_dev& a, int ox, int oy, int oz, int4 s,
+                                            unsigned long long& window, float& gx, float& gy, float& gz, float& ph) {
     float dx, dy, dz, rinv3, rinv1;
-    pp_law<false>(a, ox, oy, oz, s, cut2s, dx, dy, dz, rinv3, rinv1);
+    pp_law<false>(a, ox, oy, oz, s, a.rcut2lo, dx, dy, dz, rinv3, rinv1);
+    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    window |= __ballot(r2 < a.rcut2hi) & ~__ballot(r2 < a.rcut2lo);
     gx = fmaf(-dx, rinv3, gx);
     gy = fmaf(-dy, rinv3, gy);
     gz = fmaf(-dz, rinv3, gz);
     ph -= rinv1;
+}
+__device__ __forceinline__ void pp_pair_open(const tpm_box_dev& a, int ox, int oy, int oz, int4 s, float& gx,
+                                             float& gy, float& gz, float& ph) {
+    const int ix = (int)((unsigned)ox - (unsigned)s.x), iy = (int)((unsigned)oy - (unsigned)s.y),
+              iz = (int)((unsigned)oz - (unsigned)s.z);
+    const float fx = (float)ix, fy = (float)iy, fz = (float)iz;
+    const float r2 = fmaf(fx, fx, fmaf(fy, fy, fz * fz));
+    if (r2 < a.rcut2lo || r2 >= a.rcut2hi || !pp_inside(a, ix, iy, iz)) return;
+    // as inside, less as outside
+#pragma unroll 1
+    for (int k = 0; k < 2; k++) {
+        float dx, dy, dz, rinv3, rinv1;
+        pp_law<false>(a, ox, oy, oz, s, k ? 0.f : 2.f * a.rcut2hi, dx, dy, dz, rinv3, rinv1);
+        const float w = k ? 1.f : -1.f;
+        gx = fmaf(w * dx, rinv3, gx);
+        gy = fmaf(w * dy, rinv3, gy);
+        gz = fmaf(w * dz, rinv3, gz);
+        ph = fmaf(w, rinv1, ph);
+    }
 }
 
 // The same law for a pair at least FAR_X0 * 2 rs and h apart: no softening,
