@@ -15,9 +15,11 @@ tpm_status tpm_fft_release(tpm_ctx* ctx);
 // host about 10 us.  Eight arrays (29 B per particle) of 32^3 particles take
 // 32 us against 99, of 64^3 151 against 220, of 93^3 434 against 495, of 128^3
 // (61 MB) 1110 against 1152, of 160^3 (119 MB) 2151 against 2173; at 200^3 (232
-// MB) the copies win by 1 % and at 256^3 by 2 %.  Larger reads and other
-// destinations (tpm_readback_direct) take one copy per array, through the
-// staging buffer where there is a map.
+// MB) the copies win by 1 % and at 256^3 by 2 %.  A single array without a map
+// is one copy call (32^3 forces' x 11.5 us, by the kernel 14.6; 128^3 156 against
+// 166; two arrays 23 against 17 and 313 against 315; one with a map 24 against 15).
+// Larger reads and other destinations (tpm_readback_direct) take one copy per
+// array, through the staging buffer where there is a map.
 constexpr int64_t READBACK_KERNEL = 64 << 20;
 struct ReadbackArgs {
     const void* src[11];
@@ -72,8 +74,12 @@ tpm_status tpm_readback(std::string& err, hipStream_t s, int64_t n, const tpm_co
     a.n = n;
     int used = 0;
     int64_t each = 0;
-    for (int k = 0; k < count; k++) each += cp[k].dst ? cp[k].bytes : 0;
-    bool kernel = each * n <= READBACK_KERNEL;
+    int wanted = 0;
+    for (int k = 0; k < count; k++) {
+        each += cp[k].dst ? cp[k].bytes : 0;
+        wanted += cp[k].dst ? 1 : 0;
+    }
+    bool kernel = each * n <= READBACK_KERNEL && (map || wanted > 1);
     tpm_readback_dst d[11];
     for (int k = 0; k < count && kernel; k++) {
         if (!cp[k].dst) continue;
