@@ -33,7 +33,6 @@
 #include "tpm_pp_device.hpp"
 #include "tpm_tiles.hpp"
 
-#include <cfloat>
 #include <climits>
 
 // Staged sources of a wave: far ones (float offsets) and near ones (int32
@@ -213,7 +212,7 @@ __device__ __forceinline__ int tile_max(int v) {
 // near pairs that close to the cutoff are decided the same way (pp_pair_cut,
 // pp_pair_open).  The decision is then the same for every tile size and
 // order.
-template <int TS, bool PME, class Sync>
+template <int TS, class Sync>
 __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, int cx, int cy, int cz, uint32_t px,
                                        uint32_t py, uint32_t pz, uint32_t rx, uint32_t ry, uint32_t rz, bool inbox,
                                        int nact, float4* __restrict__ fbuf, int4* __restrict__ nbuf, Sync lds_sync,
@@ -257,21 +256,19 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
         const int c2 = B.cell0 + (jz * C + jy) * C + jx;
         rb = a.cell_begin[c2];
         re = a.cell_begin[c2 + 1];
-        if constexpr (!PME) {
-            // A cell out of reach of the box is left out as a whole.  Its
-            // centre's offset ex, taken as the nearest image, puts a particle
-            // of it at least |ex| - half a cell - the box's half width away on
-            // that axis; a cell's planes are within C of k cell_w, 512 covers that.
-            // (Cells of rcut keep nearly all 27.  Staging every candidate of
-            // coarser ones cost more than the far law saved: chain mesh and kick
-            // of 64^3 at C = 5 1.81 ms, now 1.11, 128^3 at C = 11 7.5, now 3.7.)
-            const uint32_t w = B.cell_w;
-            const float hw = (float)(w / 2) + 512.f;
-            const float ex = fmaxf(fabsf((float)(int)((uint32_t)jx * w + w / 2 - qx)) - hw - hx, 0.f);
-            const float ey = fmaxf(fabsf((float)(int)((uint32_t)jy * w + w / 2 - qy)) - hw - hy, 0.f);
-            const float ez = fmaxf(fabsf((float)(int)((uint32_t)jz * w + w / 2 - qz)) - hw - hz, 0.f);
-            if (fmaf(ex, ex, fmaf(ey, ey, ez * ez)) >= B.far_cull2) re = rb;
-        }
+        // A cell out of reach of the box is left out as a whole.  Its
+        // centre's offset ex, taken as the nearest image, puts a particle
+        // of it at least |ex| - half a cell - the box's half width away on
+        // that axis; a cell's planes are within C of k cell_w, 512 covers that.
+        // (Cells of rcut keep nearly all 27.  Staging every candidate of
+        // coarser ones cost more than the far law saved: chain mesh and kick
+        // of 64^3 at C = 5 1.81 ms, now 1.11, 128^3 at C = 11 7.5, now 3.7.)
+        const uint32_t w = B.cell_w;
+        const float hw = (float)(w / 2) + 512.f;
+        const float ex = fmaxf(fabsf((float)(int)((uint32_t)jx * w + w / 2 - qx)) - hw - hx, 0.f);
+        const float ey = fmaxf(fabsf((float)(int)((uint32_t)jy * w + w / 2 - qy)) - hw - hy, 0.f);
+        const float ez = fmaxf(fabsf((float)(int)((uint32_t)jz * w + w / 2 - qz)) - hw - hz, 0.f);
+        if (fmaf(ex, ex, fmaf(ey, ey, ez * ez)) >= B.far_cull2) re = rb;
     }
     const uint32_t lane4 = 4u * (uint32_t)lane;
     gx = gy = gz = ph = 0.f;
@@ -302,7 +299,7 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
                         ez = fmaxf(fabsf(fz) - hz, 0.f);
             const float d2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
             unsigned long long mn = __ballot(d2 < near2), mf;
-            mf = PME ? ~0ull : __ballot(d2 < B.far_cull2);
+            mf = __ballot(d2 < B.far_cull2);
             if (!cull)
                 // a difference of float offsets does not wrap round the
                 // box as the int32 one does: sources for which it would
@@ -346,16 +343,10 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
                 for (int k = 0; k < 4; k++) s[k] = fbuf[q + k * SPLIT + stream];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    if constexpr (PME) {
-                        const float dx = s[k].x - fox, dy = s[k].y - foy, dz = s[k].z - foz;
-                        const float u = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) * fu;
-                        pp_far(dx, dy, dz, u, __builtin_amdgcn_exp2f(-u), gx, gy, gz, ph);
-                    } else {
-                        pp_far_cut(s[k], fox, foy, foz, fu, ulo, uhi, window, gx, gy, gz, ph);
-                    }
+                    pp_far_cut(s[k], fox, foy, foz, fu, ulo, uhi, window, gx, gy, gz, ph);
                 }
             }
-            if (!PME && window) {
+            if (window) {
                 for (int q = 0; q < nblk; q += SPLIT) {
                     const float4 s = fbuf[q + stream];
                     const float dx = s.x - fox, dy = s.y - foy, dz = s.z - foz;
@@ -387,21 +378,18 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
             // alone, 1.67 with every near pair decided in the loop, 1.45 so.
             int q0 = stream;
             unsigned long long window = 0ull;
-            if (PME || near_in) {
+            if (near_in) {
                 const int full = nnear / SPLIT * SPLIT;
                 const int4* const nl = nbuf + stream;
 #pragma unroll 2
-                for (int q = 0; q < full; q += SPLIT) pp_pair<PME>(B, ox, oy, oz, nl[q], ngx, ngy, ngz, nph);
+                for (int q = 0; q < full; q += SPLIT) pp_pair<false>(B, ox, oy, oz, nl[q], ngx, ngy, ngz, nph);
                 q0 += full;
             }
 #pragma unroll 2
             for (int q = q0; q < nnear; q += SPLIT) {
-                if constexpr (PME)
-                    pp_pair<true>(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
-                else
-                    pp_pair_cut(B, ox, oy, oz, nbuf[q], window, ngx, ngy, ngz, nph);
+                pp_pair_cut(B, ox, oy, oz, nbuf[q], window, ngx, ngy, ngz, nph);
             }
-            if (!PME && window)
+            if (window)
                 for (int q = q0; q < nnear; q += SPLIT) pp_pair_open(B, ox, oy, oz, nbuf[q], ngx, ngy, ngz, nph);
             executed += (unsigned long long)nnear * (unsigned long long)nact;
             nnear = 0;
@@ -414,6 +402,63 @@ __device__ __forceinline__ void pp_sum(const PPArgs& a, const tpm_box_dev& B, in
     gy = fmaf(ngy, 0x1p64f, gy * B.far_g);
     gz = fmaf(ngz, 0x1p64f, gz * B.far_g);
     ph = fmaf(nph, 0x1p32f, -ph * B.far_ph);
+}
+
+// kick_pme's sums of one tile: every particle of the 27 cells by the general
+// law, exact integer differences, in the cells' order.  (The far law is three times
+// nearer to the FP64 sums here, 1.0e-5 of the z force's rms instead of 3.0e-5 at
+// 60^3 with displacements of 0.3 cells, and takes 12.6 instead of 15.2 ms at 60^3.
+// But with no cutoff a sink's sum is a small difference of large parts, whose rounding
+// depends on each step of the sum: the forces moved by up to 2.6e-5, more than results may.)
+template <int TS, class Sync>
+__device__ __forceinline__ void pp_sum_pme(const PPArgs& a, const tpm_box_dev& B, int cx, int cy, int cz, int ox,
+                                           int oy, int oz, uint32_t rx, uint32_t ry, uint32_t rz, int nact,
+                                           int4* __restrict__ sbuf, Sync lds_sync, float& gx, float& gy, float& gz,
+                                           float& ph, unsigned long long& executed) {
+    constexpr int SPLIT = 64 / TS;
+    constexpr int FLUSH_AT = 128;
+    static_assert(FLUSH_AT + 64 + 2 * SPLIT <= FAR_CAP + NEAR_CAP, "room for the source read ahead");
+    const int lane = (int)lane_id(), stream = lane / TS;
+    const int C = B.C;
+    int nbuf = 0;
+    gx = gy = gz = ph = 0.f;
+    auto flush = [&]() {
+        // whole rounds of SPLIT sources, the next one read ahead, then the
+        // streams that still have one (no padding source: the law has no cutoff)
+        const int full = nbuf / SPLIT * SPLIT;
+        lds_sync();
+        int4 s = sbuf[stream];
+#pragma unroll 2
+        for (int q = 0; q < full; q += SPLIT) {
+            const int4 sn = sbuf[q + SPLIT + stream];
+            pp_pair<true>(B, ox, oy, oz, s, gx, gy, gz, ph);
+            s = sn;
+        }
+        if (full + stream < nbuf) pp_pair<true>(B, ox, oy, oz, s, gx, gy, gz, ph);
+        executed += (unsigned long long)nbuf * (unsigned long long)nact;
+        nbuf = 0;
+        lds_sync();
+    };
+    for (int nb = 0; nb < 27; nb++) {
+        int jx = cx + nb % 3 - 1, jy = cy + (nb / 3) % 3 - 1, jz = cz + nb / 9 - 1;
+        jx += jx < 0 ? C : (jx >= C ? -C : 0);
+        jy += jy < 0 ? C : (jy >= C ? -C : 0);
+        jz += jz < 0 ? C : (jz >= C ? -C : 0);
+        const int c2 = B.cell0 + (jz * C + jy) * C + jx;
+        const int sb = a.cell_begin[c2], se = a.cell_begin[c2 + 1];
+        for (int j0 = sb; j0 < se; j0 += 64) {
+            const int j = j0 + lane;
+            if (j < se)
+                sbuf[nbuf + lane] = make_int4((int)(a.x[j] - rx), (int)(a.y[j] - ry), (int)(a.z[j] - rz), j);
+            nbuf += min(64, se - j0);
+            if (nbuf > FLUSH_AT) flush();
+        }
+    }
+    if (nbuf > 0) flush();
+    gx *= 0x1p64f;
+    gy *= 0x1p64f;
+    gz *= 0x1p64f;
+    ph *= 0x1p32f;
 }
 
 // The same sums with per-sink source lists (16-sink tiles, culling on).
@@ -638,11 +683,12 @@ __global__ __launch_bounds__(64 * WPG, PERSIST ? 1 : (LISTS ? 7 : 8)) void pp_ki
                                      active, sbuf, (uint8_t*)(sbuf + LSBUF + 16), (float4*)(sbuf + LSBUF), lds_sync,
                                      gx, gy, gz, ph, executed);
                 }
-                if (!lists)
-                    // (kick_pme's sums do not depend on which other particles
-                    // are active, and stay so: its box holds all of the tile)
-                    pp_sum<TS, PME>(a, B, cx, cy, cz, px, py, pz, rx, ry, rz, PME ? valid : active, nact, (float4*)sbuf,
-                                    sbuf + FAR_CAP, lds_sync, gx, gy, gz, ph, executed);
+                if constexpr (PME)
+                    pp_sum_pme<TS>(a, B, cx, cy, cz, (int)(px - rx), (int)(py - ry), (int)(pz - rz), rx, ry, rz, nact,
+                                   sbuf, lds_sync, gx, gy, gz, ph, executed);
+                else if (!lists)
+                    pp_sum<TS>(a, B, cx, cy, cz, px, py, pz, rx, ry, rz, active, nact, (float4*)sbuf,
+                               sbuf + FAR_CAP, lds_sync, gx, gy, gz, ph, executed);
                 // sum the source streams
 #pragma unroll
                 for (int o = TS; o < 64; o <<= 1) {
@@ -1038,12 +1084,6 @@ static void pp_launch(int ts, bool persistent, unsigned grid, hipStream_t s, con
 // Waves, 4 per workgroup, up to a grid that fills the chip many times over.
 static unsigned wave_grid(int64_t waves) { return (unsigned)std::min<int64_t>((waves + 3) / 4, 65536); }
 
-// The squared distance from which a source is a far one, raw units.
-static float far_near2(const tpm_params& p) {
-    const double nr = std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * 4294967296.0 + 2048.0;
-    return (float)(nr * nr * (1.0 + 1e-6));
-}
-
 void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_call, double t0, double scale) {
     b->C = p.chain_dim;
     b->M = p.mesh_dim;
@@ -1089,7 +1129,8 @@ void tpm_box_fill(tpm_box_dev* b, const tpm_params& p, int min_rung, int first_c
         // (below C = 5 a softened pair beyond rcut, h > rcut, has always counted)
         const double cr = (b->cull ? p.rcut : std::max(p.rcut, p.hsoft)) * two32 + 2048.0;
         b->far_cull2 = (float)(cr * cr * (1.0 + 1e-6));
-        b->far_near2 = std::min(far_near2(p), b->far_cull2);
+        const double nr = std::max(FAR_X0 * 2.0 * p.rs, p.hsoft) * two32 + 2048.0;
+        b->far_near2 = std::min((float)(nr * nr * (1.0 + 1e-6)), b->far_cull2);
         const double wide = std::min(FAR_WIDE * p.rs, 0.5) * two32;
         b->far_wide = (float)wide;
         b->far_all2 = b->far_cull2;
@@ -1190,8 +1231,6 @@ tpm_status tpm_pp_kick(tpm_ctx* ctx, int min_rung, double scale, double t0, int 
     if (pme) {
         // kick_pme: every pair of the 27 cells counts, and phi starts at 0
         a.box0.cull = 0;
-        a.box0.far_near2 = far_near2(ctx->p);
-        a.box0.far_all2 = FLT_MAX;
         a.box0.phi0 = 0.f;
     }
     a.flags = flags & (TPM_SKIP_PP | TPM_SKIP_PM | TPM_SKIP_KICK);
