@@ -401,7 +401,7 @@ def main():
     ap.add_argument("--pp-newton", type=int, default=-1,
                     help="each pair evaluated once, both ends (0, 1; -1: default)")
     ap.add_argument("--fft", type=int, default=0,
-                    help="mesh FFTs: 0 = LDS-tiled transforms where there is one for the size, 1 = rocFFT")
+                    help="mesh FFTs: 0 = LDS-tiled transform for power-of-two meshes, 1 = rocFFT")
     ap.add_argument("--probe-copy", action="store_true",
                     help="also run one plain 1 GiB device copy (reference kernel for HBM byte counters)")
     args = ap.parse_args()

@@ -1,7 +1,6 @@
-"""GPU: the mesh FFTs of sizes with a prime factor between 19 and 101, which go
-through the general LDS kernels: the smallest and the largest size and prime,
-one and two large primes, every small radix beside them, odd and even, and
-partial tiles of rows (8 complex rows, 16 real ones per workgroup).  Against
+"""GPU: the mesh FFTs of sizes with a prime factor between 19 and 101, which are
+rocFFT's, as every size that is no power of two: small and large sizes and primes,
+one and two large primes, every small radix beside them, odd and even.  Against
 numpy's FP64 transforms, with the tolerance of the other FFT tests
 (relative rms 2e-6), and bit for bit with itself."""
 import numpy as np

@@ -1,6 +1,6 @@
-"""Downloads into page-locked buffers (one kernel for all arrays) equal those into ordinary ones (a copy each): every
-subset of arrays that is asked for, unaligned destinations, a destination that is only partly page-locked memory's
-neighbour, the reference's order, and boxes on both sides of the size where the copies take over."""
+"""Downloads into page-locked buffers (one kernel for all arrays) equal those into ordinary ones (a copy each): several
+subsets of arrays, unaligned destinations, ordinary ones beside page-locked ones in one call, the reference's order,
+and boxes on both sides of the size where the copies take over."""
 import ctypes
 
 import numpy as np

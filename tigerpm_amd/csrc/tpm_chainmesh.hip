@@ -10,7 +10,7 @@
 // keys.  Cell ranges equal the reference partition's; the in-cell order is
 // deterministic (sub-cell, then previous order) so CPU and GPU agree bit for
 // bit.  The PP kernel's sink tiles are
-// made from the cells by every kick (tpm_pp.hip).
+// made from the cells by every kick (tpm_tiles.hip).
 #include <cstring>
 
 #include <rocprim/device/device_radix_sort.hpp>

@@ -178,7 +178,7 @@ struct tpm_ctx {
     bool chain_valid = false;
     int chain_C = 0;
     int tile = 16;        // sinks per PP tile: 16, 32 or 64 (tuning)
-    int chain_tile = 0;   // tile size the current tile list was built with
+    int chain_tile = 0;   // tile size at the last chain-mesh build; a kick after a change of it is refused
     int deposit_block = 0;  // chain cells per deposit block edge; 0 auto, -1 per-particle atomics
     int pp_waves = TPM_PP_WAVES_DEFAULT;  // PP tiles per workgroup (1 or 4)
     int pp_lists = TPM_PP_LISTS_DEFAULT;  // per-sink source lists (16-sink tiles)
@@ -605,8 +605,6 @@ struct tpm_copy {
 // nullptr; staging: n words on the device, needed with a map.
 tpm_status tpm_readback(std::string& err, hipStream_t s, int64_t n, const tpm_copy* cp, int count,
                         const uint32_t* map, uint32_t* staging);
-// Exclusive scan (tpm_chainmesh.hip).
-tpm_status tpm_scan_i32(std::string& err, hipStream_t s, const int32_t* in, int64_t n, int32_t* part, int32_t* out);
 tpm_status tpm_fill_u64(tpm_ctx* ctx, unsigned long long* p, int64_t n);
 
 // FP64 momentum / energy reductions (tpm_moments.hip).  part holds

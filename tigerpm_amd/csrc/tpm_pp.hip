@@ -14,7 +14,8 @@
 // distance exceeds rcut has r >= rcut to every sink, so dropping it changes
 // no result; smaller tiles have tighter boxes and drop more.  Near pairs
 // evaluate compute_pp_interaction (kick_treepm.cu:242-283), far ones the same
-// law without its softening (pp_far).
+// law without its softening (pp_far).  kick_pme evaluates every pair with the former
+// (pp_sum_pme).
 //
 // Near pairs: distances are int32(sink - source) converted to float, which is the
 // reference's distance() (gravity_short.hpp:20-22) in units of 2^-32; every

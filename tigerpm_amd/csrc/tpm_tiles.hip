@@ -10,10 +10,10 @@
 // The order splits a cell's active particles in halves at the median of the
 // longest axis until <= ts remain, so a tile's box is near a cube: at 512^3
 // 16-sink tiles stage 1580 sources instead of 1930 with runs of the Morton
-// order (a CPU model of the boxes).  Count and build take 0.11 + 0.49 ms at
-// 256^3 and 0.9 + 3.5 ms at 512^3; the pair kernel went from 22.2 to 19.0 ms at 256^3.
+// order (a CPU model of the boxes).  Count and build take 0.05 + 0.52 ms at
+// 256^3 and 0.32 + 3.7 ms at 512^3; the pair kernel went from 22.2 to 19.0 ms at 256^3.
 // Tiles of active sinks only: with an eighth of 256^3 particles active the
-// kernel has an eighth of the tiles (11.9 -> 4.7 ms).
+// kernel has an eighth of the tiles (11.9 -> 4.8 ms).
 #include "tpm_tiles.hpp"
 #include "tpm_tile_order.hpp"
 
